@@ -68,3 +68,31 @@ def test_update_matches_oracle_and_adapts():
         assert np.array_equal(w, want)
     # the weights now follow where accepted events lie: every dimension sums to one
     assert np.allclose(w.sum(axis=2), 1.0)
+
+
+@pytest.mark.parametrize("n_out,counts,cfg", [
+    (4, [1], dict()),                                   # one event
+    (2, [1025 * 256 + 7], dict()),                      # one tile more than the workgroups of the histogram
+    (3, [1000, 255, 0, 64, 1, 4097], dict(block=64)),   # odd n_x: threads without an element; many short segments
+    (6, [300, 70001, 2], dict(block=64, ept=4)),        # several tiles per run, runs that end inside a range
+    (4, [400_000, 1, 300_000], dict()),                 # more elements per thread than a private count holds
+])
+def test_update_counts_every_accepted_event(n_out, counts, cfg):
+    """The histogram at its edges: the counts are whole numbers, so the weights are exact."""
+    import torch
+    import gpu_phs_amd as G
+    proc = W.process_shapes(n_out, 3)
+    counts = (counts + [0] * proc.n_channels)[:proc.n_channels]
+    ph, plan, bufs, chans = _plan(proc, counts, **cfg)
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    for b in bufs:
+        b.x.copy_(torch.rand(b.x.shape, generator=gen, device="cuda", dtype=torch.float64) ** 2)
+        b.ok.copy_(torch.rand(b.ok.shape, generator=gen, device="cuda") < 0.7)
+    bufs[0].x.view(-1)[0], bufs[0].x.view(-1)[1] = 1.0, 0.0   # the ends of the range
+    grid = G.Grid(ph)
+    w = grid.weights()
+    grid.update(plan)
+    x = np.concatenate([b.x.cpu().numpy() for b in bufs])
+    ok = np.concatenate([b.ok.cpu().numpy().astype(bool) for b in bufs])
+    ch = np.repeat(chans, [b.x.shape[0] for b in bufs])
+    assert np.array_equal(grid.weights(), oracle.grid_update(w, x, ok, ch))
