@@ -35,79 +35,142 @@ __device__ __forceinline__ void philox4x32_10(uint32_t c[4], uint32_t k0, uint32
   }
 }
 
+// ((a 2^32 + b) >> 11) 2^-53: both terms and their sum are exact.
 __device__ __forceinline__ double u53(uint32_t a, uint32_t b) {
-  return (double)((((uint64_t)a << 32) | b) >> 11) * 0x1.0p-53;
+  return __builtin_fma((double)a, 0x1.0p-32, (double)(b >> 11) * 0x1.0p-53);
 }
 
-// cdf: [channel][dim][kGridBins + 1] cumulative bin probabilities of the plan's channels.  One
-// wave per workgroup: it copies its tile's channel table into LDS, then draws the tile's events
-// 64 at a time.  The bin is the number of interior bounds F[1..9] at or below u, counted
-// without branches.  Each lane puts its event's randoms into its column of an LDS table
-// x[k][lane]; the wave then stores the 64 rows as one contiguous run (16-byte words where the
-// row length is even and the rows are 16-byte aligned), so the writes leave as whole lines.
-constexpr int kGenLanes = 64;
+// What a bin contributes: x = edge + (u - F) / rho, with the quotient's reciprocal at hand.  40
+// bytes: lanes that read different bins of one dimension meet different LDS banks.
+struct BinRec {
+  double F, next, rho, inv, edge;   // F_b, F_{b+1}, density (F_{b+1} - F_b) / width, 1 / rho, b / kGridBins
+};
 
-__global__ __launch_bounds__(kGenLanes) void grid_generate_kernel(const TileDesc* __restrict__ tiles, int n_tiles,
-                                                                  const SegDesc* __restrict__ segs,
-                                                                  const ChannelDesc* __restrict__ chans,
-                                                                  const double* __restrict__ cdf, int n_dim,
-                                                                  uint64_t seed) {
-  extern __shared__ double cdf_l[];   // n_dim * (kGridBins + 1), then n_dim rows of kGenLanes + 1
+// (u - F) / rho, correctly rounded as the division is: the product with the rounded reciprocal,
+// then one step with the exact remainder (P. Markstein, IBM J. Res. Dev. 34 (1990) 111).  A bin
+// that holds some u > 0 has rho > 2^-107; for the others (inv = 0) only u = F = 0 occurs.
+__device__ __forceinline__ double in_bin(const BinRec& r, double u) {
+  const double n = u - r.F;
+  const double q = n * r.inv;
+  return __builtin_fma(__builtin_fma(-r.rho, q, n), r.inv, q);
+}
+
+// cdf: [channel][dim][kGridBins + 1] cumulative bin probabilities of the plan's channels.
+//
+// Bound by integer and FP64 issue (10 rounds of two 32 x 32-bit products per two randoms), not by
+// its writes, so the work per random is kept down: the top bits of u give the first bin it can lie
+// in, and the bounds are compared from there (the bin is the number of interior bounds at or below
+// u, and the bounds rise); the division by the bin's density is a product with its reciprocal,
+// corrected; and the rows leave without a division per word.  A workgroup takes a contiguous range
+// of the tile table (as the histogram below), builds the tables of a channel once per run of tiles
+// in LDS, and its waves then take 64 events each: every lane puts its event's randoms into its column of the
+// wave's table x[k][lane], and the wave stores the 64 rows as one contiguous run (16-byte words
+// where the row length is even and the rows are 16-byte aligned).  4e6 events of 8 randoms: 70 us
+// (57 VALU instructions per random, the vector units busy throughout; 79 us with both tables at
+// strides whose lanes met the same banks), against 103 us with nine bounds read per random, two
+// divisions and a division per word stored.
+constexpr int kGenWaves = 4;
+constexpr int kGenThreads = 64 * kGenWaves;
+constexpr int kGenGroups = 4096;
+constexpr int kGenRow = 68;   // the lanes that read one another's columns meet different LDS banks
+constexpr int kGenCellBits = 6, kGenCells = 1 << kGenCellBits;
+
+__global__ __launch_bounds__(kGenThreads) void grid_generate_kernel(const TileDesc* __restrict__ tiles, int n_tiles,
+                                                                    const SegDesc* __restrict__ segs,
+                                                                    const ChannelDesc* __restrict__ chans,
+                                                                    const double* __restrict__ cdf, int n_dim,
+                                                                    uint64_t seed) {
+  // n_dim * kGridBins records, per wave n_dim rows of kGenRow doubles, n_dim * kGenCells first bins
+  extern __shared__ BinRec rec[];
   constexpr int NB1 = kGridBins + 1;
-  constexpr int S = kGenLanes + 1;
-  double* xs = cdf_l + n_dim * NB1;
-  const int lane = (int)threadIdx.x;
-  for (int t = (int)blockIdx.x; t < n_tiles; t += (int)gridDim.x) {
+  const int lane = (int)threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  double* xs0 = (double*)(rec + n_dim * kGridBins);
+  double* xs = xs0 + wave * n_dim * kGenRow;
+  uint8_t* first = (uint8_t*)(xs0 + kGenWaves * n_dim * kGenRow);
+  const int t1 = (int)((int64_t)n_tiles * ((int64_t)blockIdx.x + 1) / gridDim.x);
+  for (int t = (int)((int64_t)n_tiles * blockIdx.x / gridDim.x); t < t1;) {
     const TileDesc td = tiles[t];
     const SegDesc sd = segs[td.seg];
     const int n_x = chans[sd.channel].n_x;
     const double* F0 = cdf + (size_t)sd.channel * n_dim * NB1;
-    __syncthreads();   // the previous tile's tables have been read
-    for (int i = lane; i < n_x * NB1; i += kGenLanes) cdf_l[i] = F0[i];
+    // the run: this tile and the following ones of its segment, up to the range's end
+    const int64_t left = (sd.n_events - td.e0 + td.count - 1) / td.count;
+    const int run = left < t1 - t ? (int)left : t1 - t;
+    const int64_t e_run = td.e0 + (int64_t)run * td.count;
+    const int64_t e_end = e_run < sd.n_events ? e_run : sd.n_events;
+    t += run;
+    __syncthreads();   // the previous run's records have been read
+    for (int i = (int)threadIdx.x; i < n_x * kGridBins; i += kGenThreads) {
+      const int k = i / kGridBins, b = i - k * kGridBins;
+      const double f0 = F0[k * NB1 + b], f1 = F0[k * NB1 + b + 1];
+      const double rho = (f1 - f0) * kGridBins;
+      // (no u is above the last bin's bound)
+      rec[i] = BinRec{f0, b < kGridBins - 1 ? f1 : 2.0, rho, rho > 0x1.0p-1000 ? 1.0 / rho : 0.0, (double)b / kGridBins};
+    }
+    for (int i = (int)threadIdx.x; i < n_x * kGenCells; i += kGenThreads) {
+      const double* F = F0 + i / kGenCells * NB1;
+      const double u = (double)(i % kGenCells) / kGenCells;
+      int b = 0;
+      for (int q = 1; q < kGridBins; q++) b += F[q] <= u ? 1 : 0;
+      first[i] = (uint8_t)b;
+    }
     __syncthreads();
     const bool vec = (sd.align16 & 1) && (n_x % 2 == 0);
-    for (int base = 0; base < td.count; base += kGenLanes) {
-      const int cnt = min(kGenLanes, td.count - base);
-      const int64_t e = td.e0 + base + lane;
-      if (lane < cnt) {
-        for (int j = 0; 2 * j < n_x; j++) {
-          uint32_t c[4] = {(uint32_t)e, (uint32_t)((uint64_t)e >> 32), (uint32_t)td.seg, (uint32_t)j};
-          philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
+    // word w of a wave's rows holds doubles w * step ..: event (w * step) / n_x, random the rest;
+    // 64 words on, both advance by constants
+    const int step = vec ? 2 : 1;
+    const int ev0 = lane * step / n_x, k0 = lane * step - ev0 * n_x;
+    const int dev = 64 * step / n_x, dk = 64 * step - dev * n_x;
+    // (tiles start at multiples of 64 events, so an event's low index word is the unit's with the lane)
+    for (int64_t e = td.e0 + 64 * wave; e < e_end; e += kGenThreads) {
+      const int cnt = e_end - e < 64 ? (int)(e_end - e) : 64;
+      const uint32_t e_lo = (uint32_t)e + (uint32_t)lane, e_hi = (uint32_t)((uint64_t)e >> 32);
+      for (int j = 0; 2 * j < n_x; j++) {
+        uint32_t c[4] = {e_lo, e_hi, (uint32_t)td.seg, (uint32_t)j};
+        philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
 #pragma unroll
-          for (int h = 0; h < 2; h++) {
-            const int k = 2 * j + h;
-            if (k >= n_x) break;
-            const double u = u53(c[2 * h], c[2 * h + 1]);
-            const double* F = cdf_l + k * NB1;
-            int b = 0;
-#pragma unroll
-            for (int q = 1; q < kGridBins; q++) b += F[q] <= u ? 1 : 0;
-            const double rho = (F[b + 1] - F[b]) * kGridBins;   // density of bin b (width 1 / kGridBins)
-            xs[k * S + lane] = (double)b / kGridBins + (u - F[b]) / rho;
-          }
+        for (int h = 0; h < 2; h++) {
+          const int k = 2 * j + h;
+          if (k >= n_x) break;
+          const double u = u53(c[2 * h], c[2 * h + 1]);
+          const BinRec* at = rec + k * kGridBins + first[k * kGenCells + (int)(c[2 * h] >> (32 - kGenCellBits))];
+          BinRec r = *at;
+          while (r.next <= u) r = *++at;
+          xs[k * kGenRow + lane] = r.edge + in_bin(r, u);
         }
       }
-      __syncthreads();
-      // rows [e0 + base, e0 + base + cnt) of x are cnt * n_x consecutive doubles
+      // the wave's lanes read one another's columns: no other wave is concerned
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      // rows [e, e + cnt) of x are cnt * n_x consecutive doubles
       const int n = cnt * n_x;
-      double* dst = const_cast<double*>(sd.x) + (td.e0 + base) * (int64_t)n_x;
+      double* dst = const_cast<double*>(sd.x) + e * (int64_t)n_x;
+      int ev = ev0, k = k0;
       if (vec) {
         gdouble2* d2 = (gdouble2*)dst;
-        for (int w = lane; 2 * w < n; w += kGenLanes) {
-          const int i = 2 * w, ev = i / n_x, k = i - ev * n_x;   // k even, so k + 1 < n_x
-          dvec2 v;
-          v.x = xs[k * S + ev];
-          v.y = xs[(k + 1) * S + ev];
+        for (int w = lane; 2 * w < n; w += 64) {
+          dvec2 v;   // k is even, so k + 1 < n_x
+          v.x = xs[k * kGenRow + ev];
+          v.y = xs[(k + 1) * kGenRow + ev];
           d2[w] = v;
+          ev += dev;
+          k += dk;
+          if (k >= n_x) { k -= n_x; ev++; }
         }
       } else {
         gdouble* d1 = as_global(dst);
-        for (int i = lane; i < n; i += kGenLanes) {
-          const int ev = i / n_x;
-          d1[i] = xs[(i - ev * n_x) * S + ev];
+        for (int w = lane; w < n; w += 64) {
+          d1[w] = xs[k * kGenRow + ev];
+          ev += dev;
+          k += dk;
+          if (k >= n_x) { k -= n_x; ev++; }
         }
       }
-      __syncthreads();   // the table is read before the next events overwrite it
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();   // the table is read before the next events overwrite it
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
   }
 }
@@ -214,9 +277,9 @@ __global__ void fill_u64_kernel(unsigned long long* p, size_t n) {
 
 hipError_t launch_grid_generate(const DevicePlan& dp, const double* cdf, int n_dim, uint64_t seed, hipStream_t stream) {
   if (dp.n_tiles <= 0) return hipSuccess;
-  const size_t shmem = ((size_t)n_dim * (kGridBins + 1) + (size_t)n_dim * (kGenLanes + 1)) * sizeof(double);
-  hipLaunchKernelGGL(grid_generate_kernel, dim3(dp.n_tiles), dim3(kGenLanes), shmem, stream, dp.tiles, dp.n_tiles,
-                     dp.segs, dp.chans, cdf, n_dim, seed);
+  const size_t shmem = (size_t)n_dim * (kGridBins * sizeof(BinRec) + kGenWaves * kGenRow * sizeof(double) + kGenCells);
+  hipLaunchKernelGGL(grid_generate_kernel, dim3(std::min(dp.n_tiles, kGenGroups)), dim3(kGenThreads), shmem, stream,
+                     dp.tiles, dp.n_tiles, dp.segs, dp.chans, cdf, n_dim, seed);
   return hipGetLastError();
 }
 

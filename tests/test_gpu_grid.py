@@ -96,3 +96,33 @@ def test_update_counts_every_accepted_event(n_out, counts, cfg):
     ok = np.concatenate([b.ok.cpu().numpy().astype(bool) for b in bufs])
     ch = np.repeat(chans, [b.x.shape[0] for b in bufs])
     assert np.array_equal(grid.weights(), oracle.grid_update(w, x, ok, ch))
+
+
+@pytest.mark.parametrize("n_out,counts,cfg", [
+    (2, [1], dict()),
+    (3, [65, 0, 4097, 1], dict(block=64)),          # odd rows: 8-byte words; several runs per workgroup
+    (4, [4097 * 256 + 63], dict()),                 # more tiles than workgroups
+    (6, [64, 63, 300_001], dict(block=128, ept=2)),
+])
+def test_generate_edges_match_oracle(n_out, counts, cfg):
+    """Draws at the edges of the kernel's tables: bins without weight at both ends and in a row, weights over
+    many orders of magnitude (several bounds inside one cell of the first-bin table), one full bin."""
+    import torch
+    import gpu_phs_amd as G
+    proc = W.process_shapes(n_out, 3)
+    counts = (counts + [0] * proc.n_channels)[:proc.n_channels]
+    ph, plan, bufs, chans = _plan(proc, counts, **cfg)
+    grid = G.Grid(ph)
+    rng = np.random.default_rng(n_out)
+    w = 10.0 ** rng.uniform(-6, 0, grid.shape)
+    w[:, 0, 0] = w[:, 0, 9] = 0.0
+    w[:, 1, 3:7] = 0.0
+    w[0, 1, :9] = 0.0
+    grid.set_weights(w)
+    seed = 0xFEDC_BA98_7654_3210
+    grid.generate(plan, seed)
+    torch.cuda.synchronize()
+    F = oracle.grid_cdf(w)
+    for s, (b, c) in enumerate(zip(bufs, chans)):
+        got = b.x.cpu().numpy()
+        assert np.array_equal(got, oracle.grid_sample(F[c], oracle.grid_uniforms(seed, s, got.shape[0], proc.n_x)))
