@@ -48,6 +48,8 @@ int inverse_prepare(PlanObj& pl, const int64_t* seg_row0, int64_t n_rows) {
   std::vector<InvStep> steps(n_ch);
   for (int k = 0; k < n_ch; k++) {
     steps[k].channel = order[k];
+    steps[k].node0 = cp.channels[order[k]].node0;
+    steps[k].shape = cp.channels[order[k]].shape;
     steps[k].new_group = k == 0 || root_key(order[k]) != root_key(order[k - 1]) ? 1 : 0;
   }
   // save-bank levels of the subtrees deferred below the root (the root's own deferred daughter
@@ -109,6 +111,20 @@ int inverse_prepare(PlanObj& pl, const int64_t* seg_row0, int64_t n_rows) {
   return ok_status();
 }
 
+// Ranges of channels that each 64-event unit is split over, one wave each: as many as give every
+// SIMD its three waves (any split, also single channels), then as many as give a dozen rounds of
+// waves, so that the last round's idle SIMDs cost little, but no fewer than kMinChannels channels
+// each, since a range stages the momenta and evaluates its first root anew.  2e5 events x 120
+// channels (3190 units): 0.96 ms at 13 ranges, 1.08 at 4, 1.05 at 51; 1e6 events x 3 channels (15,627
+// units): 113 us unsplit, 138 at 3 ranges.
+int inverse_chunks(const InverseTables& it, int64_t units) {
+  constexpr int64_t kFillWaves = 256 * 4 * 3, kManyWaves = 40000, kMinChannels = 4;
+  if (!it.shared_roots || units <= 0) return 1;
+  const int64_t fill = std::min<int64_t>((kFillWaves + units - 1) / units, it.n_ch);
+  const int64_t many = std::min<int64_t>((kManyWaves + units - 1) / units, it.n_ch / kMinChannels);
+  return (int)std::max<int64_t>(1, std::max(fill, many));
+}
+
 }  // namespace
 
 int gphs::plan_inverse(PlanObj& pl, const int64_t* seg_row0, int64_t n_rows, double* factors, double* x_out, int block,
@@ -119,16 +135,16 @@ int gphs::plan_inverse(PlanObj& pl, const int64_t* seg_row0, int64_t n_rows, dou
     return set_error(GPU_PHS_E_ARG, "inverse: block must be 64, 128, 192 or 256");
   int rc = inverse_prepare(pl, seg_row0, n_rows);
   if (rc) return rc;
-  // the default workgroup: 256 threads for processes of a few channels (the 3 c1 channels: 1.72
-  // against 1.79 ms for 1e7 events at 128), 128 for many (the 120 c2 channels: 7.65 against
-  // 7.70-7.83 ms for 1e6 events at 256), each where its LDS tables fit
+  // the default workgroup: one wave with shared roots (its waves work alone), else 256 threads for
+  // processes of a few channels, 128 for many, each where its LDS tables fit
   if (block == 0) {
-    block = pl.inv.n_ch <= 16 ? 256 : 128;
+    block = pl.inv.shared_roots ? 64 : pl.inv.n_ch <= 16 ? 256 : 128;
     while (block > 64 && inverse_lds_bytes(pl.inv, block) > forward_lds_limit()) block -= 64;
   }
   if (inverse_lds_bytes(pl.inv, block) > forward_lds_limit())
     return set_error(GPU_PHS_E_ARG, "inverse: the trees need more LDS than a workgroup of this size may use");
-  hipError_t e = launch_inverse(pl.inv, pl.dp.tiles, pl.dp.n_tiles, pl.dp.segs, block, 0, factors, x_out, n_rows, stream);
+  hipError_t e = launch_inverse(pl.inv, pl.dp.tiles, pl.dp.n_tiles, std::max(1, (pl.tile_max + 63) / 64), pl.dp.segs,
+                                block, inverse_chunks(pl.inv, pl.n_units), factors, x_out, n_rows, stream);
   if (e != hipSuccess) return hip_error(e, "inverse launch");
   return ok_status();
 }

@@ -187,6 +187,12 @@ int plan_build(PlanObj& pl) {
     return pl.order == 1 && tile_depth[a] > tile_depth[b];
   });
   pl.tiles.resize(tiles.size());
+  pl.tile_max = 0;
+  pl.n_units = 0;
+  for (const TileDesc& td : tiles) {
+    pl.tile_max = std::max(pl.tile_max, (int)td.count);
+    pl.n_units += (td.count + 63) / 64;
+  }
   for (int c = 0; c < kTileClasses; c++) pl.class_begin[c] = pl.class_end[c] = 0;
   for (size_t i = 0; i < idx.size(); i++) {
     const TileDesc& td = tiles[idx[i]];

@@ -49,29 +49,35 @@ constexpr int kInvRootBankWords = 7;
 extern __shared__ double inv_lds[];
 
 // x and the map factor of an internal daughter from its msq (mappings_gpu.hpp:15-172; STEP_H
-// as phs_cpu.cpp:95-101, whose root of the quadratic is the right one).
+// as phs_cpu.cpp:95-101, whose root of the quadratic is the right one).  INV: the constants are the
+// program's, and so are the reciprocals of the common maps' divisors (ChildCmd::inv0, inv1).
+template <bool INV>
 __device__ __forceinline__ void x_from_msq(const ChildCmd& c, double msq, double s, double& x, double& f) {
+  auto over = [](double n, double d, double r) {
+    if constexpr (INV) return math::divide(n, math::Divisor{d, r});
+    else return n / d;
+  };
   switch (c.kind) {
     case MK_LINEAR:
-      x = (msq - c.msq_min) / (c.msq_max - c.msq_min);
+      x = over(msq - c.msq_min, c.msq_max - c.msq_min, c.inv0);
       f = c.f_lin;
       break;
     case MK_BREIT_WIGNER: {
-      const double z = (msq - c.m * c.m) / (c.m * c.w);
-      x = (atan(z) - c.a0) / (c.a1 - c.a0);
+      const double z = over(msq - c.m * c.m, c.m * c.w, c.inv0);
+      x = over(atan(z) - c.a0, c.a1 - c.a0, c.inv1);
       f = c.a2 * (1 + z * z);
       break;
     }
     case MK_EXP: {
       const double z = msq - c.msq_min + c.a0;
-      x = math::log_bounded(z / c.a0) / c.a1;
+      x = over(math::log_bounded(over(z, c.a0, c.inv0)), c.a1, c.inv1);
       f = c.a2 * z;
       break;
     }
     case MK_TU: {
       const bool lo = msq < (c.msq_max + c.msq_min) / 2;
       const double z = lo ? msq - c.msq_min + c.a0 : c.msq_max - msq + c.a0;
-      const double l = math::log_bounded(z / c.a0) / c.a1;
+      const double l = over(math::log_bounded(over(z, c.a0, c.inv0)), c.a1, c.inv1);
       x = lo ? l : 1 - l;
       f = c.a2 * z;
       break;
@@ -94,15 +100,19 @@ __device__ __forceinline__ void x_from_msq(const ChildCmd& c, double msq, double
   }
 }
 
-// x and factor of cos theta (mappings_gpu.hpp:181-219).
-__device__ __forceinline__ void x_from_ct(int kind, double ct, double b0, double b1, double& x, double& f) {
-  if (kind == CK_FLAT) {
+// x and factor of cos theta (mappings_gpu.hpp:181-219); INV as above (NodeCmd::inv_b0, inv_2b1).
+template <bool INV>
+__device__ __forceinline__ void x_from_ct(const NodeCmd& nc, double ct, double b0, double b1, double& x, double& f) {
+  if (nc.ct_kind == CK_FLAT) {
     x = (ct + 1) / 2;
     f = 1;
   } else {
     const bool neg = ct < 0;
     const double t = neg ? ct + b0 + 1 : -ct + b0 + 1;
-    const double l = math::log_bounded(t / b0) / (2 * b1);
+    double l;
+    if constexpr (INV)
+      l = math::divide(math::log_bounded(math::divide(t, {b0, nc.inv_b0})), {2 * b1, nc.inv_2b1});
+    else l = math::log_bounded(t / b0) / (2 * b1);
     x = neg ? l : 1 - l;
     f = t * b1;
   }
@@ -166,9 +176,9 @@ __device__ __forceinline__ void rotate_back(double (&G)[16], double ct, double s
 
 // One branch's decay from its own msq and mass and its daughters' msq (phs.cu:658-664):
 // p_decay, the factor sqrt(lambda) / msq (0 where lambda <= 0, phs_cpu.cpp:275-279), and the
-// boost bg = p_parent / m.  The quotients are IEEE divisions, as in the reference: they feed
-// the frames of the daughters and so the cosines that the peaked maps take near +-1, where an
-// ulp of cos theta is amplified by up to sqrt(s) / m^2 in the map's factor.
+// boost bg = p_parent / m.  The quotients are correctly rounded, as the reference's divisions
+// are: they feed the frames of the daughters and so the cosines that the peaked maps take near
+// +-1, where an ulp of cos theta is amplified by up to sqrt(s) / m^2 in the map's factor.
 struct Decay {
   double pk, lam, bg;
 };
@@ -176,16 +186,17 @@ __device__ __forceinline__ Decay decay(double cur_msq, double cur_m, double cur_
   const double lda = (cur_msq - msq0 - msq1) * (cur_msq - msq0 - msq1) - 4 * msq0 * msq1;
   const bool pos = lda > 0;
   const double sl = pos ? math::sqrt_phys(lda) : 0.0;
+  const math::Divisor m = math::divisor(cur_m);
   Decay d;
-  d.pk = sl / (2 * cur_m);
+  d.pk = math::divide(sl, {2 * cur_m, 0.5 * m.r});
   d.lam = pos ? sl / cur_msq : 0.0;
-  d.bg = cur_m > 0 ? cur_p / cur_m : 0.0;
+  d.bg = cur_m > 0 ? math::divide(cur_p, m) : 0.0;
   return d;
 }
 
 // Polar and azimuthal angles of the direction v (mappings_gpu.hpp:196-219 inverted): the
-// cosines and sines of both angles (IEEE divisions, as above) and x_phi = atan2(v1, v0) / 2 pi
-// in [0, 1], formed in turns by math::atan2_turns.
+// cosines and sines of both angles (correctly rounded quotients, as above) and
+// x_phi = atan2(v1, v0) / 2 pi in [0, 1], formed in turns by math::atan2_turns.
 struct Dir {
   double xphi, ct, st, cp, sp;
 };
@@ -194,10 +205,11 @@ __device__ __forceinline__ Dir direction(double v0, double v1, double v2) {
   const double vv = math::sqrt_phys(v0 * v0 + v1 * v1 + v2 * v2);
   Dir d;
   d.xphi = math::atan2_turns(v1, v0);
-  d.cp = rho > 0 ? v0 / rho : 1.0;
-  d.sp = rho > 0 ? v1 / rho : 0.0;
-  d.ct = v2 / vv;
-  d.st = rho / vv;
+  const math::Divisor dr = math::divisor(rho), dv = math::divisor(vv);
+  d.cp = rho > 0 ? math::divide(v0, dr) : 1.0;
+  d.sp = rho > 0 ? math::divide(v1, dr) : 0.0;
+  d.ct = math::divide(v2, dv);
+  d.st = math::divide(rho, dv);
   return d;
 }
 
@@ -290,10 +302,20 @@ __device__ __forceinline__ void static_for(F&& f) {
   }
 }
 
-// The inverse of one event into channel `cd` (program `prog`) from its root group's geometry
+// G of the root's daughters: the root's rotation R_y(-theta) R_z(-phi) of the identity, without
+// the products by 0 and 1 (rotate_back's bits, up to the sign of a zero).
+__device__ __forceinline__ void root_frame(double (&G)[16], const RootGeo& g) {
+  G[0] = 1; G[1] = 0;            G[2] = 0;            G[3] = 0;
+  G[4] = 0; G[5] = g.ct * g.cp;  G[6] = g.ct * g.sp;  G[7] = -g.st;
+  G[8] = 0; G[9] = -g.sp;        G[10] = g.cp;        G[11] = 0;
+  G[12] = 0; G[13] = g.st * g.cp; G[14] = g.st * g.sp; G[15] = g.ct;
+}
+
+// The inverse of one event into the channel of program `prog` from its root group's geometry
 // `g`: the randoms go to xo[0..n_x), returns the factor.  SID >= 0: the channel's program has
 // shape SID of the compile-time table and every branch's structure is a constant; SID < 0: it
-// is read from the program.  No branch has a friend.
+// is read from the program.  No branch has a friend.  `cd` is any channel of the process (only
+// what its channels share is read).
 template <int SID, bool PEV, class XO>
 __device__ __forceinline__ double inverse_channel(const ChannelDesc& cd, const EvBeams& eb,
                                                   const NodeCmd* __restrict__ prog, const RootGeo& g,
@@ -302,32 +324,35 @@ __device__ __forceinline__ double inverse_channel(const ChannelDesc& cd, const E
   using W = Walk<SID>;
   const double s = eb.s;
   double factor = 1;
+  auto map_msq = [&](const NodeCmd& nc, int i, int d, double msq) {
+    double x, f;
+    if constexpr (PEV) x_from_msq<false>(child_at(nc.k[d], eb.sqrts, s, cd.m_tot), msq, s, x, f);
+    else x_from_msq<true>(nc.k[d], msq, s, x, f);
+    xo[W::xi(nc, i, d)] = x;
+    factor *= f;
+  };
+  auto map_ct = [&](const NodeCmd& nc, int i, double ct) {
+    double x, f, m_max, b0 = nc.b0, b1 = nc.b1;
+    if constexpr (PEV) node_at(nc, i == 0, eb, cd.m_tot, m_max, b0, b1);
+    x_from_ct<!PEV>(nc, ct, b0, b1, x, f);
+    xo[W::xphi(nc, i) + 1] = x;
+    factor *= f;
+  };
   // the root: this channel's maps of the shared numbers
   {
     const NodeCmd& nc = prog[0];
 #pragma unroll
-    for (int d = 0; d < 2; d++) {
-      if (!W::leaf(nc, 0, d)) {
-        double x, f;
-        if constexpr (PEV) x_from_msq(child_at(nc.k[d], eb.sqrts, s, cd.m_tot), g.msq[d], s, x, f);
-        else x_from_msq(nc.k[d], g.msq[d], s, x, f);
-        xo[W::xi(nc, 0, d)] = x;
-        factor *= f;
-      }
-    }
+    for (int d = 0; d < 2; d++)
+      if (!W::leaf(nc, 0, d)) map_msq(nc, 0, d, g.msq[d]);
     factor *= g.lam;
     xo[W::xphi(nc, 0)] = g.xphi;
-    double xc, fct, m_max, cb0 = nc.b0, cb1 = nc.b1;
-    if constexpr (PEV) node_at(nc, true, eb, cd.m_tot, m_max, cb0, cb1);
-    x_from_ct(nc.ct_kind, g.ct, cb0, cb1, xc, fct);
-    xo[W::xphi(nc, 0) + 1] = xc;
-    factor *= fct;
+    map_ct(nc, 0, g.ct);
   }
   if (W::n_nodes(cd) == 1) return factor;
 
   // the root's frame, and the daughter the walk descends into
-  double G[16] = {1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1};
-  rotate_back(G, g.ct, g.st, g.cp, g.sp);
+  double G[16];
+  root_frame(G, g);
   const int rdesc = W::desc(prog[0], 0);
   double cur_msq = g.msq[rdesc], cur_m = g.m[rdesc], cur_p = rdesc == 0 ? g.pk : -g.pk;
   bool root_pending = W::push(prog[0], 0) >= 0;
@@ -347,37 +372,43 @@ __device__ __forceinline__ double inverse_channel(const ChannelDesc& cd, const E
     const double msq0 = q0[0] * q0[0] - q0[1] * q0[1] - q0[2] * q0[2] - q0[3] * q0[3];
     const double msq1 = q1[0] * q1[0] - q1[1] * q1[1] - q1[2] * q1[2] - q1[3] * q1[3];
 #pragma unroll
-    for (int d = 0; d < 2; d++) {
-      if (!W::leaf(nc, i, d)) {
-        double x, f;
-        if constexpr (PEV) x_from_msq(child_at(nc.k[d], eb.sqrts, s, cd.m_tot), d == 0 ? msq0 : msq1, s, x, f);
-        else x_from_msq(nc.k[d], d == 0 ? msq0 : msq1, s, x, f);
-        xo[W::xi(nc, i, d)] = x;
-        factor *= f;
-      }
-    }
+    for (int d = 0; d < 2; d++)
+      if (!W::leaf(nc, i, d)) map_msq(nc, i, d, d == 0 ? msq0 : msq1);
     const Decay dk = decay(cur_msq, cur_m, cur_p, msq0, msq1);
     const double pk = dk.pk, bg = dk.bg;
     factor *= dk.lam;
 
     const double gm = math::sqrt_phys(1 + bg * bg);
+    double v0, v1;
+    // a daughter of the root: the zeros and ones of the root's frame are known
+    bool first = false;
+    if constexpr (SID >= 0) first = kShapes[SID < 0 ? 0 : SID].node[decltype(ic)::value].parent == 0;
+    if (first) {
+      G[0] = gm;
+      G[12] = -bg;
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const double r0 = G[j], r3 = G[12 + j];
-      G[j] = gm * r0 - bg * r3;
-      G[12 + j] = -bg * r0 + gm * r3;
+      for (int j = 1; j < 4; j++) {
+        const double r3 = G[12 + j];
+        G[j] = -(bg * r3);
+        G[12 + j] = gm * r3;
+      }
+      v0 = G[5] * q0[1] + G[6] * q0[2] + G[7] * q0[3];
+      v1 = G[9] * q0[1] + G[10] * q0[2];
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const double r0 = G[j], r3 = G[12 + j];
+        G[j] = gm * r0 - bg * r3;
+        G[12 + j] = -bg * r0 + gm * r3;
+      }
+      v0 = G[4] * q0[0] + G[5] * q0[1] + G[6] * q0[2] + G[7] * q0[3];
+      v1 = G[8] * q0[0] + G[9] * q0[1] + G[10] * q0[2] + G[11] * q0[3];
     }
-    const double v0 = G[4] * q0[0] + G[5] * q0[1] + G[6] * q0[2] + G[7] * q0[3];
-    const double v1 = G[8] * q0[0] + G[9] * q0[1] + G[10] * q0[2] + G[11] * q0[3];
     const double v2 = G[12] * q0[0] + G[13] * q0[1] + G[14] * q0[2] + G[15] * q0[3];
     const Dir dr = direction(v0, v1, v2);
     const double ct = dr.ct, st = dr.st, cp = dr.cp, sp = dr.sp;
     xo[W::xphi(nc, i)] = dr.xphi;
-    double xc, fct, m_max, cb0 = nc.b0, cb1 = nc.b1;
-    if constexpr (PEV) node_at(nc, false, eb, cd.m_tot, m_max, cb0, cb1);
-    x_from_ct(nc.ct_kind, ct, cb0, cb1, xc, fct);
-    xo[W::xphi(nc, i) + 1] = xc;
-    factor *= fct;
+    map_ct(nc, i, ct);
     rotate_back(G, ct, st, cp, sp);
 
     const int push = W::push(nc, i), desc = W::desc(nc, i);
@@ -407,9 +438,7 @@ __device__ __forceinline__ double inverse_channel(const ChannelDesc& cd, const E
       // the subtree the root deferred: the root's frame again, re-formed bit for bit
       root_pending = false;
       const int rp = 1 - rdesc;
-#pragma unroll
-      for (int j = 0; j < 16; j++) G[j] = (j % 5 == 0) ? 1.0 : 0.0;
-      rotate_back(G, g.ct, g.st, g.cp, g.sp);
+      root_frame(G, g);
       cur_msq = g.msq[rp];
       cur_m = g.m[rp];
       cur_p = rp == 0 ? g.pk : -g.pk;
@@ -445,8 +474,8 @@ __device__ __forceinline__ double inverse_event(const ChannelDesc& cd, const EvB
     for (int d = 0; d < 2; d++) {
       if (!nc.k[d].leaf) {
         double x, f;
-        if constexpr (PEV) x_from_msq(child_at(nc.k[d], eb.sqrts, s, cd.m_tot), d == 0 ? msq0 : msq1, s, x, f);
-        else x_from_msq(nc.k[d], d == 0 ? msq0 : msq1, s, x, f);
+        if constexpr (PEV) x_from_msq<false>(child_at(nc.k[d], eb.sqrts, s, cd.m_tot), d == 0 ? msq0 : msq1, s, x, f);
+        else x_from_msq<false>(nc.k[d], d == 0 ? msq0 : msq1, s, x, f);
         xo[nc.k[d].xi] = x;
         factor *= f;
       }
@@ -495,7 +524,7 @@ __device__ __forceinline__ double inverse_event(const ChannelDesc& cd, const EvB
     xo[nc.x_phi] = dr.xphi;
     double xc, fct, m_max, cb0 = nc.b0, cb1 = nc.b1;
     if constexpr (PEV) node_at(nc, i == 0, eb, cd.m_tot, m_max, cb0, cb1);
-    x_from_ct(nc.ct_kind, ct, cb0, cb1, xc, fct);
+    x_from_ct<false>(nc, ct, cb0, cb1, xc, fct);
     xo[nc.x_phi + 1] = xc;
     factor *= fct;
     rotate_back(G, ct, st, cp, sp);
@@ -604,127 +633,182 @@ __global__ __launch_bounds__(256) void inverse_kernel(const TileDesc* __restrict
 
 // Shared roots (processes without friends): the channels in the order of `steps`, a root
 // evaluated where a group starts.  Channels of up to four final-state particles run the walk
-// specialised for their shape; the others the walk that reads its structure from the program,
-// which only the GEN instances contain (it needs some thirty more registers than the
-// specialised walks).  WPE: waves per SIMD the register allocation aims at (0: the compiler's
-// choice).
-// LDS per workgroup: the momenta column (4 n_out rows of blockDim.x + 1 doubles), the save
-// banks of subtrees deferred below the root (19 rows of blockDim.x doubles per level), then the
-// randoms table of the channel being inverted (n_x rows of blockDim.x + 1 doubles).
-template <bool PEV, bool GEN, int WPE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void inverse_kernel_shared(const TileDesc* __restrict__ tiles, int n_tiles,
-                                                             const SegDesc* __restrict__ segs,
-                                                             const InvSeg* __restrict__ isegs,
-                                                             const InvStep* __restrict__ steps,
-                                                             const ChannelDesc* __restrict__ chans,
-                                                             const NodeCmd* __restrict__ nodes, int n_ch, int n_out,
-                                                             int n_x, int64_t n_rows, int rest_banks,
-                                                             double* __restrict__ factors,
-                                                             double* __restrict__ x_out) {
-  const int B = (int)blockDim.x;
-  const int S = B + 1;
-  const int lane = (int)threadIdx.x;
-  double* ps = inv_lds;
-  double* bank = ps + 4 * n_out * S + lane;
-  double* pl = ps + lane;
-  // each channel's randoms of the sub-tile go through the table xs[k][event], then to x_out as
-  // one contiguous run of rows (whole lines, streaming stores) instead of 8-byte pieces 8 n_x
-  // bytes apart
-  double* xs = ps + 4 * n_out * S + kInvBankWords * rest_banks * B;
-  const XColumn xl{xs + lane, S};
-  const int q_step_r = B / n_x, q_step_k = B % n_x;
-  for (int t = (int)blockIdx.x; t < n_tiles; t += (int)gridDim.x) {
-    const TileDesc td = tiles[t];
-    const SegDesc sd = segs[td.seg];
-    const InvSeg is = isegs[td.seg];
-    for (int base = 0; base < td.count; base += B) {
-      const int cnt = min(B, td.count - base);
-      const bool valid = lane < cnt;   // lanes past the end stage the last event and store nothing
-      const int64_t e = td.e0 + base + (valid ? lane : cnt - 1);
-      const int64_t row = is.row0 + e;
-      EvBeams eb;
-      if constexpr (PEV) eb = event_beams(chans[0], as_global(sd.e1)[e], as_global(sd.e2)[e]);
-      else eb = fixed_beams(chans[0]);
-      const gdouble* pe = as_global((const double*)sd.p) + e * 4 * n_out;
-      for (int j = 0; j < n_out; j++) {
-        double q0 = pe[4 * j], q1 = pe[4 * j + 1], q2 = pe[4 * j + 2], q3 = pe[4 * j + 3];
-        if (eb.bg_lab != 0) {
-          const double a = eb.g_lab * q0 - eb.bg_lab * q3;
-          const double b = -eb.bg_lab * q0 + eb.g_lab * q3;
-          q0 = a; q3 = b;
+// specialised for their shape (NX > 0: the process's n_x, a constant); the others the walk that
+// reads its structure from the program (NX = 0), which needs some thirty more registers.  WPE:
+// waves per SIMD the register allocation aims at (0: the compiler's choice).
+//
+// Bound by FP64 issue and latency.  Every wavefront works alone, without barriers, on one unit: 64
+// events of a tile times one of n_chunks ranges of `steps`, so that a batch of few events still
+// gives every SIMD its waves (the launch picks n_chunks).  Its lanes exchange data only through
+// the wave's own randoms table.
+// LDS per wave: the momenta column (4 n_out rows of 64 doubles), the save banks of subtrees
+// deferred below the root (19 rows of 64 doubles per level), then the randoms table of the channel
+// being inverted (n_x rows of kInvRow doubles).
+constexpr int kInvRow = 68;   // lanes that read one another's columns meet different LDS banks
+
+// LDS of one wave, in doubles.
+__host__ __device__ inline int inverse_wave_words(int n_out, int n_x, int rest_banks) {
+  return 64 * (4 * n_out + kInvBankWords * rest_banks) + kInvRow * n_x;
+}
+
+// The wave's randoms table to rows [0, cnt) of dst [..][n_x], one contiguous run of streaming
+// stores: 16-byte words where rows are even and dst is aligned.
+template <int NX>
+__device__ __forceinline__ void store_rows(const double* __restrict__ xs, int cnt, int n_x_rt, bool aligned,
+                                           gdouble* __restrict__ dst) {
+  const int lane = (int)threadIdx.x & 63;
+  if constexpr (NX > 0 && NX % 2 == 0) {
+    if (aligned) {
+      gdouble2* d2 = (gdouble2*)dst;
+#pragma unroll
+      for (int u = 0; u < NX / 2; u++) {   // word w: doubles 2 w and 2 w + 1, of one row
+        const int w = lane + 64 * u, r = 2 * w / NX, k = 2 * w - r * NX;
+        if (cnt == 64 || r < cnt) {
+          dvec2 v;
+          v.x = xs[k * kInvRow + r];
+          v.y = xs[(k + 1) * kInvRow + r];
+          __builtin_nontemporal_store(v, d2 + w);
         }
-        pl[(4 * j) * S] = q0; pl[(4 * j + 1) * S] = q1; pl[(4 * j + 2) * S] = q2; pl[(4 * j + 3) * S] = q3;
       }
-      RootGeo geo;
-      for (int k = 0; k < n_ch; k++) {
-        const InvStep st = steps[k];
-        const int c = st.channel;
-        const ChannelDesc cd = chans[c];
-        const NodeCmd* prog = nodes + cd.node0;
-        if (st.new_group) geo = root_geometry(prog[0], eb, pl, S, n_out);
-        if (c == is.own) {
-          if (valid) {
-            const gdouble* xi = as_global(sd.x) + e * n_x;
-            for (int q = 0; q < n_x; q++) xl[q] = xi[q];
-            as_global(factors)[row * n_ch + c] = as_global((const double*)sd.factor)[e];
-          }
-        } else if (valid) {
-          double f;
-          switch (cd.shape) {
-            case 0: f = inverse_channel<0, PEV>(cd, eb, prog, geo, pl, S, bank, B, xl); break;
-            case 1: f = inverse_channel<1, PEV>(cd, eb, prog, geo, pl, S, bank, B, xl); break;
-            case 2: f = inverse_channel<2, PEV>(cd, eb, prog, geo, pl, S, bank, B, xl); break;
-            case 3: f = inverse_channel<3, PEV>(cd, eb, prog, geo, pl, S, bank, B, xl); break;
-            case 4: f = inverse_channel<4, PEV>(cd, eb, prog, geo, pl, S, bank, B, xl); break;
-            case 5: f = inverse_channel<5, PEV>(cd, eb, prog, geo, pl, S, bank, B, xl); break;
-            case 6: f = inverse_channel<6, PEV>(cd, eb, prog, geo, pl, S, bank, B, xl); break;
-            case 7: f = inverse_channel<7, PEV>(cd, eb, prog, geo, pl, S, bank, B, xl); break;
-            default:
-              if constexpr (GEN) f = inverse_channel<-1, PEV>(cd, eb, prog, geo, pl, S, bank, B, xl);
-              else f = 0;   // not reached: the host runs channels of other programs with GEN
-              break;
-          }
-          as_global(factors)[row * n_ch + c] = f;
-        }
-        // the sub-tile's rows of channel c, x_out[c][row0 + e0 + base ...][n_x]: element q of
-        // the run is row r = q / n_x, random k = q % n_x of the table
-        __syncthreads();
-        gdouble* dst = as_global(x_out) + ((int64_t)c * n_rows + is.row0 + td.e0 + base) * n_x;
-        int r = lane / n_x, kx = lane % n_x;
-        for (int q = lane; q < cnt * n_x; q += B) {
-          __builtin_nontemporal_store(xs[kx * S + r], dst + q);
-          r += q_step_r;
-          kx += q_step_k;
-          if (kx >= n_x) { kx -= n_x; r++; }
-        }
-        __syncthreads();
-      }
+      return;
     }
   }
+  const int n_x = NX > 0 ? NX : n_x_rt;
+  int r = lane / n_x, k = lane - r * n_x;
+  const int dr = 64 / n_x, dk = 64 - dr * n_x;
+  for (int q = lane; q < cnt * n_x; q += 64) {
+    __builtin_nontemporal_store(xs[k * kInvRow + r], dst + q);
+    r += dr;
+    k += dk;
+    if (k >= n_x) { k -= n_x; r++; }
+  }
 }
+
+// Lanes read LDS words that other lanes of the wave wrote before (the accesses of one wave stay in
+// order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <bool PEV, int NX, int WPE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void inverse_kernel_shared(
+    const TileDesc* __restrict__ tiles, int n_units, int n_sub, int n_chunks, const SegDesc* __restrict__ segs,
+    const InvSeg* __restrict__ isegs, const InvStep* __restrict__ steps, const ChannelDesc* __restrict__ chans,
+    const NodeCmd* __restrict__ nodes, int n_ch, int n_out_rt, int n_x_rt, int64_t n_rows, int rest_banks, int aligned,
+    double* __restrict__ factors, double* __restrict__ x_out) {
+  const int n_x = NX > 0 ? NX : n_x_rt, n_out = NX > 0 ? (NX + 4) / 3 : n_out_rt;
+  const int lane = (int)threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int u = (int)blockIdx.x * ((int)blockDim.x >> 6) + wave;
+  if (u >= n_units) return;
+  const int us = u / n_chunks, chunk = u - us * n_chunks;
+  const int t = us / n_sub, base = 64 * (us - t * n_sub);
+  const TileDesc td = tiles[t];
+  if (base >= td.count) return;
+  const SegDesc sd = segs[td.seg];
+  const InvSeg is = isegs[td.seg];
+  double* ps = inv_lds + wave * inverse_wave_words(n_out, n_x, rest_banks);
+  double* pl = ps + lane;
+  double* bank = ps + 64 * 4 * n_out + lane;
+  double* xs = ps + 64 * (4 * n_out + kInvBankWords * rest_banks);
+  const XColumn xl{xs + lane, kInvRow};
+  const int cnt = min(64, td.count - base);
+  const bool valid = lane < cnt;   // lanes past the end stage the last event and store nothing
+  const int64_t e = td.e0 + base + (valid ? lane : cnt - 1);
+  const int64_t row = is.row0 + e;
+  const ChannelDesc cd = chans[0];   // only what all channels of the process share is read
+  EvBeams eb;
+  if constexpr (PEV) eb = event_beams(cd, as_global(sd.e1)[e], as_global(sd.e2)[e]);
+  else eb = fixed_beams(cd);
+  const gdouble* pe = as_global((const double*)sd.p) + e * 4 * n_out;
+  for (int j = 0; j < n_out; j++) {
+    double q0 = pe[4 * j], q1 = pe[4 * j + 1], q2 = pe[4 * j + 2], q3 = pe[4 * j + 3];
+    if (eb.bg_lab != 0) {
+      const double a = eb.g_lab * q0 - eb.bg_lab * q3;
+      const double b = -eb.bg_lab * q0 + eb.g_lab * q3;
+      q0 = a; q3 = b;
+    }
+    pl[(4 * j) * 64] = q0; pl[(4 * j + 1) * 64] = q1; pl[(4 * j + 2) * 64] = q2; pl[(4 * j + 3) * 64] = q3;
+  }
+  gdouble* f_row = as_global(factors) + row * n_ch;
+  gdouble* x_rows = as_global(x_out) + (is.row0 + td.e0 + base) * n_x;
+  const int k_begin = (int)((int64_t)n_ch * chunk / n_chunks), k_end = (int)((int64_t)n_ch * (chunk + 1) / n_chunks);
+  RootGeo geo;
+  for (int k = k_begin; k < k_end; k++) {
+    const InvStep st = steps[k];
+    const int c = st.channel;
+    const NodeCmd* prog = nodes + st.node0;
+    if (st.new_group || k == k_begin) geo = root_geometry(prog[0], eb, pl, 64, n_out);
+    double f;
+    if (c == is.own) {
+      const gdouble* xi = as_global(sd.x) + e * n_x;
+      for (int q = 0; q < n_x; q++) xl[q] = xi[q];
+      f = as_global((const double*)sd.factor)[e];
+    } else if constexpr (NX == 0) {
+      f = inverse_channel<-1, PEV>(cd, eb, prog, geo, pl, 64, bank, 64, xl);
+    } else if constexpr (NX == 2) {
+      f = inverse_channel<0, PEV>(cd, eb, prog, geo, pl, 64, bank, 64, xl);
+    } else if constexpr (NX == 5) {
+      if (st.shape == 1) f = inverse_channel<1, PEV>(cd, eb, prog, geo, pl, 64, bank, 64, xl);
+      else f = inverse_channel<2, PEV>(cd, eb, prog, geo, pl, 64, bank, 64, xl);
+    } else {
+      switch (st.shape) {
+        case 3: f = inverse_channel<3, PEV>(cd, eb, prog, geo, pl, 64, bank, 64, xl); break;
+        case 4: f = inverse_channel<4, PEV>(cd, eb, prog, geo, pl, 64, bank, 64, xl); break;
+        case 5: f = inverse_channel<5, PEV>(cd, eb, prog, geo, pl, 64, bank, 64, xl); break;
+        case 6: f = inverse_channel<6, PEV>(cd, eb, prog, geo, pl, 64, bank, 64, xl); break;
+        default: f = inverse_channel<7, PEV>(cd, eb, prog, geo, pl, 64, bank, 64, xl); break;
+      }
+    }
+    if (valid) f_row[c] = f;
+    wave_sync();
+    store_rows<NX>(xs, cnt, n_x, aligned != 0, x_rows + (int64_t)c * n_rows * n_x);
+    wave_sync();
+  }
+}
+
+// The shapes behind each NX above.
+static_assert(kShapes[0].n_out == 2 && kShapes[1].n_out == 3 && kShapes[2].n_out == 3 && kShapes[3].n_out == 4 &&
+                  kShapes[7].n_out == 4 && kInvShapes == 8 && (kNumShapes == 8 || kShapes[8].n_out > 4),
+              "inverse walks per n_x");
 
 }  // namespace
 
 size_t inverse_lds_bytes(const InverseTables& it, int block) {
-  if (it.shared_roots)
-    return ((size_t)4 * it.n_out * (block + 1) + (size_t)kInvBankWords * it.rest_banks * block +
-            (size_t)it.n_x * (block + 1)) * sizeof(double);
+  if (it.shared_roots) return (size_t)(block / 64) * inverse_wave_words(it.n_out, it.n_x, it.rest_banks) * sizeof(double);
   const size_t words = it.root_bank ? kInvRootBankWords : kInvBankWords;
   return ((size_t)4 * it.n_out * (block + 1) + words * it.n_banks * block) * sizeof(double);
 }
 
-hipError_t launch_inverse(const InverseTables& it, const TileDesc* tiles, int n_tiles, const SegDesc* segs,
-                          int block, int grid, double* factors, double* x_out, int64_t n_rows, hipStream_t stream) {
+namespace {
+
+template <bool PEV>
+auto pick_shared(const InverseTables& it) {
+  if (it.generic) return inverse_kernel_shared<PEV, 0, 0>;
+  return it.n_x == 2 ? inverse_kernel_shared<PEV, 2, 3>
+                     : it.n_x == 5 ? inverse_kernel_shared<PEV, 5, 3> : inverse_kernel_shared<PEV, 8, 3>;
+}
+
+}  // namespace
+
+hipError_t launch_inverse(const InverseTables& it, const TileDesc* tiles, int n_tiles, int n_sub, const SegDesc* segs,
+                          int block, int n_chunks, double* factors, double* x_out, int64_t n_rows,
+                          hipStream_t stream) {
   if (n_tiles <= 0) return hipSuccess;
-  if (block < 64 || block > 256 || block % 64) return hipErrorInvalidValue;
+  if (block < 64 || block > 256 || block % 64 || n_sub < 1 || n_chunks < 1 || n_chunks > it.n_ch)
+    return hipErrorInvalidValue;
   const size_t shmem = inverse_lds_bytes(it, block);
   if (shmem > forward_lds_limit()) return hipErrorInvalidValue;
-  const int g = grid > 0 ? (grid < n_tiles ? grid : n_tiles) : n_tiles;
   if (it.shared_roots) {
-    auto k = it.per_event_beams ? (it.generic ? inverse_kernel_shared<true, true, 0> : inverse_kernel_shared<true, false, 3>)
-                                : (it.generic ? inverse_kernel_shared<false, true, 0> : inverse_kernel_shared<false, false, 3>);
-    hipLaunchKernelGGL(k, dim3(g), dim3(block), shmem, stream, tiles, n_tiles, segs, it.isegs, it.steps, it.chans,
-                       it.nodes, it.n_ch, it.n_out, it.n_x, n_rows, it.rest_banks, factors, x_out);
+    const int64_t units = (int64_t)n_tiles * n_sub * n_chunks, waves = block / 64;
+    if (units > 0x7fffffff) return hipErrorInvalidValue;
+    auto k = it.per_event_beams ? pick_shared<true>(it) : pick_shared<false>(it);
+    const int aligned = reinterpret_cast<uintptr_t>(x_out) % 16 == 0 ? 1 : 0;
+    hipLaunchKernelGGL(k, dim3((unsigned)((units + waves - 1) / waves)), dim3(block), shmem, stream, tiles, (int)units,
+                       n_sub, n_chunks, segs, it.isegs, it.steps, it.chans, it.nodes, it.n_ch, it.n_out, it.n_x,
+                       n_rows, it.rest_banks, aligned, factors, x_out);
     return hipGetLastError();
   }
   using K = decltype(&inverse_kernel<false, false, false>);
@@ -735,7 +819,7 @@ hipError_t launch_inverse(const InverseTables& it, const TileDesc* tiles, int n_
   else
     k = it.per_event_beams ? (it.has_friends ? inverse_kernel<true, true, false> : inverse_kernel<false, true, false>)
                            : (it.has_friends ? inverse_kernel<true, false, false> : inverse_kernel<false, false, false>);
-  hipLaunchKernelGGL(k, dim3(g), dim3(block), shmem, stream, tiles, n_tiles, segs, it.isegs, it.chans, it.nodes,
+  hipLaunchKernelGGL(k, dim3(n_tiles), dim3(block), shmem, stream, tiles, n_tiles, segs, it.isegs, it.chans, it.nodes,
                      it.n_ch, it.n_out, it.n_x, n_rows, factors, x_out);
   return hipGetLastError();
 }

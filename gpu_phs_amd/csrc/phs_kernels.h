@@ -87,6 +87,8 @@ struct InvSeg {
 struct InvStep {
   int32_t channel;
   int32_t new_group;
+  int32_t node0;   // the channel's first NodeCmd
+  int32_t shape;   // its tree shape
 };
 // Device copies of one process's complete channel table (every channel is a target).
 struct InverseTables {
@@ -105,9 +107,10 @@ struct InverseTables {
 // compile-time table (the trees of two to four final-state particles).
 constexpr int kInvShapes = 8;
 size_t inverse_lds_bytes(const InverseTables& it, int block);
-// factors [n_rows][n_ch] and x_out [n_ch][n_rows][n_x] for the events of tiles [0, n_tiles).
-hipError_t launch_inverse(const InverseTables& it, const TileDesc* tiles, int n_tiles, const SegDesc* segs,
-                          int block, int grid, double* factors, double* x_out, int64_t n_rows, hipStream_t stream);
+// factors [n_rows][n_ch] and x_out [n_ch][n_rows][n_x] for the events of tiles [0, n_tiles), none of
+// which holds more than 64 n_sub events; with shared roots, the channels in n_chunks ranges of steps.
+hipError_t launch_inverse(const InverseTables& it, const TileDesc* tiles, int n_tiles, int n_sub, const SegDesc* segs,
+                          int block, int n_chunks, double* factors, double* x_out, int64_t n_rows, hipStream_t stream);
 
 // Adaptive grids of the randoms (rng.cpp:5: 10 equal bins per channel and dimension).
 constexpr int kGridBins = 10;

@@ -162,6 +162,35 @@ GPHS_MATH_FN double recip(double b) {
 #endif
 }
 
+// Correctly rounded quotients by one divisor, with the divisor's reciprocal formed once: the
+// reciprocal estimate refined by two Newton steps, then per quotient the product, one step with the
+// exact remainder, and the fixup that gives zeros, infinities and NaN as the division does.  These
+// are the steps of the compiler's own double division without its rescaling, which only operands
+// beyond 2^+-700 or so need: the same bits, in 4 instructions per quotient and 5 per divisor
+// instead of 11 per quotient.  `r` may also be the rounded reciprocal from elsewhere.
+struct Divisor {
+  double d, r;
+};
+GPHS_MATH_FN Divisor divisor(double d) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  double r = __builtin_amdgcn_rcp(d);
+  double e = __builtin_fma(-d, r, 1.0);
+  r = __builtin_fma(r, e, r);
+  e = __builtin_fma(-d, r, 1.0);
+  return Divisor{d, __builtin_fma(r, e, r)};
+#else
+  return Divisor{d, 1.0 / d};
+#endif
+}
+GPHS_MATH_FN double divide(double n, Divisor v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const double q = n * v.r;
+  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-v.d, q, n), v.r, q), v.d, n);
+#else
+  return n / v.d;
+#endif
+}
+
 // sqrt(x): the reciprocal square root estimate refined by one Goldschmidt step and two Newton
 // corrections -- the compiler's own sequence for a double sqrt without its rescaling of inputs
 // below 2^-767, which the kernels' arguments (squared masses and momenta of physical size,

@@ -48,6 +48,8 @@ struct PlanObj {
   std::vector<NodeCmd> nodes;
   std::vector<SegDesc> segs;
   std::vector<TileDesc> tiles;
+  int tile_max = 0;                        // events of the largest tile
+  int64_t n_units = 0;                     // wavefronts of 64 events the tiles fill
   std::vector<int> seg_tile_begin, seg_tile_end;  // tile ranges per segment (segment order)
   int n_banks = 0;
   // Tile classes: channels of up to 8 randoms whose only deferring branch is the root (class 0)

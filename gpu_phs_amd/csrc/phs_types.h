@@ -53,7 +53,18 @@ struct ChildCmd {
   int32_t sum_len;
   int32_t pad1;
   uint64_t sum_code;
+  // rounded reciprocals of the inverse map's divisors (inv_divisor0, inv_divisor1; 0 where the
+  // map divides by something else)
+  double inv0, inv1;
 };
+
+// What x_from_msq divides by in the linear, Breit-Wigner, exponential and t/u maps.
+inline double inv_divisor0(int32_t kind, double a0, double m, double w, double msq_min, double msq_max) {
+  return kind == MK_LINEAR ? msq_max - msq_min : kind == MK_BREIT_WIGNER ? m * w : kind <= MK_TU ? a0 : 0.0;
+}
+inline double inv_divisor1(int32_t kind, double a0, double a1) {
+  return kind == MK_BREIT_WIGNER ? a1 - a0 : kind == MK_EXP || kind == MK_TU ? a1 : 0.0;
+}
 
 constexpr int kSumPush = 14;
 constexpr int kSumMerge = 15;
@@ -75,6 +86,7 @@ struct NodeCmd {
   double m_min;      // sum of leaf masses below the branch
   double m;          // map mass of this branch (cos-theta constants per event)
   double db_dm[2];   // d b[k] / d M (adjoint)
+  double inv_b0, inv_2b1;   // rounded 1 / b0 and 1 / (2 b1) of a peaked cos-theta map (inverse mapping)
   ChildCmd k[2];
 };
 

@@ -117,6 +117,29 @@ def test_shared_roots_identical_to_per_channel(name):
     assert np.array_equal(x1, x2, equal_nan=True)
 
 
+@pytest.mark.parametrize("n_out,n,block,unaligned", [
+    (2, 1, 0, False), (2, 4133, 128, True), (3, 65, 0, False), (3, 5003, 192, True), (4, 63, 0, False),
+    (4, 64, 256, True), (4, 20011, 0, False), (5, 3001, 64, True), (6, 2003, 128, False)])
+def test_inverse_units_identical_to_per_channel(n_out, n, block, unaligned):
+    """One wave per 64 events and range of channels: remainders of every size, workgroups of one to four
+    waves, few units (a range per channel) and many, rows of x_out at 8-byte alignment."""
+    import torch
+    proc = W.process_shapes(n_out, 2)
+    rng = np.random.default_rng(n)
+    ch = rng.integers(0, proc.n_channels, n).astype(np.int32)
+    out, plan, bufs = run_gpu(proc, rng.random((n, proc.n_x)), ch)
+    room = torch.full((proc.n_channels * n * proc.n_x + 2,), -7.0, dtype=torch.float64, device="cuda")
+    at = 1 if unaligned else 0
+    x_out = room[at:at + proc.n_channels * n * proc.n_x].view(proc.n_channels, n, proc.n_x)
+    f1, x1 = (t.cpu().numpy() for t in plan.inverse(x_out=x_out, block=block))
+    rest = torch.cat([room[:at], room[at + x_out.numel():]]).cpu().numpy()
+    assert (rest == -7.0).all()
+    plan.set_specialize(False)
+    f2, x2 = (t.cpu().numpy() for t in plan.inverse())
+    assert np.array_equal(f1, f2, equal_nan=True)
+    assert np.array_equal(x1, x2, equal_nan=True)
+
+
 def test_inverse_unequal_beams():
     proc = W.process_friends(4)
     E1, E2 = 650.0, 1000.0 ** 2 / (4 * 650.0)
