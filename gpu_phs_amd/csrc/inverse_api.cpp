@@ -3,13 +3,35 @@
 // phs.cu:1491-1554).
 #include <algorithm>
 #include <cstring>
-#include <tuple>
+#include <string>
+#include <utility>
 
 #include "phs_state.h"
 
 using namespace gphs;
 
 namespace {
+
+// How a daughter's momentum is added up (a sum of two does not depend on their order).
+std::string association(const NodeCmd* prog, const ChildCmd& k) {
+  if (k.leaf) return std::to_string(k.out);
+  if (k.sum_len <= 0) return "i" + std::to_string(k.leaves);   // in index order
+  std::string a = association(prog, prog[k.node].k[0]), b = association(prog, prog[k.node].k[1]);
+  if (b < a) std::swap(a, b);
+  return "(" + a + " " + b + ")";
+}
+
+// Per branch of channel c in visit order: everything its geometry depends on.
+std::vector<std::string> branch_keys(const CompiledProcess& cp, int c) {
+  const ChannelDesc& cd = cp.channels[c];
+  const NodeCmd* prog = &cp.nodes[cd.node0];
+  std::vector<std::string> keys;
+  for (int i = 0; i < cd.n_nodes; i++) {
+    std::string up = i == 0 ? "" : keys[prog[i].parent] + "/" + std::to_string(prog[i].slot) + ":";
+    keys.push_back(up + association(prog, prog[i].k[0]) + "," + association(prog, prog[i].k[1]));
+  }
+  return keys;
+}
 
 // Device tables of the inverse: per-segment (generating channel, first row), then the
 // process's channels and programs.  Re-uploaded only when the rows change.
@@ -35,22 +57,31 @@ int inverse_prepare(PlanObj& pl, const int64_t* seg_row0, int64_t n_rows) {
       std::memcmp(is.data(), pl.inv_segs.data(), is.size() * sizeof(InvSeg)) == 0)
     return ok_status();
   const int n_ch = (int)cp.channels.size();
-  // channel order: by the root's daughters (final-state particles and sum program of each), so
-  // that channels sharing their root's evaluation are adjacent; channel index within a group
-  auto root_key = [&](int c) {
-    const NodeCmd& r = cp.nodes[cp.channels[c].node0];
-    return std::make_tuple(r.k[0].leaves, r.k[0].sum_len, r.k[0].sum_code, r.k[1].leaves, r.k[1].sum_len,
-                           r.k[1].sum_code);
-  };
+  // channel order: by what each branch, root first, computes from an event -- where it hangs, and both
+  // daughters' final-state particles with the association their momenta are added in -- so that
+  // channels sharing their first branches' evaluation are adjacent; channel index within a group
+  std::vector<std::vector<std::string>> keys(n_ch);
+  for (int c = 0; shared && c < n_ch; c++) keys[c] = branch_keys(cp, c);
   std::vector<int> order(n_ch);
   for (int c = 0; c < n_ch; c++) order[c] = c;
-  if (shared) std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return root_key(a) < root_key(b); });
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return keys[a] < keys[b]; });
   std::vector<InvStep> steps(n_ch);
+  std::vector<std::string> last(kMaxOut);
+  int branches = 0, evaluated = 0;   // below the roots
   for (int k = 0; k < n_ch; k++) {
-    steps[k].channel = order[k];
-    steps[k].node0 = cp.channels[order[k]].node0;
-    steps[k].shape = cp.channels[order[k]].shape;
-    steps[k].new_group = k == 0 || root_key(order[k]) != root_key(order[k - 1]) ? 1 : 0;
+    const int c = order[k];
+    steps[k].channel = c;
+    steps[k].node0 = cp.channels[c].node0;
+    steps[k].shape = cp.channels[c].shape;
+    steps[k].eval = 0;
+    for (size_t i = 0; i < keys[c].size(); i++) {
+      if (i > 0) branches++;
+      if (keys[c][i] != last[i]) {
+        steps[k].eval |= 1 << i;
+        if (i > 0) evaluated++;
+      }
+      last[i] = keys[c][i];
+    }
   }
   // save-bank levels of the subtrees deferred below the root (the root's own deferred daughter
   // is re-formed from the shared root)
@@ -103,6 +134,9 @@ int inverse_prepare(PlanObj& pl, const int64_t* seg_row0, int64_t n_rows) {
   pl.inv.per_event_beams = pl.dp.per_event_beams;
   pl.inv.shared_roots = shared ? 1 : 0;
   pl.inv.rest_banks = rest_banks;
+  // a repeated branch saves about a third of its channel's work, the tests for it cost a tenth of
+  // every channel's: worth it where a quarter of the branches repeat
+  pl.inv.shared_branches = shared && 4 * evaluated <= 3 * branches ? 1 : 0;
   pl.inv.generic = 0;
   for (const ChannelDesc& c : cp.channels)
     if (c.shape < 0 || c.shape >= kInvShapes) pl.inv.generic = 1;

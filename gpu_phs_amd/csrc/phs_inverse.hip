@@ -64,7 +64,8 @@ __device__ __forceinline__ void x_from_msq(const ChildCmd& c, double msq, double
       break;
     case MK_BREIT_WIGNER: {
       const double z = over(msq - c.m * c.m, c.m * c.w, c.inv0);
-      x = over(atan(z) - c.a0, c.a1 - c.a0, c.inv1);
+      // (the device library's atan keeps its coefficients in forty vector registers)
+      x = over(math::atan_radians(z) - c.a0, c.a1 - c.a0, c.inv1);
       f = c.a2 * (1 + z * z);
       break;
     }
@@ -311,107 +312,198 @@ __device__ __forceinline__ void root_frame(double (&G)[16], const RootGeo& g) {
   G[12] = 0; G[13] = g.st * g.cp; G[14] = g.st * g.sp; G[15] = g.ct;
 }
 
-// The inverse of one event into the channel of program `prog` from its root group's geometry
-// `g`: the randoms go to xo[0..n_x), returns the factor.  SID >= 0: the channel's program has
-// shape SID of the compile-time table and every branch's structure is a constant; SID < 0: it
-// is read from the program.  No branch has a friend.  `cd` is any channel of the process (only
-// what its channels share is read).
+// One channel's maps of the shared geometry: x and factor of an internal daughter's msq (daughter d
+// of branch i) and of a branch's cos theta.  SID as in Walk.
 template <int SID, bool PEV, class XO>
+__device__ __forceinline__ void map_msq(const ChannelDesc& cd, const EvBeams& eb, const NodeCmd& nc, int i, int d,
+                                        double msq, XO xo, double& factor) {
+  double x, f;
+  if constexpr (PEV) x_from_msq<false>(child_at(nc.k[d], eb.sqrts, eb.s, cd.m_tot), msq, eb.s, x, f);
+  else x_from_msq<true>(nc.k[d], msq, eb.s, x, f);
+  xo[Walk<SID>::xi(nc, i, d)] = x;
+  factor *= f;
+}
+template <int SID, bool PEV, class XO>
+__device__ __forceinline__ void map_angles(const ChannelDesc& cd, const EvBeams& eb, const NodeCmd& nc, int i,
+                                           double xphi, double ct, XO xo, double& factor) {
+  xo[Walk<SID>::xphi(nc, i)] = xphi;
+  double x, f, m_max, b0 = nc.b0, b1 = nc.b1;
+  if constexpr (PEV) node_at(nc, i == 0, eb, cd.m_tot, m_max, b0, b1);
+  x_from_ct<!PEV>(nc, ct, b0, b1, x, f);
+  xo[Walk<SID>::xphi(nc, i) + 1] = x;
+  factor *= f;
+}
+
+// ---- shared branches (trees of up to four final-state particles) ---------------------------
+//
+// Below the root the same holds branch by branch: what a branch computes from the event depends on
+// its ancestors' final-state particles and daughter order, its own daughters' and their
+// association, and not on any map.  The host orders the channels by the branches of their trees, root
+// first, and marks in each step which branches differ from the last ones evaluated
+// (InvStep::eval); the others keep their numbers, and the channel only applies its maps.  The 120
+// channels of random 2->4 trees evaluate 30 roots and 129 branches instead of 240 (690 VALU
+// instructions per event and channel instead of 897).  Where few branches repeat, the tests keep the
+// compiler from interleaving a branch's evaluation with the maps and cost more than they save (the
+// three 2->4 resonance channels, which share nothing: 134 against 120 us for 1e6 events), so the
+// kernel without them (SHARE = false) runs, which also leaves out the generating channel's branches.
+
+// What a branch below the root leaves behind: msq of its internal daughter (if any), sqrt(lambda) /
+// msq, the first daughter's angles, and what its daughters' frame is formed from.
+struct BranchGeo {
+  double msqi, lam, xphi, ct, st, cp, sp, bg, gm, pk;
+};
+
+// Geometry of branch I >= 1 of shape SID from the root's and, for a branch below branch 1, branch 1's.
+template <int SID, int I>
+__device__ __forceinline__ BranchGeo branch_geometry(const NodeCmd* __restrict__ prog, const RootGeo& g,
+                                                     const BranchGeo& up, const double* __restrict__ pl, int S) {
+  constexpr ShapeNode N = kShapes[SID].node[I];
+  constexpr ShapeNode P = kShapes[SID].node[N.parent < 0 ? 0 : N.parent];
+  constexpr int slot = P.node0 == I ? 0 : 1;   // which daughter of its parent the branch is
+  double q0[4], q1[4];
+  daughter_sum<SID, I, 0>(prog, pl, S, q0);
+  daughter_sum<SID, I, 1>(prog, pl, S, q1);
+  const double msq0 = q0[0] * q0[0] - q0[1] * q0[1] - q0[2] * q0[2] - q0[3] * q0[3];
+  const double msq1 = q1[0] * q1[0] - q1[1] * q1[1] - q1[2] * q1[2] - q1[3] * q1[3];
+  BranchGeo r;
+  r.msqi = !N.leaf0 ? msq0 : msq1;
+  // the root's frame R_y(-theta) R_z(-phi), of which rows 1 to 3 have zeros at column 0 and [2][3]
+  double G[16];
+  root_frame(G, g);
+  double v0, v1, v2;
+  if constexpr (N.parent == 0) {
+    const Decay dk = decay(g.msq[slot], g.m[slot], slot == 0 ? g.pk : -g.pk, msq0, msq1);
+    r.pk = dk.pk; r.lam = dk.lam; r.bg = dk.bg;
+    r.gm = math::sqrt_phys(1 + dk.bg * dk.bg);
+    v0 = G[5] * q0[1] + G[6] * q0[2] + G[7] * q0[3];
+    v1 = G[9] * q0[1] + G[10] * q0[2];
+    v2 = -r.bg * q0[0] + (r.gm * G[13]) * q0[1] + (r.gm * G[14]) * q0[2] + (r.gm * G[15]) * q0[3];
+  } else {
+    // branch 1's boost and rotation on the root's frame, the products with its zeros left out
+    G[0] = up.gm;
+    G[12] = -up.bg;
+#pragma unroll
+    for (int j = 1; j < 4; j++) {
+      const double r3 = G[12 + j];
+      G[j] = -(up.bg * r3);
+      G[12 + j] = up.gm * r3;
+    }
+    const double w3 = G[12];
+    G[4] = -(up.st * w3);
+    G[8] = 0;
+    G[12] = up.ct * w3;
+#pragma unroll
+    for (int j = 1; j < 4; j++) {
+      const double w1 = G[4 + j], w2 = G[8 + j], w3j = G[12 + j];
+      const double t1 = j == 3 ? up.cp * w1 : up.cp * w1 + up.sp * w2;
+      G[4 + j] = up.ct * t1 - up.st * w3j;
+      G[8 + j] = j == 3 ? -(up.sp * w1) : -up.sp * w1 + up.cp * w2;
+      G[12 + j] = up.st * t1 + up.ct * w3j;
+    }
+    const Decay dk = decay(up.msqi, math::sqrt_phys(up.msqi), slot == 0 ? up.pk : -up.pk, msq0, msq1);
+    r.pk = dk.pk; r.lam = dk.lam; r.bg = dk.bg;
+    r.gm = math::sqrt_phys(1 + dk.bg * dk.bg);
+#pragma unroll
+    for (int j = 0; j < 4; j++) G[12 + j] = -r.bg * G[j] + r.gm * G[12 + j];
+    v0 = G[4] * q0[0] + G[5] * q0[1] + G[6] * q0[2] + G[7] * q0[3];
+    v1 = G[9] * q0[1] + G[10] * q0[2] + G[11] * q0[3];
+    v2 = G[12] * q0[0] + G[13] * q0[1] + G[14] * q0[2] + G[15] * q0[3];
+  }
+  const Dir dr = direction(v0, v1, v2);
+  r.xphi = dr.xphi; r.ct = dr.ct; r.st = dr.st; r.cp = dr.cp; r.sp = dr.sp;
+  return r;
+}
+
+// The inverse of one event into the channel of program `prog`, whose tree has shape SID (at most
+// three branches): the branches that `eval` marks are evaluated, then (unless `own`, the generating
+// channel, whose results come from the forward pass) the channel's maps are applied, in the order
+// of the walk: the randoms go to xo[0..n_x), returns the factor.
+template <int SID, bool PEV, bool SHARE, class XO>
+__device__ __forceinline__ double inverse_shape(const ChannelDesc& cd, const EvBeams& eb,
+                                                const NodeCmd* __restrict__ prog, int eval, bool own, const RootGeo& g,
+                                                BranchGeo& g1, BranchGeo& g2, const double* __restrict__ pl, int S,
+                                                XO xo) {
+  constexpr const ShapeProg& sh = kShapes[SID];
+  static_assert(sh.n_nodes <= 3, "trees of up to four final-state particles");
+  if (!SHARE && own) return 1;
+  if constexpr (sh.n_nodes > 1) {
+    if (!SHARE || (eval & 2)) g1 = branch_geometry<SID, 1>(prog, g, g1, pl, S);
+  }
+  if constexpr (sh.n_nodes > 2) {
+    if (!SHARE || (eval & 4)) g2 = branch_geometry<SID, 2>(prog, g, g1, pl, S);
+  }
+  double factor = 1;
+  if (own) return factor;
+#pragma unroll
+  for (int d = 0; d < 2; d++)
+    if (!(d == 0 ? sh.node[0].leaf0 : sh.node[0].leaf1)) map_msq<SID, PEV>(cd, eb, prog[0], 0, d, g.msq[d], xo, factor);
+  factor *= g.lam;
+  map_angles<SID, PEV>(cd, eb, prog[0], 0, g.xphi, g.ct, xo, factor);
+  static_for<1, sh.n_nodes>([&](auto ic) {
+    constexpr int i = decltype(ic)::value;
+    const BranchGeo& b = i == 1 ? g1 : g2;
+    if constexpr (!sh.node[i].leaf0) map_msq<SID, PEV>(cd, eb, prog[i], i, 0, b.msqi, xo, factor);
+    if constexpr (!sh.node[i].leaf1) map_msq<SID, PEV>(cd, eb, prog[i], i, 1, b.msqi, xo, factor);
+    factor *= b.lam;
+    map_angles<SID, PEV>(cd, eb, prog[i], i, b.xphi, b.ct, xo, factor);
+  });
+  return factor;
+}
+
+// The inverse of one event into the channel of program `prog` from its root group's geometry `g`,
+// the tree's structure read from the program: the randoms go to xo[0..n_x), returns the factor.  No
+// branch has a friend.  `cd` is any channel of the process (only what its channels share is read).
+template <bool PEV, class XO>
 __device__ __forceinline__ double inverse_channel(const ChannelDesc& cd, const EvBeams& eb,
                                                   const NodeCmd* __restrict__ prog, const RootGeo& g,
                                                   const double* __restrict__ pl, int S, double* bank, int B,
                                                   XO xo) {
-  using W = Walk<SID>;
-  const double s = eb.s;
   double factor = 1;
-  auto map_msq = [&](const NodeCmd& nc, int i, int d, double msq) {
-    double x, f;
-    if constexpr (PEV) x_from_msq<false>(child_at(nc.k[d], eb.sqrts, s, cd.m_tot), msq, s, x, f);
-    else x_from_msq<true>(nc.k[d], msq, s, x, f);
-    xo[W::xi(nc, i, d)] = x;
-    factor *= f;
-  };
-  auto map_ct = [&](const NodeCmd& nc, int i, double ct) {
-    double x, f, m_max, b0 = nc.b0, b1 = nc.b1;
-    if constexpr (PEV) node_at(nc, i == 0, eb, cd.m_tot, m_max, b0, b1);
-    x_from_ct<!PEV>(nc, ct, b0, b1, x, f);
-    xo[W::xphi(nc, i) + 1] = x;
-    factor *= f;
-  };
   // the root: this channel's maps of the shared numbers
-  {
-    const NodeCmd& nc = prog[0];
 #pragma unroll
-    for (int d = 0; d < 2; d++)
-      if (!W::leaf(nc, 0, d)) map_msq(nc, 0, d, g.msq[d]);
-    factor *= g.lam;
-    xo[W::xphi(nc, 0)] = g.xphi;
-    map_ct(nc, 0, g.ct);
-  }
-  if (W::n_nodes(cd) == 1) return factor;
+  for (int d = 0; d < 2; d++)
+    if (!prog[0].k[d].leaf) map_msq<-1, PEV>(cd, eb, prog[0], 0, d, g.msq[d], xo, factor);
+  factor *= g.lam;
+  map_angles<-1, PEV>(cd, eb, prog[0], 0, g.xphi, g.ct, xo, factor);
+  if (cd.n_nodes == 1) return factor;
 
   // the root's frame, and the daughter the walk descends into
   double G[16];
   root_frame(G, g);
-  const int rdesc = W::desc(prog[0], 0);
+  const int rdesc = prog[0].desc;
   double cur_msq = g.msq[rdesc], cur_m = g.m[rdesc], cur_p = rdesc == 0 ? g.pk : -g.pk;
-  bool root_pending = W::push(prog[0], 0) >= 0;
+  bool root_pending = prog[0].push >= 0;
   int depth = 0;   // save-bank entries of subtrees deferred below the root
 
-  auto branch = [&](auto ic) {
-    const int i = ic;
+  for (int i = 1; i < cd.n_nodes; ++i) {
     const NodeCmd& nc = prog[i];
     double q0[4], q1[4];
-    if constexpr (SID >= 0) {
-      daughter_sum<(SID < 0 ? 0 : SID), decltype(ic)::value, 0>(prog, pl, S, q0);
-      daughter_sum<(SID < 0 ? 0 : SID), decltype(ic)::value, 1>(prog, pl, S, q1);
-    } else {
-      branch_sum(pl, S, cd.n_out, nc.k[0], q0);
-      branch_sum(pl, S, cd.n_out, nc.k[1], q1);
-    }
+    branch_sum(pl, S, cd.n_out, nc.k[0], q0);
+    branch_sum(pl, S, cd.n_out, nc.k[1], q1);
     const double msq0 = q0[0] * q0[0] - q0[1] * q0[1] - q0[2] * q0[2] - q0[3] * q0[3];
     const double msq1 = q1[0] * q1[0] - q1[1] * q1[1] - q1[2] * q1[2] - q1[3] * q1[3];
 #pragma unroll
     for (int d = 0; d < 2; d++)
-      if (!W::leaf(nc, i, d)) map_msq(nc, i, d, d == 0 ? msq0 : msq1);
+      if (!nc.k[d].leaf) map_msq<-1, PEV>(cd, eb, nc, i, d, d == 0 ? msq0 : msq1, xo, factor);
     const Decay dk = decay(cur_msq, cur_m, cur_p, msq0, msq1);
     const double pk = dk.pk, bg = dk.bg;
     factor *= dk.lam;
 
     const double gm = math::sqrt_phys(1 + bg * bg);
-    double v0, v1;
-    // a daughter of the root: the zeros and ones of the root's frame are known
-    bool first = false;
-    if constexpr (SID >= 0) first = kShapes[SID < 0 ? 0 : SID].node[decltype(ic)::value].parent == 0;
-    if (first) {
-      G[0] = gm;
-      G[12] = -bg;
 #pragma unroll
-      for (int j = 1; j < 4; j++) {
-        const double r3 = G[12 + j];
-        G[j] = -(bg * r3);
-        G[12 + j] = gm * r3;
-      }
-      v0 = G[5] * q0[1] + G[6] * q0[2] + G[7] * q0[3];
-      v1 = G[9] * q0[1] + G[10] * q0[2];
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const double r0 = G[j], r3 = G[12 + j];
-        G[j] = gm * r0 - bg * r3;
-        G[12 + j] = -bg * r0 + gm * r3;
-      }
-      v0 = G[4] * q0[0] + G[5] * q0[1] + G[6] * q0[2] + G[7] * q0[3];
-      v1 = G[8] * q0[0] + G[9] * q0[1] + G[10] * q0[2] + G[11] * q0[3];
+    for (int j = 0; j < 4; j++) {
+      const double r0 = G[j], r3 = G[12 + j];
+      G[j] = gm * r0 - bg * r3;
+      G[12 + j] = -bg * r0 + gm * r3;
     }
+    const double v0 = G[4] * q0[0] + G[5] * q0[1] + G[6] * q0[2] + G[7] * q0[3];
+    const double v1 = G[8] * q0[0] + G[9] * q0[1] + G[10] * q0[2] + G[11] * q0[3];
     const double v2 = G[12] * q0[0] + G[13] * q0[1] + G[14] * q0[2] + G[15] * q0[3];
     const Dir dr = direction(v0, v1, v2);
-    const double ct = dr.ct, st = dr.st, cp = dr.cp, sp = dr.sp;
-    xo[W::xphi(nc, i)] = dr.xphi;
-    map_ct(nc, i, ct);
-    rotate_back(G, ct, st, cp, sp);
+    map_angles<-1, PEV>(cd, eb, nc, i, dr.xphi, dr.ct, xo, factor);
+    rotate_back(G, dr.ct, dr.st, dr.cp, dr.sp);
 
-    const int push = W::push(nc, i), desc = W::desc(nc, i);
+    const int push = nc.push, desc = nc.desc;
     if (push >= 0) {
       const double mp = push == 0 ? msq0 : msq1;
       double* b = bank + kInvBankWords * depth * B;
@@ -443,11 +535,6 @@ __device__ __forceinline__ double inverse_channel(const ChannelDesc& cd, const E
       cur_m = g.m[rp];
       cur_p = rp == 0 ? g.pk : -g.pk;
     }
-  };
-  if constexpr (SID >= 0) {
-    static_for<1, kShapes[SID < 0 ? 0 : SID].n_nodes>(branch);
-  } else {
-    for (int i = 1; i < cd.n_nodes; ++i) branch(i);
   }
   return factor;
 }
@@ -692,7 +779,7 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <bool PEV, int NX, int WPE>
+template <bool PEV, int NX, bool SHARE, int WPE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void inverse_kernel_shared(
     const TileDesc* __restrict__ tiles, int n_units, int n_sub, int n_chunks, const SegDesc* __restrict__ segs,
     const InvSeg* __restrict__ isegs, const InvStep* __restrict__ steps, const ChannelDesc* __restrict__ chans,
@@ -722,6 +809,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
   EvBeams eb;
   if constexpr (PEV) eb = event_beams(cd, as_global(sd.e1)[e], as_global(sd.e2)[e]);
   else eb = fixed_beams(cd);
+  gdouble* f_row = as_global(factors) + row * n_ch;
+  gdouble* x_rows = as_global(x_out) + (is.row0 + td.e0 + base) * n_x;
+  // the generating channel's slot: the forward pass's factor, and its randoms, whose rows lie as
+  // x_out's do (loaded here, beside the momenta, and stored below)
+  const gdouble* x_own = as_global(sd.x) + (td.e0 + base) * n_x;
+  gdouble* x_dst = x_rows + (int64_t)is.own * n_rows * n_x;
+  const int n_own = chunk == 0 ? cnt * n_x : 0;
+  double xo[NX > 0 ? NX : 1], f_own = 0;
+  if constexpr (NX > 0) {
+#pragma unroll
+    for (int q = 0; q < NX; q++)
+      if (lane + 64 * q < n_own) xo[q] = x_own[lane + 64 * q];
+    if (n_own > 0) f_own = as_global((const double*)sd.factor)[e];
+  }
   const gdouble* pe = as_global((const double*)sd.p) + e * 4 * n_out;
   for (int j = 0; j < n_out; j++) {
     double q0 = pe[4 * j], q1 = pe[4 * j + 1], q2 = pe[4 * j + 2], q3 = pe[4 * j + 3];
@@ -732,36 +833,47 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     }
     pl[(4 * j) * 64] = q0; pl[(4 * j + 1) * 64] = q1; pl[(4 * j + 2) * 64] = q2; pl[(4 * j + 3) * 64] = q3;
   }
-  gdouble* f_row = as_global(factors) + row * n_ch;
-  gdouble* x_rows = as_global(x_out) + (is.row0 + td.e0 + base) * n_x;
+  if constexpr (NX > 0) {
+#pragma unroll
+    for (int q = 0; q < NX; q++)
+      if (lane + 64 * q < n_own) __builtin_nontemporal_store(xo[q], x_dst + lane + 64 * q);
+  } else {
+    for (int q = lane; q < n_own; q += 64) __builtin_nontemporal_store(x_own[q], x_dst + q);
+    if (n_own > 0) f_own = as_global((const double*)sd.factor)[e];
+  }
+  if (n_own > 0 && valid) f_row[is.own] = f_own;
   const int k_begin = (int)((int64_t)n_ch * chunk / n_chunks), k_end = (int)((int64_t)n_ch * (chunk + 1) / n_chunks);
   RootGeo geo;
+  BranchGeo g1, g2;
   for (int k = k_begin; k < k_end; k++) {
     const InvStep st = steps[k];
     const int c = st.channel;
     const NodeCmd* prog = nodes + st.node0;
-    if (st.new_group || k == k_begin) geo = root_geometry(prog[0], eb, pl, 64, n_out);
-    double f;
-    if (c == is.own) {
-      const gdouble* xi = as_global(sd.x) + e * n_x;
-      for (int q = 0; q < n_x; q++) xl[q] = xi[q];
-      f = as_global((const double*)sd.factor)[e];
-    } else if constexpr (NX == 0) {
-      f = inverse_channel<-1, PEV>(cd, eb, prog, geo, pl, 64, bank, 64, xl);
+    const int eval = k == k_begin ? ~0 : st.eval;
+    const bool own = c == is.own;
+    if (eval & 1) geo = root_geometry(prog[0], eb, pl, 64, n_out);
+    double f = 0;
+    auto walk = [&](auto sid) {
+      f = inverse_shape<decltype(sid)::value, PEV, SHARE>(cd, eb, prog, eval, own, geo, g1, g2, pl, 64, xl);
+    };
+    using std::integral_constant;
+    if constexpr (NX == 0) {
+      if (!own) f = inverse_channel<PEV>(cd, eb, prog, geo, pl, 64, bank, 64, xl);
     } else if constexpr (NX == 2) {
-      f = inverse_channel<0, PEV>(cd, eb, prog, geo, pl, 64, bank, 64, xl);
+      walk(integral_constant<int, 0>{});
     } else if constexpr (NX == 5) {
-      if (st.shape == 1) f = inverse_channel<1, PEV>(cd, eb, prog, geo, pl, 64, bank, 64, xl);
-      else f = inverse_channel<2, PEV>(cd, eb, prog, geo, pl, 64, bank, 64, xl);
+      if (st.shape == 1) walk(integral_constant<int, 1>{});
+      else walk(integral_constant<int, 2>{});
     } else {
       switch (st.shape) {
-        case 3: f = inverse_channel<3, PEV>(cd, eb, prog, geo, pl, 64, bank, 64, xl); break;
-        case 4: f = inverse_channel<4, PEV>(cd, eb, prog, geo, pl, 64, bank, 64, xl); break;
-        case 5: f = inverse_channel<5, PEV>(cd, eb, prog, geo, pl, 64, bank, 64, xl); break;
-        case 6: f = inverse_channel<6, PEV>(cd, eb, prog, geo, pl, 64, bank, 64, xl); break;
-        default: f = inverse_channel<7, PEV>(cd, eb, prog, geo, pl, 64, bank, 64, xl); break;
+        case 3: walk(integral_constant<int, 3>{}); break;
+        case 4: walk(integral_constant<int, 4>{}); break;
+        case 5: walk(integral_constant<int, 5>{}); break;
+        case 6: walk(integral_constant<int, 6>{}); break;
+        default: walk(integral_constant<int, 7>{}); break;
       }
     }
+    if (own) continue;
     if (valid) f_row[c] = f;
     wave_sync();
     store_rows<NX>(xs, cnt, n_x, aligned != 0, x_rows + (int64_t)c * n_rows * n_x);
@@ -786,9 +898,10 @@ namespace {
 
 template <bool PEV>
 auto pick_shared(const InverseTables& it) {
-  if (it.generic) return inverse_kernel_shared<PEV, 0, 0>;
-  return it.n_x == 2 ? inverse_kernel_shared<PEV, 2, 3>
-                     : it.n_x == 5 ? inverse_kernel_shared<PEV, 5, 3> : inverse_kernel_shared<PEV, 8, 3>;
+  if (it.generic) return inverse_kernel_shared<PEV, 0, false, 0>;
+  if (it.n_x == 2) return inverse_kernel_shared<PEV, 2, false, 3>;
+  if (it.n_x == 5) return it.shared_branches ? inverse_kernel_shared<PEV, 5, true, 3> : inverse_kernel_shared<PEV, 5, false, 3>;
+  return it.shared_branches ? inverse_kernel_shared<PEV, 8, true, 3> : inverse_kernel_shared<PEV, 8, false, 3>;
 }
 
 }  // namespace

@@ -81,12 +81,13 @@ struct InvSeg {
   int32_t pad;
   int64_t row0;
 };
-// One channel of the inverse's channel order: channels whose roots share their evaluation
-// (the same daughters' final-state particles, added in the same association) follow one
-// another, and the first of each group has new_group set.
+// One channel of the inverse's channel order: channels whose trees agree from the root down (the
+// same daughters' final-state particles, added in the same association) follow one another, and
+// bit i of eval marks that the branch visited i-th differs from the last one evaluated there (bits
+// above 0 only for trees of up to four final-state particles).
 struct InvStep {
   int32_t channel;
-  int32_t new_group;
+  int32_t eval;
   int32_t node0;   // the channel's first NodeCmd
   int32_t shape;   // its tree shape
 };
@@ -101,6 +102,7 @@ struct InverseTables {
   // shared roots (no friends): the channels in the order of `steps`; save-bank levels of the
   // subtrees deferred below the root
   int shared_roots = 0, rest_banks = 0;
+  int shared_branches = 0;   // enough branches below the roots repeat from step to step
   int generic = 0;   // some channel's program has none of the shapes of up to four final-state particles
 };
 // The inverse walks specialised per tree shape cover the shapes 0 .. kInvShapes - 1 of the

@@ -325,9 +325,10 @@ constexpr double kAtanR4 = 0x1.921fb54442d18p-1, kAtanR4Lo = 0x1.1a62633145c07p-
 GPHS_MATH_FN double atan_radians(double x) {
   const double ax = __builtin_fabs(x);
   const bool swap = ax > 1.0;
-  const double a = swap ? 1.0 / ax : ax;
+  const Divisor by_ax = divisor(ax);
+  const double a = swap ? divide(1.0, by_ax) : ax;
   // 1 / ax = a + a_lo (the residual of the division; 0 where 1 / ax is no longer normal)
-  const double a_lo = swap && ax < 0x1p1000 ? __builtin_fma(-a, ax, 1.0) / ax : 0.0;
+  const double a_lo = swap && ax < 0x1p1000 ? __builtin_fma(-a, ax, 1.0) * by_ax.r : 0.0;
   const double k = __builtin_rint(4.0 * a);
   const double c = 0.25 * k;
   const double num = a - c;                                  // exact (Sterbenz)
@@ -336,8 +337,9 @@ GPHS_MATH_FN double atan_radians(double x) {
   const double pce = __builtin_fma(a, c, -pc) + a_lo * c;
   const double den_hi = 1.0 + pc;
   const double den_lo = ((1.0 - den_hi) + pc) + pce;
-  const double t = num / den_hi;
-  const double t_lo = (__builtin_fma(-t, den_hi, num) + (a_lo - t * den_lo)) / den_hi;
+  const Divisor by_den = divisor(den_hi);
+  const double t = divide(num, by_den);
+  const double t_lo = (__builtin_fma(-t, den_hi, num) + (a_lo - t * den_lo)) * by_den.r;
   const double z = t * t;
   double p = GPHS_LIN(z, 1.0 / 17.0, -1.0 / 15.0);
   p = GPHS_FMA(p, z, 1.0 / 13.0);

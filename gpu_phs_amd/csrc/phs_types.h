@@ -87,8 +87,10 @@ struct NodeCmd {
   double m;          // map mass of this branch (cos-theta constants per event)
   double db_dm[2];   // d b[k] / d M (adjoint)
   double inv_b0, inv_2b1;   // rounded 1 / b0 and 1 / (2 b1) of a peaked cos-theta map (inverse mapping)
+  double pad1[2];
   ChildCmd k[2];
 };
+static_assert(sizeof(NodeCmd) % 64 == 0, "every record starts on a line of the scalar cache");
 
 struct ChannelDesc {
   int32_t node0;     // first NodeCmd
