@@ -313,99 +313,151 @@ __device__ __forceinline__ void store_momenta(const double* __restrict__ ps, int
   }
 }
 
+// One sub-tile: up to B events of tile `td` from its event `base` on, momenta through the table
+// ps (LDS, rows of B + 1 doubles).
+template <int BANK, int XN, bool FR, bool PEV, int SID, int BLK>
+__device__ __forceinline__ void forward_sub_tile(const TileDesc& td, const SegDesc& sd, const ChannelDesc& cd,
+                                                 const NodeCmd* __restrict__ prog, int base, int B,
+                                                 double* __restrict__ ps, double* __restrict__ xs, double* bank_base) {
+  constexpr int kNout = SID >= 0 ? kShapes[SID < 0 ? 0 : SID].n_out : 0;
+  const int S = B + 1, lane = (int)threadIdx.x;
+  const int cnt = min(B, td.count - base);
+  const int64_t e0 = td.e0 + base;
+  const bool valid = lane < cnt;
+  // lanes past the end of a sub-tile repeat its last event and store nothing
+  const int64_t e = e0 + (valid ? lane : cnt - 1);
+  double factor;
+  bool ok;
+  // (loading the next sub-tile's randoms during this one measured slower: the extra
+  // registers cost a wave per SIMD)
+  double xv[XN > 0 ? XN : 1];
+  load_randoms<XN, SID>(sd.x + e * cd.n_x, cd.n_x, xv, xs + lane, S);
+  EvBeams eb;
+  if constexpr (PEV) eb = event_beams(cd, as_global(sd.e1)[e], as_global(sd.e2)[e]);
+  else eb = fixed_beams(cd);
+  // the msq output is wave-uniform; lanes past the end write their (repeated) last event's
+  // values again, identical ones
+  const bool want_msq = sd.msq != nullptr;
+  gdouble* msq_row = want_msq ? as_global(sd.msq) + e * ((1 << cd.n_out) - 1) : nullptr;
+  forward_event<BANK, XN, FR, PEV, SID>(cd, eb, prog, xv, ps + lane, xs + lane, S, bank_base, want_msq, msq_row,
+                                        factor, ok);
+  if (valid) {
+    __builtin_nontemporal_store(factor, as_global(sd.factor) + e0 + lane);
+    __builtin_nontemporal_store(eb.volume, as_global(sd.volume) + e0 + lane);
+    as_global(sd.ok)[e0 + lane] = ok ? 1 : 0;
+  }
+  __syncthreads();
+  store_momenta<kNout, BLK>(ps, S, cnt, cd, sd.align16 & 2, sd.p + e0 * (int64_t)cd.n_out * 4);
+}
+
 // WPE > 0 asks the register allocator for at least WPE waves per SIMD (fewer VGPRs, spills
 // allowed); the autotuner measures which occupancy target wins.
 //
 // LDS per workgroup (S = blockDim.x + 1 doubles per row): momenta 4 nout_max rows, the
 // randoms nx_max rows (XN = kXLds), then the save banks (BANK = BK_LDS).  A tile of `count`
-// events is done in sub-tiles of blockDim.x events.
+// events is done in sub-tiles of blockDim.x events, ept of them in the largest tile.
 //
 // BLK > 0: the workgroup size is that compile-time constant (shape kernels), so the LDS offsets
 // of the momentum table and of the store phase are immediates.
 //
-// ONE: the launch has one workgroup per tile and tiles of at most blockDim.x events, so each
-// loop below makes one pass; both end after it, so that they are no loops to the compiler,
-// which would otherwise keep constants hoisted out of them in vector registers (the kernels of
-// 2-4 final-state particles: 118 instead of 159 VGPRs, four waves per SIMD instead of three).
+// ONE: the launch has one workgroup per sub-tile (ept per tile), so there is no loop, out of
+// which the compiler would keep constants hoisted in vector registers (the kernels of 2-4
+// final-state particles: 118 instead of 159 VGPRs, four waves per SIMD instead of three; of six:
+// 150-160 instead of 199-205, three instead of two).
 template <int BANK, int WPE, int XN, bool FR, bool PEV, int SID, int BLK, bool ONE = false>
 __global__ __launch_bounds__(BLK > 0 ? BLK : 256) __attribute__((amdgpu_waves_per_eu(WPE > 0 ? WPE : 1)))
-void forward_kernel(const TileDesc* __restrict__ tiles, int t_begin, int t_end, const SegDesc* __restrict__ segs,
-                    const ChannelDesc* __restrict__ chans, const NodeCmd* __restrict__ nodes, int nx_max,
-                    int nout_max) {
+void forward_kernel(const TileDesc* __restrict__ tiles, int t_begin, int t_end, int ept,
+                    const SegDesc* __restrict__ segs, const ChannelDesc* __restrict__ chans,
+                    const NodeCmd* __restrict__ nodes, int nx_max, int nout_max) {
   const int B = BLK > 0 ? BLK : (int)blockDim.x;
   const int S = B + 1;
   double* ps = lds;
   double* xs = ps + 4 * nout_max * S;
   double* bank_base = xs + (XN == kXLds ? nx_max * S : 0);
-  const int lane = (int)threadIdx.x;
-  constexpr int kNout = SID >= 0 ? kShapes[SID < 0 ? 0 : SID].n_out : 0;
-  for (int t = t_begin + (int)blockIdx.x; t < t_end; t += (int)gridDim.x) {
-    const TileDesc td = tiles[t];
+  if constexpr (ONE) {
+    const int tl = (int)((unsigned)blockIdx.x / (unsigned)ept), base = ((int)blockIdx.x - tl * ept) * B;
+    const TileDesc td = tiles[t_begin + tl];
+    if (base >= td.count) return;
     const SegDesc sd = segs[td.seg];
     const ChannelDesc cd = chans[sd.channel];
-    const NodeCmd* prog = nodes + cd.node0;
-    // lanes past the end of a sub-tile repeat its last event and store nothing
-    auto event_of = [&](int base) -> int64_t {
-      const int cnt = min(B, td.count - base);
-      return td.e0 + base + (lane < cnt ? lane : cnt - 1);
-    };
-    for (int base = 0; base < td.count; base += B) {
-      const int cnt = min(B, td.count - base);
-      const int64_t e0 = td.e0 + base;
-      const bool valid = lane < cnt;
-      double factor;
-      bool ok;
-      __syncthreads();   // the previous sub-tile's momentum table has been read
-      const int64_t e = event_of(base);
-      // (loading the next sub-tile's randoms during this one measured slower: the extra
-      // registers cost a wave per SIMD)
-      double xv[XN > 0 ? XN : 1];
-      load_randoms<XN, SID>(sd.x + e * cd.n_x, cd.n_x, xv, xs + lane, S);
-      EvBeams eb;
-      if constexpr (PEV) eb = event_beams(cd, as_global(sd.e1)[e], as_global(sd.e2)[e]);
-      else eb = fixed_beams(cd);
-      // the msq output is wave-uniform; lanes past the end write their (repeated) last event's
-      // values again, identical ones
-      const bool want_msq = sd.msq != nullptr;
-      gdouble* msq_row = want_msq ? as_global(sd.msq) + e * ((1 << cd.n_out) - 1) : nullptr;
-      forward_event<BANK, XN, FR, PEV, SID>(cd, eb, prog, xv, ps + lane, xs + lane, S, bank_base, want_msq, msq_row,
-                                            factor, ok);
-      if (valid) {
-        __builtin_nontemporal_store(factor, as_global(sd.factor) + e0 + lane);
-        __builtin_nontemporal_store(eb.volume, as_global(sd.volume) + e0 + lane);
-        as_global(sd.ok)[e0 + lane] = ok ? 1 : 0;
+    forward_sub_tile<BANK, XN, FR, PEV, SID, BLK>(td, sd, cd, nodes + cd.node0, base, B, ps, xs, bank_base);
+  } else {
+    for (int t = t_begin + (int)blockIdx.x; t < t_end; t += (int)gridDim.x) {
+      const TileDesc td = tiles[t];
+      const SegDesc sd = segs[td.seg];
+      const ChannelDesc cd = chans[sd.channel];
+      for (int base = 0; base < td.count; base += B) {
+        __syncthreads();   // the previous sub-tile's momentum table has been read
+        forward_sub_tile<BANK, XN, FR, PEV, SID, BLK>(td, sd, cd, nodes + cd.node0, base, B, ps, xs, bank_base);
       }
-      __syncthreads();
-      store_momenta<kNout, BLK>(ps, S, cnt, cd, sd.align16 & 2, sd.p + e0 * (int64_t)cd.n_out * 4);
-      if constexpr (ONE) break;
     }
-    if constexpr (ONE) break;
   }
 }
 
-using FwdKernel = void (*)(const TileDesc*, int, int, const SegDesc*, const ChannelDesc*, const NodeCmd*, int, int);
+// The bank of a shape's kernel: the root's boost parameters when only the root defers a daughter,
+// one level of registers when another branch does.
+template <int SID>
+constexpr int shape_bank() {
+  return kShapes[SID].banks == 0 ? BK_NONE : (kShapes[SID].root_only ? BK_ROOT : BK_VGPR);
+}
 
-// Kernels specialised for one tree shape: randoms in the shape's n_x registers, the root's
-// boost parameters as the save bank when only the root defers a daughter, one level of
-// registers when another branch does, fixed beams, no friends.
-template <int SID, int WPE, int BLK, bool ONE = false>
+// Sub-tiles of several shapes in one launch: every workgroup takes the code specialised for its
+// tile's shape, one of [LO, HI).  A launch lasts at least one wave's lifetime however few tiles it
+// has, so the shapes that are too small for a launch of their own share this one.  The tiles are
+// sorted by shape: the waves of a CU mostly run the same code.
+template <int LO, int HI, bool PEV, int BLK>
+__device__ __forceinline__ void sub_tile_of_shape(int shape, const TileDesc& td, const SegDesc& sd,
+                                                  const ChannelDesc& cd, const NodeCmd* __restrict__ prog, int base) {
+  if constexpr (HI - LO == 1) {
+    forward_sub_tile<shape_bank<LO>(), kShapes[LO].n_x, false, PEV, LO, BLK>(td, sd, cd, prog, base, BLK, lds, lds,
+                                                                             nullptr);
+  } else {
+    constexpr int MID = (LO + HI) / 2;
+    if (shape < MID) sub_tile_of_shape<LO, MID, PEV, BLK>(shape, td, sd, cd, prog, base);
+    else sub_tile_of_shape<MID, HI, PEV, BLK>(shape, td, sd, cd, prog, base);
+  }
+}
+
+template <int LO, int HI, int WPE, bool PEV, int BLK>
+__global__ __launch_bounds__(BLK) __attribute__((amdgpu_waves_per_eu(WPE)))
+void forward_shapes_kernel(const TileDesc* __restrict__ tiles, int t_begin, int t_end, int ept,
+                           const SegDesc* __restrict__ segs, const ChannelDesc* __restrict__ chans,
+                           const NodeCmd* __restrict__ nodes, int nx_max, int nout_max) {
+  const int tl = (int)((unsigned)blockIdx.x / (unsigned)ept), base = ((int)blockIdx.x - tl * ept) * BLK;
+  const TileDesc td = tiles[t_begin + tl];
+  if (base >= td.count) return;
+  const SegDesc sd = segs[td.seg];
+  const ChannelDesc cd = chans[sd.channel];
+  sub_tile_of_shape<LO, HI, PEV, BLK>(cd.shape, td, sd, cd, nodes + cd.node0, base);
+}
+
+using FwdKernel = void (*)(const TileDesc*, int, int, int, const SegDesc*, const ChannelDesc*, const NodeCmd*, int, int);
+
+// Kernels specialised for one tree shape: randoms in the shape's n_x registers, shape_bank, fixed
+// beams (or with PEV each event's own), no friends.
+template <int SID, int WPE, int BLK, bool ONE = false, bool PEV = false>
 FwdKernel shape_kernel() {
-  constexpr const ShapeProg& sh = kShapes[SID];
-  constexpr int bank = sh.banks == 0 ? BK_NONE : (sh.root_only ? BK_ROOT : BK_VGPR);
-  return forward_kernel<bank, WPE, sh.n_x, false, false, SID, BLK, ONE>;
+  return forward_kernel<shape_bank<SID>(), WPE, kShapes[SID].n_x, false, PEV, SID, BLK, ONE>;
 }
 
 // The shape kernels of shapes [lo, hi) (one translation unit each): the variant for register
 // budget `wpe` and workgroup size `block`, or null for a shape outside the range.
-// one: the launch has one workgroup per tile and tiles of at most `block` events (the
-// one-pass variants of the trees of up to four final-state particles)
-FwdKernel pick_shape_0_8(int sid, int wpe, int block, bool one);
+// *one: on entry, whether the launch has one workgroup per tile (grid 0); on return, whether the
+// kernel is a one-pass variant, to be launched with a workgroup per sub-tile
+FwdKernel pick_shape_0_8(int sid, int wpe, int block, bool* one);
 // per-event beam energies: shapes [0, kPevShapes), the trees of up to four final-state particles
-FwdKernel pick_shape_pev_0_8(int sid, int wpe, int block, bool one);
-FwdKernel pick_shape_8_22(int sid, int wpe, int block, bool one);
-FwdKernel pick_shape_22_36(int sid, int wpe, int block, bool one);
-FwdKernel pick_shape_36_50(int sid, int wpe, int block, bool one);
-FwdKernel pick_shape_50_64(int sid, int wpe, int block, bool one);
+FwdKernel pick_shape_pev_0_8(int sid, int wpe, int block, bool* one);
+FwdKernel pick_shape_8_22(int sid, int wpe, int block, bool* one);
+FwdKernel pick_shape_22_36(int sid, int wpe, int block, bool* one);
+FwdKernel pick_shape_36_50(int sid, int wpe, int block, bool* one);
+FwdKernel pick_shape_50_64(int sid, int wpe, int block, bool* one);
+
+// The kernels of several shapes: of shape group 0 (the trees of 2-4 final-state particles, fixed or
+// per-event beams), 1 (five) and 2 (six), or null for a workgroup size they are not built for.
+FwdKernel pick_shapes_0(int block);
+FwdKernel pick_shapes_pev_0(int block);
+FwdKernel pick_shapes_1(int block);
+FwdKernel pick_shapes_2(int block);
 
 }  // namespace fwd
 

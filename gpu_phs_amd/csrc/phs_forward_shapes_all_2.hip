@@ -1,0 +1,14 @@
+// The one-pass forward kernel of all the shapes of six final-state particles ([22, 64) of the shape
+// table): plans whose shapes are too small for launches of their own.
+#include "phs_forward.h"
+
+namespace gphs {
+namespace fwd {
+
+FwdKernel pick_shapes_2(int block) {
+  static_assert(kShapes[22].n_out == 6 && kShapes[63].n_out == 6 && 64 <= kNumShapes, "shape range");
+  return block == 64 ? forward_shapes_kernel<22, 64, 3, false, 64> : nullptr;
+}
+
+}  // namespace fwd
+}  // namespace gphs

@@ -48,6 +48,13 @@ constexpr int kPevShapes = 8;
 constexpr int kAdjShapes = 8;
 hipError_t launch_forward_shape(const DevicePlan& dp, int sid, int t_begin, int t_end, const LaunchConfig& lc,
                                 hipStream_t stream);
+// The same for tiles of several shapes of one group in one launch: group 0 the trees of up to four
+// final-state particles, 1 of five, 2 of six.  There is no such kernel for persistent grids,
+// per-event beams above four particles and some workgroup sizes (has_shapes_kernel).
+constexpr int shape_group(int n_out) { return n_out <= 4 ? 0 : n_out - 4; }
+bool has_shapes_kernel(const DevicePlan& dp, int group, const LaunchConfig& lc);
+hipError_t launch_forward_shapes(const DevicePlan& dp, int group, int t_begin, int t_end, const LaunchConfig& lc,
+                                 hipStream_t stream);
 
 // Per-lane LDS layout of the adjoint (in doubles, lane-strided): boost parameters of every
 // branch [0, off_in), branch inputs [off_in, off_st), stash [off_st, off_acc), (M, Gamma)

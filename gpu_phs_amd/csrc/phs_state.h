@@ -30,20 +30,26 @@ struct ProcessObj {
 constexpr int kTileClasses = 2;
 constexpr int kMaxStreams = 4;
 
-// A run of consecutive tiles of one tile class whose channels share one tree shape (or -1:
-// channels without a shape).
-using ShapeRun = TileRun;
+// A run of consecutive tiles of one tile class whose channels share one tree shape (sid), or belong
+// to one group of shapes (kRunOfGroup - group), or have no shape (-1), with the algorithmic bytes of
+// its events.
+struct ShapeRun {
+  int sid, begin, end;
+  double bytes;
+};
+constexpr int kRunOfGroup = -2;
 
 struct PlanObj {
   std::vector<gpu_phs_segment> user;       // segments as given
   std::vector<const double*> beam_e1, beam_e2;   // per-event beam energies of each segment, or null
   std::vector<double*> seg_msq;            // per-branch msq output of each segment, or null
   int specialize = 1;                      // 1: trees with a shape run the shape-specialised kernels
-  // a shape whose tiles in a class hold fewer events than this runs in the class's one launch
-  // of the generic kernel instead of a launch of its own (a launch of a few tiles costs about
-  // one wave's lifetime however small it is)
+  // 0: every shape its own launch.  Otherwise the shapes of a group share the group's launch, where
+  // the class's launch shape has such a kernel; where not, a shape whose tiles in the class hold
+  // fewer events than this runs in the class's one launch of the generic kernel
   int64_t merge_below = kMergeBelowDefault;
-  std::vector<ShapeRun> shape_runs[2];     // each tile class split by shape (empty: one generic launch)
+  // each tile class split by shape (empty: one generic launch), and by shape group
+  std::vector<ShapeRun> shape_runs[2], group_runs[2];
   std::vector<ChannelDesc> chans;
   std::vector<NodeCmd> nodes;
   std::vector<SegDesc> segs;
@@ -79,11 +85,6 @@ struct PlanObj {
   int n_streams = 1;
   hipStream_t lane_streams[kMaxStreams - 1] = {};
   hipEvent_t lane_join[kMaxStreams - 1] = {};
-  struct Job {
-    int cls, begin, end, sid;
-    double bytes;   // algorithmic bytes of its events
-  };
-  std::vector<Job> jobs;   // every launch of a run of the plan, heaviest first
   // adjoint: a copy of the tables with the gradient buffers, per-tile partials, tiles by channel
   void* adj_dev = nullptr;
   size_t adj_bytes = 0;

@@ -250,3 +250,47 @@ def test_copy_bandwidth_calibration():
     assert 1000 < gb_s < 8000
     with pytest.raises(G.GpuPhsError):
         G.copy_bandwidth(1024, 1)
+
+
+@pytest.mark.parametrize("cfg", [dict(), dict(block=64, ept=4), dict(block=128, ept=3), dict(block=192, ept=2),
+                                 dict(block=64, ept=16), dict(block=64, ept=2, grid=7)])
+@pytest.mark.parametrize("parts", [(2, 3, 4), (5, 6), (4, 6, 8, "friends")])
+def test_shared_launches_identical_to_own(parts, cfg):
+    """Shapes of one group in one launch (workgroup sizes it is built for, one or several sub-tiles
+    per tile, or the fallback for the others and for persistent grids), channels without a shape
+    beside them, against a launch per shape and the generic kernel: the same bits, also with
+    per-event beams."""
+    torch = _torch()
+    import gpu_phs_amd as G
+    gen = torch.Generator(device="cuda").manual_seed(11)
+    rng = np.random.default_rng(12)
+    segs, bufs, beams = [], [], []
+    for part in parts:
+        proc = W.process_friends(4) if part == "friends" else W.process_large(8, 6) if part == 8 else \
+            W.process_shapes(part, 2)
+        ph = G.ProcessHandle(proc)
+        for c in range(proc.n_channels):
+            n = int(rng.choice([1, 63, 64, 65, 255, 257, 700]))
+            x = torch.rand((n, proc.n_x), dtype=torch.float64, device="cuda", generator=gen)
+            bufs.append(G.EventBuffers.allocate(x, proc.n_out))
+            segs.append((ph, c, bufs[-1]))
+            beams.append([proc.sqrts / 2 * (0.8 + 0.2 * torch.rand(n, dtype=torch.float64, device="cuda", generator=gen))
+                          for _ in range(2)])
+    print("shared launches", parts, cfg, flush=True)
+    plan = G.Plan(segs, **cfg)
+    for events in (False, True):
+        if events:
+            for i, (e1, e2) in enumerate(beams):
+                plan.set_event_beams(i, e1, e2)
+        results = []
+        for merge, specialize in ((1 << 40, True), (200, True), (0, True), (0, False)):
+            plan.set_merge_below(merge)
+            plan.set_specialize(specialize)
+            for b in bufs:
+                b.p.fill_(-3.0), b.factor.fill_(-3.0), b.volume.fill_(-3.0), b.ok.fill_(7)
+            plan.run()
+            torch.cuda.synchronize()
+            results.append([t.clone() for b in bufs for t in (b.p, b.factor, b.volume, b.ok)])
+        for r in results[1:]:
+            for a, b in zip(results[0], r):
+                assert torch.equal(torch.nan_to_num(a), torch.nan_to_num(b))
