@@ -209,6 +209,42 @@ __device__ __forceinline__ void compose_cols03(double (&M)[16], double g, double
   }
 }
 
+// The root's own L1 is a rotation: its parent boost is the identity and its p_decay 0, so g = 1 and
+// bg = 0 (phs_cpu.cpp:195, 568-573).
+struct RootRot {
+  double ct, st, cp, sp;
+};
+
+// M = L1(root) * L1 for a daughter of the root: compose's sums without the products with the zeros and
+// ones of the root's matrix (the same bits, up to the sign of a zero).  COLS03: columns 0 and 3 only.
+template <bool COLS03>
+__device__ __forceinline__ void compose_on_root(double (&M)[16], const RootRot& r, double g, double bg, double ct,
+                                                double st, double cp, double sp) {
+  const double l01 = -bg * st, l03 = bg * ct;
+  const double l11 = ct * cp, l12 = -sp, l13 = st * cp;
+  const double l21 = ct * sp, l22 = cp, l23 = st * sp;
+  const double l31 = -g * st, l33 = g * ct;
+  M[0] = g;
+  M[3] = l03;
+  if (!COLS03) { M[1] = l01; M[2] = 0; }
+#pragma unroll
+  for (int i = 1; i < 3; i++) {
+    const double r1 = r.ct * (i == 1 ? r.cp : r.sp), r2 = i == 1 ? -r.sp : r.cp, r3 = r.st * (i == 1 ? r.cp : r.sp);
+    M[4 * i] = r3 * bg;
+    M[4 * i + 3] = __builtin_fma(r3, l33, __builtin_fma(r2, l23, r1 * l13));
+    if (COLS03) continue;
+    M[4 * i + 1] = __builtin_fma(r3, l31, __builtin_fma(r2, l21, r1 * l11));
+    M[4 * i + 2] = __builtin_fma(r2, l22, r1 * l12);
+  }
+  const double r1 = -r.st, r3 = r.ct;
+  M[12] = r3 * bg;
+  M[15] = __builtin_fma(r3, l33, r1 * l13);
+  if (!COLS03) {
+    M[13] = __builtin_fma(r3, l31, r1 * l11);
+    M[14] = r1 * l12;
+  }
+}
+
 // The beam's direction in the branch's rest frame, n / |n| = (a0, a1, c), with the
 // intermediates the adjoint needs (u0 and u3: the beam's energy and z component seen from the
 // parent frame, n2 = -bg u0 + g u3).

@@ -163,6 +163,7 @@ __device__ __forceinline__ void forward_event(const ChannelDesc& cd, const EvBea
   bool ok = true;
   int depth = 0;
   double cur_m = eb.sqrts;  // sqrt(msq) of the branch being visited, carried from its parent
+  RootRot rot{};
   if (want_msq) msq_row[(1 << cd.n_out) - 2] = s;
 
   auto branch = [&](const int i) {
@@ -196,9 +197,11 @@ __device__ __forceinline__ void forward_event(const ChannelDesc& cd, const EvBea
     const double pk = 0.5 * (sl * rm);
     factor *= f0 * f1 * math::quot(sl, cur_msq);
 
-    // angles and the boost of this branch (phs_cpu.cpp:299-340)
-    const double bg = m > 0 ? cur_p * rm : 0.0;
-    const double g = math::sqrt_phys(1 + bg * bg);
+    // angles and the boost of this branch (phs_cpu.cpp:299-340).  Shape kernels: the root's boost is the
+    // identity (root), and its daughters (on_root) compose onto its rotation
+    const bool root = SID >= 0 && i == 0, on_root = SID >= 0 && i > 0 && kShapes[SID < 0 ? 0 : SID].node[i].parent == 0;
+    const double bg = root ? 0.0 : m > 0 ? cur_p * rm : 0.0;
+    const double g = root ? 1.0 : math::sqrt_phys(1 + bg * bg);
     double sp, cp;
     math::sincos_turns(GPHS_X(W::xphi(nc, i)), sp, cp);  // phi = 2 pi x
     double ct, st, fct;
@@ -209,6 +212,9 @@ __device__ __forceinline__ void forward_event(const ChannelDesc& cd, const EvBea
     // daughters' momenta use are formed.  A branch with a friend takes its polar axis from
     // an incoming beam (phs.cu:853-910).
     if (FR && nc.friend_sign != 0) compose_friend(M, g, bg, ct, st, cp, sp, (double)nc.friend_sign);
+    else if (root) rot = RootRot{ct, st, cp, sp};
+    else if (on_root && leaf0 && leaf1) compose_on_root<true>(M, rot, g, bg, ct, st, cp, sp);
+    else if (on_root) compose_on_root<false>(M, rot, g, bg, ct, st, cp, sp);
     else if (i == 0) set_l1(M, g, bg, ct, st, cp, sp);
     else if (leaf0 && leaf1) compose_cols03(M, g, bg, ct, st, cp, sp);
     else compose(M, g, bg, ct, st, cp, sp);
@@ -221,10 +227,10 @@ __device__ __forceinline__ void forward_event(const ChannelDesc& cd, const EvBea
         const double pc = c == 0 ? pk : -pk;
         const double E = nc.k[c].msq_leaf == 0 ? fabs(pc) : math::sqrt_phys(nc.k[c].msq_leaf + pc * pc);
         // rows of L (E, 0, 0, pc), the second product fused
-        double q0 = __builtin_fma(M[3], pc, M[0] * E);
-        const double q1 = __builtin_fma(M[7], pc, M[4] * E);
-        const double q2 = __builtin_fma(M[11], pc, M[8] * E);
-        double q3 = __builtin_fma(M[15], pc, M[12] * E);
+        double q0 = root ? E : __builtin_fma(M[3], pc, M[0] * E);
+        const double q1 = root ? st * cp * pc : __builtin_fma(M[7], pc, M[4] * E);
+        const double q2 = root ? st * sp * pc : __builtin_fma(M[11], pc, M[8] * E);
+        double q3 = root ? ct * pc : __builtin_fma(M[15], pc, M[12] * E);
         if (eb.bg_lab != 0) {
           const double b0 = eb.g_lab * q0 + eb.bg_lab * q3;
           const double b3 = eb.bg_lab * q0 + eb.g_lab * q3;

@@ -207,7 +207,7 @@ GPHS_MATH_FN double sqrt_phys(double x) {
   g = __builtin_fma(d, h, g);
   d = __builtin_fma(-g, g, x);
   g = __builtin_fma(d, h, g);
-  return (x == 0 || x == __builtin_inf()) ? x : g;
+  return __builtin_amdgcn_class(x, 0x260) ? x : g;   // +-0 or +inf
 #else
   return __builtin_sqrt(x);
 #endif
@@ -256,12 +256,12 @@ GPHS_MATH_FN double tan_radians(double z) {
   double s0, c0;
   sincos_reduced(r, s0, c0);
   const bool odd = ((int)q) & 1;
-  return (odd ? -c0 : s0) / (odd ? s0 : c0);
+  return divide(odd ? -c0 : s0, divisor(odd ? s0 : c0));
 }
 
 // e^x; overflows to +inf above ~709.8 and underflows to 0 below ~-745 like exp().
 GPHS_MATH_FN double exp_bounded(double x) {
-  const double xc = x > 709.8 ? 709.8 : (x < -745.2 ? -745.2 : x);   // keeps k in int range
+  const double xc = __builtin_fmin(__builtin_fmax(x, -745.2), 709.8);   // keeps k in int range
   const double k = __builtin_rint(xc * GPHS_PIN(kLog2e, xc));
   const double r = __builtin_fma(-k, GPHS_PIN(kLn2Lo, k), __builtin_fma(-k, GPHS_PIN(kLn2Hi, k), xc));
   double p = GPHS_LIN(r, 1.0 / 6227020800.0, 1.0 / 479001600.0);
@@ -276,9 +276,7 @@ GPHS_MATH_FN double exp_bounded(double x) {
   p = GPHS_FMA(p, r, 1.0 / 6.0);
   p = __builtin_fma(p, r, 0.5);
   p = __builtin_fma(p, r * r, r) + 1.0;   // 1 + r + r^2 (1/2 + r/6 + ...)
-  // 2^k in two steps, so that 2^k itself need not be representable near the ends of the range
-  const int ki = (int)k;
-  const double y = __builtin_ldexp(__builtin_ldexp(p, ki / 2), ki - ki / 2);
+  const double y = __builtin_ldexp(p, (int)k);   // (rounded once, also where it is no longer normal)
   return x != x ? x : y;
 }
 
@@ -288,7 +286,7 @@ GPHS_MATH_FN double log_bounded(double x) {
   double m = __builtin_frexp(x, &e);   // x = m 2^e, m in [1/2, 1)
   if (m < GPHS_PIN(kSqrtHalf, m)) { m = 2 * m; e -= 1; }
   const double f = m - 1.0;             // exact
-  const double s = f / (2.0 + f);
+  const double s = divide(f, divisor(2.0 + f));
   const double z = s * s;
   double p = GPHS_LIN(z, 1.0 / 21.0, 1.0 / 19.0);
   p = GPHS_FMA(p, z, 1.0 / 17.0);
