@@ -12,6 +12,31 @@ using namespace gphs;
 
 namespace {
 
+// The map constants of a branch as the specialised walks read them: p0, p1, q0, q1 and c are msq_min,
+// msq_max - msq_min, -, -, f (linear); M^2, M Gamma, a0, a1 - a0, a2 (Breit-Wigner); msq_min, a0, msq_max,
+// a1, a2 (the others), with the expressions of the maps themselves.
+InvNode inv_node(const NodeCmd& nc) {
+  InvNode r{};
+  auto inverse = [](double v) { return v != 0 ? 1 / v : 0.0; };
+  for (int d = 0; d < 2; d++) {
+    const ChildCmd& c = nc.k[d];
+    if (c.leaf) continue;
+    InvMap& m = r.map[d];
+    r.kind[d] = c.kind;
+    if (c.kind == MK_LINEAR) m = InvMap{c.msq_min, c.msq_max - c.msq_min, 0, 0, 0, 0, c.f_lin};
+    else if (c.kind == MK_BREIT_WIGNER) m = InvMap{c.m * c.m, c.m * c.w, 0, c.a0, c.a1 - c.a0, 0, c.a2};
+    else m = InvMap{c.msq_min, c.a0, 0, c.msq_max, c.a1, 0, c.a2};
+    m.inv0 = inverse(m.p1);
+    m.inv1 = inverse(m.q1);
+  }
+  r.ct_kind = nc.ct_kind;
+  r.b0 = nc.b0;
+  r.b1 = nc.b1;
+  r.inv_b0 = inverse(nc.b0);
+  r.inv_2b1 = inverse(2 * nc.b1);
+  return r;
+}
+
 // How a daughter's momentum is added up (a sum of two does not depend on their order).
 std::string association(const NodeCmd* prog, const ChildCmd& k) {
   if (k.leaf) return std::to_string(k.out);
@@ -73,6 +98,12 @@ int inverse_prepare(PlanObj& pl, const int64_t* seg_row0, int64_t n_rows) {
     steps[k].channel = c;
     steps[k].node0 = cp.channels[c].node0;
     steps[k].shape = cp.channels[c].shape;
+    steps[k].outs = 0;
+    for (int i = 0; i < cp.channels[c].n_nodes && i < 8; i++)
+      for (int d = 0; d < 2; d++) {
+        const ChildCmd& k2 = cp.nodes[cp.channels[c].node0 + i].k[d];
+        if (k2.leaf) steps[k].outs |= (uint64_t)k2.out << (4 * (2 * i + d));
+      }
     steps[k].eval = 0;
     for (size_t i = 0; i < keys[c].size(); i++) {
       if (i > 0) branches++;
@@ -98,7 +129,8 @@ int inverse_prepare(PlanObj& pl, const int64_t* seg_row0, int64_t n_rows) {
   const size_t o_chans = al(is.size() * sizeof(InvSeg));
   const size_t o_nodes = o_chans + al(cp.channels.size() * sizeof(ChannelDesc));
   const size_t o_steps = o_nodes + al(cp.nodes.size() * sizeof(NodeCmd));
-  const size_t total = o_steps + al(steps.size() * sizeof(InvStep));
+  const size_t o_maps = o_steps + al(steps.size() * sizeof(InvStep));
+  const size_t total = o_maps + al(cp.nodes.size() * sizeof(InvNode));
   if (total > pl.inv_bytes) {
     if (pl.inv_dev) (void)hipFree(pl.inv_dev);
     pl.inv_dev = nullptr;
@@ -112,6 +144,10 @@ int inverse_prepare(PlanObj& pl, const int64_t* seg_row0, int64_t n_rows) {
   std::memcpy(host.data() + o_chans, cp.channels.data(), cp.channels.size() * sizeof(ChannelDesc));
   std::memcpy(host.data() + o_nodes, cp.nodes.data(), cp.nodes.size() * sizeof(NodeCmd));
   std::memcpy(host.data() + o_steps, steps.data(), steps.size() * sizeof(InvStep));
+  for (size_t i = 0; i < cp.nodes.size(); i++) {
+    const InvNode nd = inv_node(cp.nodes[i]);
+    std::memcpy(host.data() + o_maps + i * sizeof(InvNode), &nd, sizeof nd);
+  }
   hipError_t e = hipMemcpy(pl.inv_dev, host.data(), total, hipMemcpyHostToDevice);
   if (e != hipSuccess) return hip_error(e, "hipMemcpy(inverse tables)");
   char* base = (char*)pl.inv_dev;
@@ -119,6 +155,7 @@ int inverse_prepare(PlanObj& pl, const int64_t* seg_row0, int64_t n_rows) {
   pl.inv.chans = (const ChannelDesc*)(base + o_chans);
   pl.inv.nodes = (const NodeCmd*)(base + o_nodes);
   pl.inv.steps = (const InvStep*)(base + o_steps);
+  pl.inv.maps = (const InvNode*)(base + o_maps);
   pl.inv.n_ch = n_ch;
   pl.inv.n_out = cp.spec.n_out;
   pl.inv.n_x = cp.spec.n_x();
@@ -137,9 +174,10 @@ int inverse_prepare(PlanObj& pl, const int64_t* seg_row0, int64_t n_rows) {
   // a repeated branch saves about a third of its channel's work, the tests for it cost a tenth of
   // every channel's: worth it where a quarter of the branches repeat
   pl.inv.shared_branches = shared && 4 * evaluated <= 3 * branches ? 1 : 0;
-  pl.inv.generic = 0;
+  pl.inv.generic = cp.spec.n_out > (pl.dp.per_event_beams ? kInvShapeOutPev : kInvShapeOut) ? 1 : 0;
   for (const ChannelDesc& c : cp.channels)
-    if (c.shape < 0 || c.shape >= kInvShapes) pl.inv.generic = 1;
+    if (c.shape < 0) pl.inv.generic = 1;
+  if (pl.inv.generic || cp.spec.n_out > 4) pl.inv.shared_branches = 0;
   pl.inv_segs = std::move(is);
   pl.inv_process = proc;
   return ok_status();

@@ -95,14 +95,16 @@ struct InvSeg {
 struct InvStep {
   int32_t channel;
   int32_t eval;
-  int32_t node0;   // the channel's first NodeCmd
+  int32_t node0;   // the channel's first NodeCmd (and InvNode)
   int32_t shape;   // its tree shape
+  uint64_t outs;   // final-state slots of its branches' final-state daughters, 4 bits at 4 (2 branch + daughter)
 };
 // Device copies of one process's complete channel table (every channel is a target).
 struct InverseTables {
   const InvSeg* isegs = nullptr;
   const ChannelDesc* chans = nullptr;
   const NodeCmd* nodes = nullptr;
+  const InvNode* maps = nullptr;   // per NodeCmd, for the walks specialised per tree shape
   const InvStep* steps = nullptr;
   int n_ch = 0, n_out = 0, n_x = 0, n_banks = 0, has_friends = 0, per_event_beams = 0;
   int root_bank = 0;   // every deferred subtree is a daughter of the root and no root has a friend
@@ -110,11 +112,11 @@ struct InverseTables {
   // subtrees deferred below the root
   int shared_roots = 0, rest_banks = 0;
   int shared_branches = 0;   // enough branches below the roots repeat from step to step
-  int generic = 0;   // some channel's program has none of the shapes of up to four final-state particles
+  int generic = 0;   // the channels run the walk that reads their structure from the program
 };
-// The inverse walks specialised per tree shape cover the shapes 0 .. kInvShapes - 1 of the
-// compile-time table (the trees of two to four final-state particles).
-constexpr int kInvShapes = 8;
+// The inverse walks specialised per tree shape cover the trees of up to this many final-state
+// particles, with fixed and with per-event beams.
+constexpr int kInvShapeOut = 6, kInvShapeOutPev = 4;
 size_t inverse_lds_bytes(const InverseTables& it, int block);
 // factors [n_rows][n_ch] and x_out [n_ch][n_rows][n_x] for the events of tiles [0, n_tiles), none of
 // which holds more than 64 n_sub events; with shared roots, the channels in n_chunks ranges of steps.

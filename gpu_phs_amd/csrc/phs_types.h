@@ -53,18 +53,7 @@ struct ChildCmd {
   int32_t sum_len;
   int32_t pad1;
   uint64_t sum_code;
-  // rounded reciprocals of the inverse map's divisors (inv_divisor0, inv_divisor1; 0 where the
-  // map divides by something else)
-  double inv0, inv1;
 };
-
-// What x_from_msq divides by in the linear, Breit-Wigner, exponential and t/u maps.
-inline double inv_divisor0(int32_t kind, double a0, double m, double w, double msq_min, double msq_max) {
-  return kind == MK_LINEAR ? msq_max - msq_min : kind == MK_BREIT_WIGNER ? m * w : kind <= MK_TU ? a0 : 0.0;
-}
-inline double inv_divisor1(int32_t kind, double a0, double a1) {
-  return kind == MK_BREIT_WIGNER ? a1 - a0 : kind == MK_EXP || kind == MK_TU ? a1 : 0.0;
-}
 
 constexpr int kSumPush = 14;
 constexpr int kSumMerge = 15;
@@ -86,11 +75,26 @@ struct NodeCmd {
   double m_min;      // sum of leaf masses below the branch
   double m;          // map mass of this branch (cos-theta constants per event)
   double db_dm[2];   // d b[k] / d M (adjoint)
-  double inv_b0, inv_2b1;   // rounded 1 / b0 and 1 / (2 b1) of a peaked cos-theta map (inverse mapping)
-  double pad1[2];
   ChildCmd k[2];
 };
 static_assert(sizeof(NodeCmd) % 64 == 0, "every record starts on a line of the scalar cache");
+
+// What the inverse walks specialised per tree shape read of one branch's maps (fixed beams): all of it
+// in consecutive lines of the scalar cache, so that a wave waits once per branch.
+//
+// InvMap: the constants of an internal daughter's map (x_from_map says which is which), with the
+// rounded reciprocals of what it divides by.
+struct InvMap {
+  double p0, p1, inv0, q0, q1, inv1, c;
+};
+struct InvNode {
+  InvMap map[2];                    // the daughters' maps (0 for a final-state one)
+  double b0, b1, inv_b0, inv_2b1;   // cos-theta constants, 1 / b0 and 1 / (2 b1)
+  int32_t kind[2];                  // MsqKind of the daughters
+  int32_t ct_kind;
+  int32_t pad[9];
+};
+static_assert(sizeof(InvNode) == 192, "three lines of the scalar cache");
 
 struct ChannelDesc {
   int32_t node0;     // first NodeCmd

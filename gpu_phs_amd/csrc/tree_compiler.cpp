@@ -213,10 +213,6 @@ std::string compile_process(const ProcessSpec& sp, CompiledProcess& out) {
       cc.msq_min = ms[k] * ms[k];
       cc.msq_max = m_max * m_max;
       cc.f_lin = (cc.msq_max - cc.msq_min) / (sqrts * sqrts);
-      const double d0 = inv_divisor0(cc.kind, cc.a0, cc.m, cc.w, cc.msq_min, cc.msq_max);
-      const double d1 = inv_divisor1(cc.kind, cc.a0, cc.a1);
-      cc.inv0 = d0 != 0 ? 1 / d0 : 0;
-      cc.inv1 = d1 != 0 ? 1 / d1 : 0;
       return "";
     };
 
@@ -261,10 +257,6 @@ std::string compile_process(const ProcessSpec& sp, CompiledProcess& out) {
       nd.db_dm[0] = bb[0].dm; nd.db_dm[1] = bb[1].dm;
       nd.m_min = ms[b];
       nd.m = m;
-      if (nd.ct_kind == CK_PEAKED) {
-        nd.inv_b0 = 1 / nd.b0;
-        nd.inv_2b1 = 1 / (2 * nd.b1);
-      }
       for (int i = 0; i < 2; i++) {
         std::string err = fill_child(k[i], nd.k[i]);
         if (!err.empty()) return err;
