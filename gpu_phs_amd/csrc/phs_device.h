@@ -28,6 +28,39 @@ __device__ __forceinline__ guint8* as_global(uint8_t* p) { return (guint8*)p; }
 
 #define GPHS_PI 3.14159265358979323846
 
+// A wave-uniform value in scalar registers, here: the compiler may not load it later.
+__device__ __forceinline__ void keep_scalar(double& v) {
+  uint64_t b = __builtin_bit_cast(uint64_t, v);
+  asm volatile("" : "+s"(b));
+  v = __builtin_bit_cast(double, b);
+}
+__device__ __forceinline__ void keep_scalar(int32_t& v) { asm volatile("" : "+s"(v)); }
+
+// What the forward pass reads of a branch (fixed beams), all of it loaded at once, before the first branch
+// on it: the wave then waits for its program once per tree branch instead of at each use.
+__device__ __forceinline__ NodeCmd load_branch(const NodeCmd* __restrict__ p, bool leaf0, bool leaf1) {
+  NodeCmd nc = *p;
+  keep_scalar(nc.ct_kind);
+  keep_scalar(nc.m_max);
+  keep_scalar(nc.b0);
+  keep_scalar(nc.b1);
+#pragma unroll
+  for (int c = 0; c < 2; c++) {
+    ChildCmd& k = nc.k[c];
+    if (c == 0 ? leaf0 : leaf1) {
+      keep_scalar(k.out);
+      keep_scalar(k.msq_leaf);
+      keep_scalar(k.m_leaf);
+    } else {
+      keep_scalar(k.kind);
+      keep_scalar(k.a0); keep_scalar(k.a1); keep_scalar(k.a2);
+      keep_scalar(k.m); keep_scalar(k.w);
+      keep_scalar(k.msq_min); keep_scalar(k.msq_max); keep_scalar(k.f_lin);
+    }
+  }
+  return nc;
+}
+
 // msq of an internal daughter and its mapping factor (phs_cpu.cpp:12-61).
 __device__ __forceinline__ void msq_map(const ChildCmd& c, double x, double s, double& msq, double& f) {
   switch (c.kind) {

@@ -166,19 +166,14 @@ __device__ __forceinline__ void x_from_ct(const InvNode& nd, double ct, double& 
 // wave waits for it once (loads left where they are used cost a wait each: some 29 per event and
 // channel of a 2->4 tree, 39% of the waves' time).
 __device__ __forceinline__ InvNode load_node(const InvNode* __restrict__ p) { return *p; }
-__device__ __forceinline__ void keep_scalar(double& v) {
-  uint64_t b = __builtin_bit_cast(uint64_t, v);
-  asm volatile("" : "+s"(b));
-  v = __builtin_bit_cast(double, b);
-}
 template <bool MAP0, bool MAP1>
 __device__ __forceinline__ void arrived(InvNode& nd) {
-  asm volatile("" : "+s"(nd.ct_kind));
+  keep_scalar(nd.ct_kind);
   keep_scalar(nd.b0); keep_scalar(nd.b1); keep_scalar(nd.inv_b0); keep_scalar(nd.inv_2b1);
 #pragma unroll
   for (int d = 0; d < 2; d++) {
     if (!(d == 0 ? MAP0 : MAP1)) continue;
-    asm volatile("" : "+s"(nd.kind[d]));
+    keep_scalar(nd.kind[d]);
     InvMap& m = nd.map[d];
     keep_scalar(m.p0); keep_scalar(m.p1); keep_scalar(m.inv0); keep_scalar(m.q0); keep_scalar(m.q1);
     keep_scalar(m.inv1); keep_scalar(m.c);
