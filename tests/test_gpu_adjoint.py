@@ -493,3 +493,36 @@ def test_adjoint_reduction_over_many_units_per_channel():
     sc = np.abs(full).max()
     print("max rel diff", np.abs(full - parts).max() / sc)
     assert np.abs(full - parts).max() <= 1e-12 * sc
+
+
+@pytest.mark.parametrize("n_out", [3, 6, 8])
+@pytest.mark.parametrize("units", [512, 513, 1537])
+def test_adjoint_reduction_ranges(n_out, units):
+    """The reduction at the edges of its ranges (512 units of 64 events), for each of its widths (up to
+    6, up to 10 and more parameters per channel): the gradients of `units` units, the last of one event,
+    equal the sum of those of pieces of at most 300 units, one range each.  Both are sums of the same
+    fewer than 1e5 terms in trees of depth below 30: 30 * 2^-53 of the sum of magnitudes, which is below
+    1e2 of the largest gradient, so 1e-12 of it.  A repeated call gives the same bits."""
+    import torch
+    import gpu_phs_amd as G
+    proc = W.process_shapes(n_out)
+    ph = G.ProcessHandle(proc)
+    rng = np.random.default_rng(units)
+    n = 64 * (units - 1) + 1
+    channels = [0, min(3, proc.n_channels - 1)]
+    xs = [torch.from_numpy(0.02 + 0.96 * rng.random((k, proc.n_x))).cuda() for k in (n, 77)]
+
+    def gradients(parts):
+        bufs = [G.EventBuffers.allocate(x, proc.n_out) for x in parts]
+        plan = G.Plan([(ph, c, b) for c, b in zip(channels, bufs)])
+        g = [plan.adjoint([torch.empty_like(b.x) for b in bufs], loss_mode=1).cpu().numpy() for _ in range(2)]
+        assert np.array_equal(g[0], g[1])
+        return g[0], np.asarray(plan.param_map()[1])
+
+    print("adjoint reduction", n_out, units, flush=True)
+    full, chan = gradients(xs)
+    pieces = [x.contiguous() for x in xs[0].split(300 * 64)]
+    got = [gradients([p, xs[1]])[0] for p in pieces]
+    big = np.repeat(chan == channels[0], 2)
+    want = np.where(big, sum(g.ravel() for g in got), got[0].ravel())
+    assert np.abs(full.ravel() - want).max() <= 1e-12 * np.abs(full).max()
