@@ -2,6 +2,7 @@
 #include <algorithm>
 #include <cstring>
 
+#include "phs_shapes.h"
 #include "phs_state.h"
 
 namespace gphs {
@@ -146,18 +147,16 @@ int gpu_phs_plan_adjoint(int plan, const gpu_phs_adjoint_segment* adj, int loss_
                                     "give the cotangents (loss_mode 0)");
   int rc = adjoint_prepare(*pl, adj, write_forward);
   if (rc) return rc;
-  // the tile table in runs of one tree shape: a shape of up to four final-state particles
-  // takes the adjoint specialised for it, and consecutive runs of such shapes one launch of the
-  // multi-shape adjoint (so the shapes the forward pass folds into its generic launch, those
-  // with fewer than merge_below events, keep their specialised adjoint); the others the generic
-  // adjoint.  One workgroup per 64-event unit: a persistent grid measured slower (its
-  // workgroups do not all fit the LDS at once), and units without events would cost a
-  // workgroup each.
+  // the tile table in runs of one tree shape, whose adjoint is specialised (the forward pass's merge_below
+  // plays no part); launch_adjoint gives consecutive runs of one group one launch.  Other channels run the
+  // generic adjoint.  One workgroup per 64-event unit: a persistent grid measured slower (its workgroups do
+  // not all fit the LDS at once), and units without events would cost a workgroup each.
   std::vector<TileRun> runs;
+  const int n_shapes = pl->dp.per_event_beams ? kAdjPevShapes : kNumShapes;
   for (int c = 0; c < kTileClasses; c++) {
     for (int t = pl->class_begin[c]; t < pl->class_end[c]; t++) {
       const int sh = pl->chans[pl->segs[pl->tiles[t].seg].channel].shape;
-      const int sid = pl->specialize && sh >= 0 && sh < kAdjShapes ? sh : -1;
+      const int sid = pl->specialize && sh >= 0 && sh < n_shapes ? sh : -1;
       if (runs.empty() || runs.back().sid != sid || runs.back().end != t) runs.push_back(TileRun{sid, t, t + 1});
       else runs.back().end = t + 1;
     }

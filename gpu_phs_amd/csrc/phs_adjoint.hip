@@ -1,20 +1,24 @@
-// Adjoint kernel: per event, the forward pass with a tape, then the reverse sweep
-// (phs_adjoint.h).  One workgroup = one wavefront = 64 events of one tile; the tape, the
-// stash and the lane's (M, Gamma) accumulators live in LDS, lane-strided so every access is
-// conflict-free.  The parameter adjoints of a tile are reduced across the wavefront and
-// written as one partial per tile; a second kernel sums the partials of each channel in a
-// fixed order, so results do not depend on scheduling.
+// Adjoint kernels: per event, the forward pass with a tape, then the reverse sweep (phs_adjoint.h; for a
+// tree shape with fixed beams phs_adjoint_shape.h).  One workgroup = one wavefront = 64 events of one tile;
+// the tape, the stash and the lane's (M, Gamma) accumulators live in LDS, lane-strided so every access is
+// conflict-free.  The parameter adjoints of a tile are reduced across the wavefront and written as one
+// partial per unit; a second kernel sums the partials of each channel in a fixed order, so results do not
+// depend on scheduling.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <utility>
 
 #include "phs_adjoint.h"
+#include "phs_adjoint_shape.h"
 #include "phs_kernels.h"
 #include "phs_shapes.h"
 
 namespace gphs {
 
 namespace {
+
+using adj::wave_sums;
 
 // COMPACT: the stash keeps 15 of its 19 words (only the root defers; phs_adjoint.h).  Word w
 // of a lane is at base[w * 64] (one wavefront per workgroup: consecutive lanes, consecutive
@@ -55,21 +59,7 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
-// The same for the first N of v at once, step by step: N independent exchanges are in flight.
-template <int N, int M>
-__device__ __forceinline__ void wave_sums(double (&v)[M]) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    double other[N];
-#pragma unroll
-    for (int k = 0; k < N; k++) other[k] = __shfl_xor(v[k], o, 64);
-#pragma unroll
-    for (int k = 0; k < N; k++) v[k] += other[k];
-  }
-}
-
 constexpr int kAdjXReg = 8;             // n_x <= 8 <=> n_out <= 4
-constexpr int kAdjMultiShapes = kAdjShapes;   // shapes 0-7 of the table: the trees of 2-4 final-state particles
 constexpr int kSmallParams = 2 * 3;     // (M, Gamma) of the 3 branches of an n_out = 4 tree
 
 // One 64-event unit of the adjoint: sub-tile `sub` of tile t, events [64 sub, 64 sub + 64).
@@ -121,14 +111,8 @@ __device__ __forceinline__ void adjoint_unit(int t, int sub, int n_sub, const Ti
     if (sd.loss) sd.loss[e] = L;
   }
   double* part = gpart + ((int64_t)t * n_sub + sub) * part_stride;
-  if constexpr (SID >= 0) {   // all sums at once: their steps overlap
-    constexpr int kNp = 2 * kShapes[SID].n_nodes;
-    wave_sums<kNp>(accv);
-#pragma unroll
-    for (int v = 0; v < kNp; v++)
-      if (lane == 0) part[v] = accv[v];
-  } else if constexpr (XN > 0) {
-    wave_sums<kSmallParams>(accv);
+  if constexpr (XN > 0) {
+    wave_sums(accv);
 #pragma unroll
     for (int v = 0; v < kSmallParams; v++)
       if (lane == 0 && v < np) part[v] = accv[v];
@@ -140,14 +124,12 @@ __device__ __forceinline__ void adjoint_unit(int t, int sub, int n_sub, const Ti
   }
 }
 
-// The launch covers tiles [t_begin, t_begin + n_units / n_sub): unit u is sub-tile (u % n_sub)
-// of tile t_begin + u / n_sub.  SID >= 0: every tile's channel has that shape; SID = kAdjMulti:
-// every tile's channel has one of the shapes of up to four final-state particles, and each
-// workgroup takes the specialised code of its tile's shape (one launch for several shapes:
-// a launch lasts at least one wave's lifetime, so a launch per shape would add that much per
-// shape).  The register budget keeps two waves per SIMD (at most 256 VGPRs).  PEV: per-event
-// beam energies (loss mode 0).  FR: plans with friend branches (the generic walk, randoms read
-// from memory, accumulators in LDS).
+// The generic adjoint, and the one with per-event beam energies of the trees of up to four final-state
+// particles.  The launch covers tiles [t_begin, t_begin + n_units / n_sub): unit u is sub-tile (u % n_sub)
+// of tile t_begin + u / n_sub.  SID = kAdjMulti: every tile's channel has one of the shapes of up to four
+// final-state particles, and each workgroup takes the specialised code of its tile's shape.  The register
+// budget keeps two waves per SIMD (at most 256 VGPRs).  PEV: per-event beam energies (loss mode 0).  FR:
+// plans with friend branches (the generic walk, randoms read from memory, accumulators in LDS).
 constexpr int kAdjMulti = 1000;
 template <int XN, bool COMPACT, int SID, int LM, bool PEV = false, bool FR = false>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void adjoint_kernel(
@@ -222,7 +204,7 @@ __global__ __launch_bounds__(kReduceThreads) void param_reduce(
 #pragma unroll
     for (int v = 0; v < NP; v++) sum[v] += src[v < part_stride ? v : 0];
   }
-  wave_sums<NP>(sum);
+  wave_sums(sum);
 #pragma unroll
   for (int v = 0; v < NP; v++)
     if (lane == 0) red[wv][v] = sum[v];
@@ -256,27 +238,22 @@ __global__ __launch_bounds__(kReduceThreads) void param_reduce(
   if (tid == 0) done[c] = 0;
 }
 
-using AdjKernel = void (*)(const TileDesc*, int, int, int, const SegDesc*, const ChannelDesc*, const NodeCmd*,
-                           double*, int, AdjLayout);
+using AdjKernel = adj::Kernel;
 
-// The adjoint specialised for a tree shape of up to four final-state particles (n_x <= 8): the
-// randoms in the shape's n_x registers, the accumulators in registers; larger shapes run the
-// generic kernel.
-template <int SID, int LM>
-AdjKernel adj_shape(bool compact) {
-  if constexpr (kShapes[SID].n_out <= 4) {
-    constexpr int xn = kShapes[SID].n_x;
-    return compact ? adjoint_kernel<xn, true, SID, LM> : adjoint_kernel<xn, false, SID, LM>;
-  } else {
-    return nullptr;
-  }
+// The kernel of the shapes [lo, hi] that a launch has (of one group): those of one number of final-state
+// particles, or of all of two to four.  Waves per SIMD: as many as the registers hold without spills, so two
+// for the trees of four with given cotangents (10^6 events: 96 us; at three, with 108 bytes of scratch per
+// lane, 129).
+template <int LM>
+adj::Kernel pick_shapes(int lo, int hi) {
+  if (hi < 1) return adj::shapes_kernel<0, 1, LM, 4>;
+  if (lo >= 1 && hi < 3) return adj::shapes_kernel<1, 3, LM, 3>;
+  if (lo >= 3 && hi < 8) return adj::shapes_kernel<3, 8, LM, LM ? 3 : 2>;
+  if (hi < 8) return adj::shapes_kernel<0, 8, LM, LM ? 3 : 2>;
+  if (hi < 22) return adj::pick_5(LM);
+  return LM ? adj::pick_6_1() : adj::pick_6_0();
 }
-template <int... S>
-AdjKernel adj_pick_seq(int sid, bool compact, int lm, std::integer_sequence<int, S...>) {
-  AdjKernel k = nullptr;
-  (void)((sid == S ? (k = lm ? adj_shape<S, 1>(compact) : adj_shape<S, 0>(compact), true) : false) || ...);
-  return k;
-}
+
 template <int LM>
 AdjKernel adj_generic(const DevicePlan& dp, const AdjLayout& lay) {
   if (dp.has_friends) {   // the host sets no compact stash and keeps the accumulators in LDS
@@ -305,30 +282,24 @@ hipError_t launch_adjoint(const DevicePlan& dp, const AdjLayout& lay, const Tile
   if ((int64_t)dp.n_tiles * n_sub > 0x7fffffff) return hipErrorInvalidValue;
   if (dp.per_event_beams && loss_mode != 0) return hipErrorInvalidValue;
   AdjKernel generic = loss_mode ? adj_generic<1>(dp, lay) : adj_generic<0>(dp, lay);
-  AdjKernel multi = loss_mode ? (lay.compact ? adjoint_kernel<kAdjXReg, true, kAdjMulti, 1>
-                                             : adjoint_kernel<kAdjXReg, false, kAdjMulti, 1>)
-                              : (lay.compact ? adjoint_kernel<kAdjXReg, true, kAdjMulti, 0>
-                                             : adjoint_kernel<kAdjXReg, false, kAdjMulti, 0>);
-  // per-event beams: the shapes of up to four final-state particles take the multi-shape
-  // kernel also for a run of one shape (one kernel, not one per shape)
   AdjKernel multi_pev = lay.compact ? adjoint_kernel<kAdjXReg, true, kAdjMulti, 0, true>
                                     : adjoint_kernel<kAdjXReg, false, kAdjMulti, 0, true>;
-  auto small = [](int sid) { return sid >= 0 && sid < kAdjMultiShapes; };
+  auto group = [](int sid) { return sid < 0 ? -1 : shape_group(kShapes[sid].n_out); };
   for (int r = 0; r < n_runs;) {
-    // consecutive runs of the shapes of up to four final-state particles: one launch
-    int r1 = r + 1, end = runs[r].end;
-    if (small(runs[r].sid))
-      while (r1 < n_runs && small(runs[r1].sid) && runs[r1].begin == end) end = runs[r1++].end;
+    // consecutive runs of shapes of one group: one launch (a launch lasts at least one wave's lifetime)
+    int r1 = r + 1, end = runs[r].end, lo = runs[r].sid, hi = lo;
+    for (; r1 < n_runs && runs[r].sid >= 0 && group(runs[r1].sid) == group(runs[r].sid) && runs[r1].begin == end; r1++) {
+      end = runs[r1].end;
+      lo = std::min(lo, runs[r1].sid);
+      hi = std::max(hi, runs[r1].sid);
+    }
     const int units = (end - runs[r].begin) * n_sub;
-    AdjKernel k = nullptr;
-    if (dp.has_friends) k = generic;
-    else if (dp.per_event_beams) k = small(runs[r].sid) ? multi_pev : generic;
-    else if (r1 - r > 1) k = multi;
-    else if (runs[r].sid >= 0)
-      k = adj_pick_seq(runs[r].sid, lay.compact != 0, loss_mode, std::make_integer_sequence<int, kNumShapes>{});
-    if (!k) k = generic;
+    const bool shapes = lo >= 0 && !dp.has_friends, own = shapes && !dp.per_event_beams;   // own: LDS of its own
+    AdjKernel k = !shapes ? generic
+                  : !own  ? (hi < kAdjPevShapes ? multi_pev : generic)
+                          : (loss_mode ? pick_shapes<1>(lo, hi) : pick_shapes<0>(lo, hi));
     if (units > 0) {
-      hipLaunchKernelGGL(k, dim3(units), dim3(64), shmem, stream, dp.tiles, runs[r].begin, units, n_sub, dp.segs,
+      hipLaunchKernelGGL(k, dim3(units), dim3(64), own ? 0 : shmem, stream, dp.tiles, runs[r].begin, units, n_sub, dp.segs,
                          dp.chans, dp.nodes, gpart, part_stride, lay);
       hipError_t e = hipGetLastError();
       if (e != hipSuccess) return e;

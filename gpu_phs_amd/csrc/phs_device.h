@@ -37,13 +37,16 @@ __device__ __forceinline__ void keep_scalar(double& v) {
 __device__ __forceinline__ void keep_scalar(int32_t& v) { asm volatile("" : "+s"(v)); }
 
 // What the forward pass reads of a branch (fixed beams), all of it loaded at once, before the first branch
-// on it: the wave then waits for its program once per tree branch instead of at each use.
+// on it: the wave then waits for its program once per tree branch instead of at each use.  DERIVS: and the
+// derivatives of the constants.
+template <bool DERIVS = false>
 __device__ __forceinline__ NodeCmd load_branch(const NodeCmd* __restrict__ p, bool leaf0, bool leaf1) {
   NodeCmd nc = *p;
   keep_scalar(nc.ct_kind);
   keep_scalar(nc.m_max);
   keep_scalar(nc.b0);
   keep_scalar(nc.b1);
+  if (DERIVS) { keep_scalar(nc.db_dm[0]); keep_scalar(nc.db_dm[1]); }
 #pragma unroll
   for (int c = 0; c < 2; c++) {
     ChildCmd& k = nc.k[c];
@@ -56,6 +59,8 @@ __device__ __forceinline__ NodeCmd load_branch(const NodeCmd* __restrict__ p, bo
       keep_scalar(k.a0); keep_scalar(k.a1); keep_scalar(k.a2);
       keep_scalar(k.m); keep_scalar(k.w);
       keep_scalar(k.msq_min); keep_scalar(k.msq_max); keep_scalar(k.f_lin);
+#pragma unroll
+      for (int a = 0; DERIVS && a < 3; a++) { keep_scalar(k.da_dm[a]); keep_scalar(k.da_dw[a]); }
     }
   }
   return nc;

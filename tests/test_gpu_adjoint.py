@@ -526,3 +526,50 @@ def test_adjoint_reduction_ranges(n_out, units):
     big = np.repeat(chan == channels[0], 2)
     want = np.where(big, sum(g.ravel() for g in got), got[0].ravel())
     assert np.abs(full.ravel() - want).max() <= 1e-12 * np.abs(full).max()
+
+
+@pytest.mark.parametrize("n_outs,loss_mode,beams,cotangents", [
+    ((5,), 1, None, True), ((5,), 0, (700.0, 350.0), True), ((6,), 1, None, True), ((6,), 0, None, True),
+    ((6,), 0, (350.0, 700.0), True), ((6,), 0, None, False), ((2, 3, 4), 1, None, True), ((4, 2, 6, 5, 3), 0, None, True)])
+def test_shape_adjoint_identical_to_generic_larger(n_outs, loss_mode, beams, cotangents):
+    """Every ordered tree of five and six final-state particles (subtrees deferred by the root and by inner
+    branches), and plans of several particle numbers: the adjoint specialised for the shapes gives the
+    generic adjoint's forward outputs and losses, and its gradients to 1e-12: both evaluate the same sums
+    of fewer than 1e3 products, rounded in another order (1e3 * 2^-53, and as much for their
+    cancellation).  With fixed unequal beams, and without momentum cotangents too."""
+    import torch
+    import gpu_phs_amd as G
+    E1, E2 = beams or (None, None)
+    procs = [W.process_shapes(n) for n in n_outs]
+    handles = [G.ProcessHandle(p, E1=E1, E2=E2) for p in procs]
+    res = []
+    for spec in (True, False):
+        rng = np.random.default_rng(sum(n_outs) + loss_mode)
+        bufs, segs = [], []
+        for p, h in zip(procs, handles):
+            for c in range(p.n_channels):
+                k = 65 + c % 130
+                x = torch.from_numpy(0.02 + 0.96 * rng.random((k, p.n_x))).cuda()
+                bufs.append(G.EventBuffers.allocate(x, p.n_out))
+                segs.append((h, c, bufs[-1]))
+        plan = G.Plan(segs)
+        if not spec:
+            plan.set_specialize(False)
+        g_x = [torch.full_like(b.x, float("nan")) for b in bufs]
+        loss = [torch.zeros(b.x.shape[0], dtype=torch.float64, device="cuda") for b in bufs]
+        gp = [torch.from_numpy(rng.standard_normal(b.p.shape)).cuda() for b in bufs]
+        gf = [torch.from_numpy(rng.standard_normal(b.x.shape[0])).cuda() for b in bufs]
+        print("adjoint", n_outs, loss_mode, "specialised" if spec else "generic", flush=True)
+        gparam = plan.adjoint(g_x, g_p=gp if loss_mode == 0 and cotangents else None, g_f=gf if loss_mode == 0 else None,
+                              loss=loss, loss_mode=loss_mode)
+        torch.cuda.synchronize()
+        host = lambda ts: [t.cpu().numpy() for t in ts]
+        res.append((host(g_x), [gparam.cpu().numpy()], host(loss) + host([b.p for b in bufs]) +
+                    host([b.factor for b in bufs]) + host([b.ok for b in bufs])))
+    (gx, gpar, out), (gx0, gpar0, out0) = res
+    assert sum(b.ok.sum().item() for b in bufs) > 100
+    for a, b in zip(out, out0):
+        assert np.array_equal(a, b, equal_nan=True)
+    for a, b in zip(gx, gx0):
+        assert np.all(np.abs(a - b) <= 1e-12 * np.abs(b).max(axis=-1, keepdims=True))
+    assert np.all(np.abs(gpar[0] - gpar0[0]) <= 1e-12 * np.abs(gpar0[0]).max())
