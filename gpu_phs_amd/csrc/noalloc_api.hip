@@ -122,6 +122,8 @@ int gpu_phs_generate_noalloc(int process, int channel, int64_t n_events, const d
   }
   SegDesc sd{};
   sd.channel = 0;
+  sd.node0 = cd.node0;
+  sd.shape = cd.shape;
   sd.n_events = n_events;
   sd.x = x; sd.p = p; sd.factor = factors; sd.volume = volumes; sd.ok = oks;
   sd.align16 = ((reinterpret_cast<uintptr_t>(x) % 16) == 0 ? 1 : 0) | ((reinterpret_cast<uintptr_t>(p) % 16) == 0 ? 2 : 0);

@@ -570,7 +570,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     const TileDesc td = tiles[t];
     const SegDesc sd = segs[td.seg];
     const ChannelDesc cd = chans[sd.channel];
-    unit_of_shape<LO, HI, LM>(cd.shape, sub, td, sd, cd, nodes + cd.node0,
+    unit_of_shape<LO, HI, LM>(sd.shape, sub, td, sd, cd, nodes + sd.node0,
                               gpart + ((int64_t)t * n_sub + sub) * part_stride, lds);
   }
 }

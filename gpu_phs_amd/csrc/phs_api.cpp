@@ -124,6 +124,8 @@ int plan_build(PlanObj& pl) {
     }
     SegDesc sd{};
     sd.channel = ci;
+    sd.node0 = pl.chans[ci].node0;
+    sd.shape = pl.chans[ci].shape;
     sd.n_events = us.n_events;
     sd.x = us.x; sd.p = us.p; sd.factor = us.factors; sd.volume = us.volumes; sd.ok = us.oks;
     sd.align16 = ((reinterpret_cast<uintptr_t>(us.x) % 16) == 0 ? 1 : 0) |

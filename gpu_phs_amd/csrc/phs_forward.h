@@ -339,7 +339,8 @@ __device__ __forceinline__ void forward_sub_tile(const TileDesc& td, const SegDe
   // (loading the next sub-tile's randoms during this one measured slower: the extra
   // registers cost a wave per SIMD)
   double xv[XN > 0 ? XN : 1];
-  load_randoms<XN, SID>(sd.x + e * cd.n_x, cd.n_x, xv, xs + lane, S);
+  const int n_x = SID >= 0 ? kShapes[SID < 0 ? 0 : SID].n_x : cd.n_x;
+  load_randoms<XN, SID>(sd.x + e * n_x, n_x, xv, xs + lane, S);
   EvBeams eb;
   if constexpr (PEV) eb = event_beams(cd, as_global(sd.e1)[e], as_global(sd.e2)[e]);
   else eb = fixed_beams(cd);
@@ -388,7 +389,7 @@ void forward_kernel(const TileDesc* __restrict__ tiles, int t_begin, int t_end, 
     if (base >= td.count) return;
     const SegDesc sd = segs[td.seg];
     const ChannelDesc cd = chans[sd.channel];
-    forward_sub_tile<BANK, XN, FR, PEV, SID, BLK>(td, sd, cd, nodes + cd.node0, base, B, ps, xs, bank_base);
+    forward_sub_tile<BANK, XN, FR, PEV, SID, BLK>(td, sd, cd, nodes + sd.node0, base, B, ps, xs, bank_base);
   } else {
     for (int t = t_begin + (int)blockIdx.x; t < t_end; t += (int)gridDim.x) {
       const TileDesc td = tiles[t];
@@ -396,7 +397,7 @@ void forward_kernel(const TileDesc* __restrict__ tiles, int t_begin, int t_end, 
       const ChannelDesc cd = chans[sd.channel];
       for (int base = 0; base < td.count; base += B) {
         __syncthreads();   // the previous sub-tile's momentum table has been read
-        forward_sub_tile<BANK, XN, FR, PEV, SID, BLK>(td, sd, cd, nodes + cd.node0, base, B, ps, xs, bank_base);
+        forward_sub_tile<BANK, XN, FR, PEV, SID, BLK>(td, sd, cd, nodes + sd.node0, base, B, ps, xs, bank_base);
       }
     }
   }
@@ -436,7 +437,7 @@ void forward_shapes_kernel(const TileDesc* __restrict__ tiles, int t_begin, int 
   if (base >= td.count) return;
   const SegDesc sd = segs[td.seg];
   const ChannelDesc cd = chans[sd.channel];
-  sub_tile_of_shape<LO, HI, PEV, BLK>(cd.shape, td, sd, cd, nodes + cd.node0, base);
+  sub_tile_of_shape<LO, HI, PEV, BLK>(sd.shape, td, sd, cd, nodes + sd.node0, base);
 }
 
 using FwdKernel = void (*)(const TileDesc*, int, int, int, const SegDesc*, const ChannelDesc*, const NodeCmd*, int, int);

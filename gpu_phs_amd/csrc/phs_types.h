@@ -119,6 +119,9 @@ struct ChannelDesc {
 struct SegDesc {
   int32_t channel;   // index into the plan's channel table
   int32_t align16;   // bit 0: x is 16-byte aligned, bit 1: p is 16-byte aligned
+  // of the channel: a workgroup finds its randoms and its program with what it reads of the segment, while
+  // the channel's record is still on its way (one dependent read less before the first instruction on them)
+  int32_t node0, shape;
   int64_t n_events;
   const double* x;
   double* p;
