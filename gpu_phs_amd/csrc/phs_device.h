@@ -36,6 +36,14 @@ __device__ __forceinline__ void keep_scalar(double& v) {
 }
 __device__ __forceinline__ void keep_scalar(int32_t& v) { asm volatile("" : "+s"(v)); }
 
+// A value that all lanes hold, to scalar registers.
+__device__ __forceinline__ double uniform(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+
 // What the forward pass reads of a branch (fixed beams), all of it loaded at once, before the first branch
 // on it: the wave then waits for its program once per tree branch instead of at each use.  DERIVS: and the
 // derivatives of the constants.

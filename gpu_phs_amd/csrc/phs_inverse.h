@@ -244,16 +244,20 @@ __device__ __forceinline__ void rotate_back(double (&G)[16], double ct, double s
 struct Decay {
   double pk, lam, bg;
 };
-__device__ __forceinline__ Decay decay(double cur_msq, double cur_m, double cur_p, double msq0, double msq1) {
+__device__ __forceinline__ Decay decay(const math::Divisor& by_msq, const math::Divisor& m, double cur_p, double msq0,
+                                       double msq1) {
+  const double cur_msq = by_msq.d, cur_m = m.d;
   const double lda = (cur_msq - msq0 - msq1) * (cur_msq - msq0 - msq1) - 4 * msq0 * msq1;
   const bool pos = lda > 0;
   const double sl = pos ? math::sqrt_phys(lda) : 0.0;
-  const math::Divisor m = math::divisor(cur_m);
   Decay d;
   d.pk = math::divide(sl, {2 * cur_m, 0.5 * m.r});
-  d.lam = pos ? sl / cur_msq : 0.0;
+  d.lam = pos ? math::divide(sl, by_msq) : 0.0;
   d.bg = cur_m > 0 ? math::divide(cur_p, m) : 0.0;
   return d;
+}
+__device__ __forceinline__ Decay decay(double cur_msq, double cur_m, double cur_p, double msq0, double msq1) {
+  return decay(math::divisor(cur_msq), math::divisor(cur_m), cur_p, msq0, msq1);
 }
 
 // Polar and azimuthal angles of the direction v (mappings_gpu.hpp:196-219 inverted): the
@@ -263,11 +267,11 @@ struct Dir {
   double xphi, ct, st, cp, sp;
 };
 __device__ __forceinline__ Dir direction(double v0, double v1, double v2) {
-  const double rho = math::sqrt_phys(v0 * v0 + v1 * v1);
-  const double vv = math::sqrt_phys(v0 * v0 + v1 * v1 + v2 * v2);
+  math::Divisor dr, dv;
+  const double rho = math::sqrt_phys(v0 * v0 + v1 * v1, dr);
+  math::sqrt_phys(v0 * v0 + v1 * v1 + v2 * v2, dv);
   Dir d;
   d.xphi = math::atan2_turns(v1, v0);
-  const math::Divisor dr = math::divisor(rho), dv = math::divisor(vv);
   d.cp = rho > 0 ? math::divide(v0, dr) : 1.0;
   d.sp = rho > 0 ? math::divide(v1, dr) : 0.0;
   d.ct = math::divide(v2, dv);
@@ -292,21 +296,22 @@ __device__ __forceinline__ Dir direction(double v0, double v1, double v2) {
 
 struct RootGeo {
   double msq[2];          // msq of the daughters, from the sums of their final-state momenta
-  double m[2];            // sqrt(msq) of an internal daughter (unused for a final-state one)
+  math::Divisor m[2];     // sqrt(msq) of an internal daughter (unused for a final-state one)
   double lam;             // sqrt(lambda) / s, 0 where lambda <= 0 (phs_cpu.cpp:275-279)
   double pk;              // p_decay = sqrt(lambda) / (2 sqrt(s))
   double xphi;            // phi / 2 pi of daughter 0
   double ct, st, cp, sp;  // cos and sin of its polar and azimuthal angles
 };
 
+// (by_s, by_sqrts: the event's s and sqrt(s))
 __device__ __forceinline__ RootGeo root_geometry(const double (&q0)[4], const double (&q1)[4], bool leaf0, bool leaf1,
-                                                 const EvBeams& eb) {
+                                                 const math::Divisor& by_s, const math::Divisor& by_sqrts) {
   RootGeo r;
   r.msq[0] = q0[0] * q0[0] - q0[1] * q0[1] - q0[2] * q0[2] - q0[3] * q0[3];
   r.msq[1] = q1[0] * q1[0] - q1[1] * q1[1] - q1[2] * q1[2] - q1[3] * q1[3];
-  r.m[0] = leaf0 ? 0.0 : math::sqrt_phys(r.msq[0]);
-  r.m[1] = leaf1 ? 0.0 : math::sqrt_phys(r.msq[1]);
-  const Decay dk = decay(eb.s, eb.sqrts, 0.0, r.msq[0], r.msq[1]);
+  if (!leaf0) math::sqrt_phys(r.msq[0], r.m[0]);
+  if (!leaf1) math::sqrt_phys(r.msq[1], r.m[1]);
+  const Decay dk = decay(by_s, by_sqrts, 0.0, r.msq[0], r.msq[1]);
   r.pk = dk.pk;
   r.lam = dk.lam;
   // G = 1 and bg = 0 at the root: v is daughter 0's momentum
@@ -405,12 +410,13 @@ __device__ __forceinline__ void branch_maps(const ChannelDesc& cd, const EvBeams
 }
 
 template <int SID>
-__device__ __forceinline__ RootGeo root_of(uint64_t outs, const EvBeams& eb, const double* __restrict__ pl) {
+__device__ __forceinline__ RootGeo root_of(uint64_t outs, const math::Divisor& by_s, const math::Divisor& by_sqrts,
+                                           const double* __restrict__ pl) {
   constexpr ShapeNode N = kShapes[SID].node[0];
   double q0[4], q1[4];
   daughter_sum<SID, 0, 0>(outs, pl, q0);
   daughter_sum<SID, 0, 1>(outs, pl, q1);
-  return root_geometry(q0, q1, N.leaf0, N.leaf1, eb);
+  return root_geometry(q0, q1, N.leaf0, N.leaf1, by_s, by_sqrts);
 }
 
 // The rows of G that a branch below the root measures its angles in: v = rows 1 to 3 of B_z(-bg) G on
@@ -468,8 +474,9 @@ __device__ __forceinline__ double inverse_walk(const ChannelDesc& cd, const EvBe
   static_assert(sh.banks <= 1, "one deferred subtree at a time");
   double factor = 1;
   branch_maps<SID, 0, PEV>(cd, eb, rec, g.msq[0], g.msq[1], g.lam, g.xphi, g.ct, xo, factor);
-  double G[16], cur_msq = 0, cur_m = 0, cur_p = 0;
-  double bank[16], bank_msq = 0, bank_m = 0, bank_p = 0;
+  double G[16], cur_msq = 0, cur_p = 0;
+  math::Divisor cur_m{};
+  double bank[16], bank_msq = 0, bank_p = 0;
   static_for<1, sh.n_nodes>([&](auto ic) {
     constexpr int i = decltype(ic)::value;
     constexpr ShapeNode N = sh.node[i];
@@ -483,14 +490,15 @@ __device__ __forceinline__ double inverse_walk(const ChannelDesc& cd, const EvBe
     } else if constexpr (sh.node[i - 1].desc < 0) {   // the subtree deferred below the root
 #pragma unroll
       for (int j = 0; j < 16; j++) G[j] = bank[j];
-      cur_msq = bank_msq; cur_m = bank_m; cur_p = bank_p;
+      cur_msq = bank_msq; cur_p = bank_p;
+      math::sqrt_phys(cur_msq, cur_m);
     }
     double q0[4], q1[4];
     daughter_sum<SID, i, 0>(outs, pl, q0);
     daughter_sum<SID, i, 1>(outs, pl, q1);
     const double msq0 = q0[0] * q0[0] - q0[1] * q0[1] - q0[2] * q0[2] - q0[3] * q0[3];
     const double msq1 = q1[0] * q1[0] - q1[1] * q1[1] - q1[2] * q1[2] - q1[3] * q1[3];
-    const Decay dk = decay(cur_msq, cur_m, cur_p, msq0, msq1);
+    const Decay dk = decay(math::divisor(cur_msq), cur_m, cur_p, msq0, msq1);
     double v[3];
     boost_back<on_root>(G, math::sqrt_phys(1 + dk.bg * dk.bg), dk.bg, q0, v);
     const Dir dr = direction(v[0], v[1], v[2]);
@@ -502,11 +510,10 @@ __device__ __forceinline__ double inverse_walk(const ChannelDesc& cd, const EvBe
 #pragma unroll
         for (int j = 0; j < 16; j++) bank[j] = G[j];
         bank_msq = N.push == 0 ? msq0 : msq1;
-        bank_m = math::sqrt_phys(bank_msq);
         bank_p = N.push == 0 ? dk.pk : -dk.pk;
       }
       cur_msq = N.desc == 0 ? msq0 : msq1;
-      cur_m = math::sqrt_phys(cur_msq);
+      math::sqrt_phys(cur_msq, cur_m);
       cur_p = N.desc == 0 ? dk.pk : -dk.pk;
     }
   });
@@ -547,11 +554,14 @@ __device__ __forceinline__ BranchGeo branch_geometry(uint64_t outs, const RootGe
   root_frame(G, g);
   Decay dk;
   if constexpr (N.parent == 0) {
-    dk = decay(g.msq[slot], g.m[slot], slot == 0 ? g.pk : -g.pk, msq0, msq1);
+    // (the reciprocals of the root's two masses, kept from one branch to the next, took 16 bytes of scratch)
+    dk = decay(g.msq[slot], g.m[slot].d, slot == 0 ? g.pk : -g.pk, msq0, msq1);
   } else {
     boost_back<true>(G, up.gm, up.bg, q0, v);
     rotate_back_root(G, up.ct, up.st, up.cp, up.sp);
-    dk = decay(up.msqi, math::sqrt_phys(up.msqi), slot == 0 ? up.pk : -up.pk, msq0, msq1);
+    math::Divisor m;
+    math::sqrt_phys(up.msqi, m);
+    dk = decay(math::divisor(up.msqi), m, slot == 0 ? up.pk : -up.pk, msq0, msq1);
   }
   BranchGeo r;
   r.gm = math::sqrt_phys(1 + dk.bg * dk.bg);
@@ -624,7 +634,7 @@ __device__ __forceinline__ double inverse_channel(const ChannelDesc& cd, const E
   double G[16];
   root_frame(G, g);
   const int rdesc = prog[0].desc;
-  double cur_msq = g.msq[rdesc], cur_m = g.m[rdesc], cur_p = rdesc == 0 ? g.pk : -g.pk;
+  double cur_msq = rdesc == 0 ? g.msq[0] : g.msq[1], cur_m = rdesc == 0 ? g.m[0].d : g.m[1].d, cur_p = rdesc == 0 ? g.pk : -g.pk;
   bool root_pending = prog[0].push >= 0;
   int depth = 0;   // save-bank entries of subtrees deferred below the root
 
@@ -684,8 +694,8 @@ __device__ __forceinline__ double inverse_channel(const ChannelDesc& cd, const E
       root_pending = false;
       const int rp = 1 - rdesc;
       root_frame(G, g);
-      cur_msq = g.msq[rp];
-      cur_m = g.m[rp];
+      cur_msq = rp == 0 ? g.msq[0] : g.msq[1];
+      cur_m = rp == 0 ? g.m[0].d : g.m[1].d;
       cur_p = rp == 0 ? g.pk : -g.pk;
     }
   }
@@ -843,7 +853,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
   }
   if (n_own > 0 && valid) f_row[is.own] = f_own;
   const int k_begin = (int)((int64_t)n_ch * chunk / n_chunks), k_end = (int)((int64_t)n_ch * (chunk + 1) / n_chunks);
-  RootGeo geo;
+  math::Divisor by_s = math::divisor(eb.s), by_sqrts = math::divisor(eb.sqrts);
+  if constexpr (!PEV) {   // the same for all lanes: in scalar registers
+    by_s.r = uniform(by_s.r);
+    by_sqrts.r = uniform(by_sqrts.r);
+  }
+  RootGeo geo{};
   BranchGeo g1, g2;
   for (int k = k_begin; k < k_end; k++) {
     const InvStep st = steps[k];
@@ -857,14 +872,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
         double q0[4], q1[4];
         branch_sum(pl, 64, n_out, prog[0].k[0], q0);
         branch_sum(pl, 64, n_out, prog[0].k[1], q1);
-        geo = root_geometry(q0, q1, prog[0].k[0].leaf, prog[0].k[1].leaf, eb);
+        geo = root_geometry(q0, q1, prog[0].k[0].leaf, prog[0].k[1].leaf, by_s, by_sqrts);
       }
       if (!own) f = inverse_channel<PEV>(cd, eb, prog, geo, pl, 64, bank, 64, xl);
     } else {
       const Records rec{nodes + st.node0, maps + st.node0};
       for_shape<first_shape(NOUT), NOUT == 6 ? kNumShapes : first_shape(NOUT + 1)>(st.shape, [&](auto sid) {
         constexpr int SID = decltype(sid)::value;
-        if (eval & 1) geo = root_of<SID>(st.outs, eb, pl);
+        if (eval & 1) geo = root_of<SID>(st.outs, by_s, by_sqrts, pl);
         if constexpr (SHARE) f = inverse_shared<SID, PEV>(cd, eb, rec, st.outs, eval, own, geo, g1, g2, pl, xl);
         else if (!own) f = inverse_walk<SID, PEV>(cd, eb, rec, st.outs, geo, pl, xl);
       });

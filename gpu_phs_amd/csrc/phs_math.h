@@ -213,6 +213,31 @@ GPHS_MATH_FN double sqrt_phys(double x) {
 #endif
 }
 
+// The same (its bits), and the root as a divisor: the reciprocal that the last steps use, refined once more
+// (2 instructions; divisor's own takes 5, one of them the slow estimate).
+GPHS_MATH_FN double sqrt_phys(double x, Divisor& by) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  double r = __builtin_fma(-h, g, 0.5);
+  g = __builtin_fma(g, r, g);
+  h = __builtin_fma(h, r, h);
+  double d = __builtin_fma(-g, g, x);
+  g = __builtin_fma(d, h, g);
+  d = __builtin_fma(-g, g, x);
+  g = __builtin_fma(d, h, g);
+  r = h + h;
+  r = __builtin_fma(r, __builtin_fma(-g, r, 1.0), r);
+  g = __builtin_amdgcn_class(x, 0x260) ? x : g;
+  by = Divisor{g, r};
+  return g;
+#else
+  const double g = __builtin_sqrt(x);
+  by = Divisor{g, 1.0 / g};
+  return g;
+#endif
+}
+
 // sin and cos of |t| <= pi/4.
 GPHS_MATH_FN void sincos_reduced(double t, double& s, double& c) {
   const double t2 = t * t;
@@ -376,10 +401,16 @@ GPHS_MATH_FN double atan2_turns(double y, double x) {
   const double ax = __builtin_fabs(x), ay = __builtin_fabs(y);
   const bool swap = ay > ax;
   const double num = swap ? ax : ay, den = swap ? ay : ax;
-  const double a = den > 0 ? quot(num, den) : (den == den ? 0.0 : den);
+  // k from the quotient's estimate (an angle past the middle between two k by the estimate's error only adds
+  // that much to |t|), and num - c den and den + c num with one rounding each: one division
+#if defined(__HIP_DEVICE_COMPILE__)
+  const double a = den > 0 ? num * __builtin_amdgcn_rcp(den) : (den == den ? 0.0 : den);
+#else
+  const double a = den > 0 ? num / den : (den == den ? 0.0 : den);
+#endif
   const double k = __builtin_rint(4.0 * a);
   const double c = 0.25 * k;
-  const double t = quot(a - c, __builtin_fma(a, c, 1.0));   // a - c is exact (Sterbenz)
+  const double t = quot(__builtin_fma(-c, den, num), den > 0 ? __builtin_fma(c, num, den) : 1.0);
   const double z = t * t;
   double p = GPHS_LIN(z, 1.0 / 17.0, -1.0 / 15.0);
   p = GPHS_FMA(p, z, 1.0 / 13.0);
