@@ -273,3 +273,31 @@ def test_whizard_abi_large_call_identical_to_plan():
     assert np.array_equal(volumes, cat("volume"))
     assert np.array_equal(factors, f_plan.cpu().numpy(), equal_nan=True)
     assert np.array_equal(x_out, x_plan.cpu().numpy(), equal_nan=True)
+
+
+@pytest.mark.parametrize("counts", [[1, 0, 0], [0, 16_384, 0], [65_535, 0, 1], [65_530, 5, 2], [200_011, 199_989, 200_013]])
+def test_whizard_abi_staging_edges(counts):
+    """The staging of the host copies at its edges: one chunk, the smallest transfer the copy threads take
+    part in, randoms of exactly one 4 MiB chunk and just over, and more than the ring of eight chunks in
+    both directions.  A call gives, bit for bit, the plan API's results, and again when it is repeated."""
+    import torch
+    proc = W.process_c1()
+    L = setup_module_from(proc)
+    n = sum(counts)
+    x = np.random.default_rng(n).random((n, proc.n_x))
+    print("Whizard call", counts, flush=True)
+    first = gen(L, proc, x, counts, 250.0, 250.0)
+    again = gen(L, proc, x, counts, 250.0, 250.0)
+    L.c_whizard_finalize_gpu_phs()
+    ph = G.ProcessHandle(proc)
+    parts = torch.from_numpy(x).cuda().split(counts)
+    used = [c for c, k in enumerate(counts) if k]
+    bufs = [G.EventBuffers.allocate(parts[c], proc.n_out) for c in used]
+    plan = G.Plan([(ph, c, b) for c, b in zip(used, bufs)])
+    plan.run()
+    factors, x_out = plan.inverse()
+    cat = lambda k: torch.cat([getattr(b, k) for b in bufs]).cpu().numpy()
+    want = (cat("p"), factors.cpu().numpy(), cat("volume"), cat("ok").astype(bool), x_out.cpu().numpy())
+    for a, b, c in zip(first, again, want):
+        assert np.array_equal(a, c, equal_nan=True)
+        assert np.array_equal(b, c, equal_nan=True)
