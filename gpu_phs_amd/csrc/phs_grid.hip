@@ -187,7 +187,7 @@ __global__ __launch_bounds__(kGenThreads) void grid_generate_kernel(const TileDe
 // serialise (1.27 million of them, one set per 256-event tile, made the kernel 251 us for 4e6
 // events of 8 randoms in 3 channels).  Four workgroups per CU fill it with loads in flight:
 // 49 us at 1024 workgroups (5.3 TB/s of the randoms), 55 at 512, 87 at 256, 62 at 2048, where the
-// atomics show again.
+// atomics show again; fewer for few events (launch_grid_histogram).
 constexpr int kHistThreads = 512;
 constexpr int kHistGroups = 1024;
 constexpr int kHistUnroll = 8;                                     // loads in flight per thread
@@ -195,7 +195,9 @@ constexpr int kHistField = 6;                                      // bits of a 
 constexpr int kHistPasses = ((1 << kHistField) - 1) / kHistUnroll; // batches before a field is full
 static_assert(kHistField * kGridBins <= 64, "a thread's counts fill one register pair");
 
-__global__ __launch_bounds__(kHistThreads) void grid_histogram_kernel(const TileDesc* __restrict__ tiles, int n_tiles,
+// per_group, extra: workgroup b takes per_group tiles, and one more for b < extra.
+__global__ __launch_bounds__(kHistThreads) void grid_histogram_kernel(const TileDesc* __restrict__ tiles,
+                                                                      int per_group, int extra,
                                                                       const SegDesc* __restrict__ segs,
                                                                       const ChannelDesc* __restrict__ chans, int n_dim,
                                                                       unsigned long long* __restrict__ counts,
@@ -203,20 +205,24 @@ __global__ __launch_bounds__(kHistThreads) void grid_histogram_kernel(const Tile
   extern __shared__ unsigned int hist[];   // n_dim * kGridBins bins, then the accepted count
   const int nb = n_dim * kGridBins;
   const int tid = (int)threadIdx.x;
-  const int t1 = (int)((int64_t)n_tiles * ((int64_t)blockIdx.x + 1) / gridDim.x);
+  const int b0 = (int)blockIdx.x;
+  int t = b0 * per_group + (b0 < extra ? b0 : extra);
+  const int t1 = t + per_group + (b0 < extra ? 1 : 0);
   for (int i = tid; i <= nb; i += kHistThreads) hist[i] = 0;
   __syncthreads();
-  for (int t = (int)((int64_t)n_tiles * blockIdx.x / gridDim.x); t < t1;) {
+  while (t < t1) {
     const TileDesc td = tiles[t];
     const SegDesc sd = segs[td.seg];
     const int n_x = chans[sd.channel].n_x;
-    // the run: this tile and the following ones of its segment, up to the range's end
-    const int64_t left = (sd.n_events - td.e0 + td.count - 1) / td.count;
-    const int run = left < t1 - t ? (int)left : t1 - t;
+    const uint32_t div_nx = chans[sd.channel].div_nx;
+    // the run: this tile and the following ones of its segment, up to the range's end (the 64-bit division
+    // only where the segment ends within it)
+    int run = t1 - t;
+    if (sd.n_events - td.e0 < (int64_t)run * td.count) run = (int)((sd.n_events - td.e0 + td.count - 1) / td.count);
     const int64_t e_run = td.e0 + (int64_t)run * td.count;
     const int64_t e_end = e_run < sd.n_events ? e_run : sd.n_events;
-    const int per = kHistThreads / n_x;   // events per pass
-    const int k = tid % n_x, r = tid / n_x;
+    const int per = (int)__umulhi((uint32_t)kHistThreads, div_nx);   // events per pass
+    const int r = (int)__umulhi((uint32_t)tid, div_nx), k = tid - r * n_x;
     if (r < per) {
       const gdouble* xk = as_global(sd.x) + k;
       const guint8* ok = as_global(sd.ok);
@@ -232,6 +238,14 @@ __global__ __launch_bounds__(kHistThreads) void grid_histogram_kernel(const Tile
       };
       int passes = 0;
       for (int64_t e = td.e0 + r; e < e_end; e += (int64_t)per * kHistUnroll) {
+        if (e_end - (e - r) <= per) {   // one element per thread: counted at once
+          if (ok[e]) {
+            const int b = (int)(xk[e * n_x] * kGridBins);
+            atomicAdd(&hist[k * kGridBins + (b < 0 ? 0 : b > kGridBins - 1 ? kGridBins - 1 : b)], 1u);
+            accepted++;
+          }
+          break;
+        }
         double xv[kHistUnroll];
         unsigned int in[kHistUnroll];
 #pragma unroll
@@ -251,7 +265,7 @@ __global__ __launch_bounds__(kHistThreads) void grid_histogram_kernel(const Tile
         }
         if (++passes == kHistPasses) { flush(); passes = 0; }
       }
-      flush();
+      if (fields) flush();
       if (k == 0 && accepted) atomicAdd(&hist[nb], accepted);
     }
     t += run;
@@ -283,7 +297,7 @@ hipError_t launch_grid_generate(const DevicePlan& dp, const double* cdf, int n_d
   return hipGetLastError();
 }
 
-hipError_t launch_grid_histogram(const DevicePlan& dp, int n_chans, int n_dim, unsigned long long* counts,
+hipError_t launch_grid_histogram(const DevicePlan& dp, int64_t n_events, int n_chans, int n_dim, unsigned long long* counts,
                                  hipStream_t stream) {
   unsigned long long* n_ok = counts + (size_t)n_chans * n_dim * kGridBins;
   const size_t n = (size_t)n_chans * n_dim * kGridBins + n_chans;
@@ -292,8 +306,15 @@ hipError_t launch_grid_histogram(const DevicePlan& dp, int n_chans, int n_dim, u
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || dp.n_tiles <= 0) return e;
   const size_t shmem = ((size_t)n_dim * kGridBins + 1) * sizeof(unsigned int);
-  hipLaunchKernelGGL(grid_histogram_kernel, dim3(std::min(dp.n_tiles, kHistGroups)), dim3(kHistThreads), shmem, stream,
-                     dp.tiles, dp.n_tiles, dp.segs, dp.chans, n_dim, counts, n_ok);
+  // at most a workgroup for each batch of loads beyond the first kHistFew: every workgroup's counts go to the
+  // same few addresses one after the other, some 18 ns each (2 x 10^5 events of 2 randoms: 18 us at one
+  // workgroup per tile, 782; 7.8 at 98), and below that a workgroup per tile ends sooner than one for a
+  // batch of tiles (18,067 events: 5.3 us at 71, 7.6 at 8)
+  constexpr int64_t kHistFew = 128;
+  const int64_t batches = n_events * n_dim / (kHistThreads * kHistUnroll);
+  const int groups = (int)std::min<int64_t>({dp.n_tiles, kHistGroups, std::max(kHistFew, batches)});
+  hipLaunchKernelGGL(grid_histogram_kernel, dim3(groups), dim3(kHistThreads), shmem, stream, dp.tiles,
+                     dp.n_tiles / groups, dp.n_tiles % groups, dp.segs, dp.chans, n_dim, counts, n_ok);
   return hipGetLastError();
 }
 
