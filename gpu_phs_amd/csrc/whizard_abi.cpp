@@ -21,10 +21,11 @@
 namespace gphs {
 namespace {
 
-// Host copies go through a ring of pinned slots in chunks of one slot, on two streams in turn.  Large chunks
-// keep the link busy (32 MiB to the host, one stream and two: 2 MiB chunks 41 and 46 GB/s, 4 MiB 48 and 50,
-// 8 MiB 52 and 53), small ones start the first DMA and end the last host copy early (a call of 10^5 2 -> 4
-// events on one stream: 1.40 ms at 2 MiB, 1.27 at 4, 1.40 at 8).
+// Host copies go through a ring of pinned slots in chunks of one slot, to the host on two streams in turn.
+// Large chunks keep the link busy (32 MiB to the host, one stream and two: 2 MiB chunks 41 and 46 GB/s, 4 MiB 48
+// and 50, 8 MiB 52 and 53), small ones start the first DMA and end the last host copy early (a call of
+// 10^5 2 -> 4 events on one stream: 1.40 ms at 2 MiB, 1.27 at 4, 1.40 at 8).  A second stream for the smaller
+// transfers to the device gained another 0.04 ms, but cost two more calls of 7-14 ms at the start of a process.
 constexpr int kPinSlots = 8;
 constexpr size_t kPinChunk = (size_t)4 << 20;
 
@@ -54,7 +55,7 @@ struct WhizardModule {
   std::unique_ptr<PlanObj> plan;
   std::vector<gpu_phs_segment> plan_segs;
   bool plan_varying = false;
-  // the module's own streams (non-blocking, default priority): kernels and even chunks, and odd chunks
+  // the module's own streams (non-blocking, default priority): kernels and most chunks, and odd chunks to the host
   hipStream_t stream = nullptr, stream2 = nullptr;
   hipEvent_t kernels_ev = nullptr;
   // pinned staging of the host copies: a ring of slots, one chunk each (transfer below)
@@ -226,8 +227,8 @@ struct Transfer {
 
 // Copies the list between the caller's arrays and the device, on the module's stream.  The calling thread
 // issues the DMAs, ahead as far as the ring allows, while the pool copies in pieces between the slots and
-// the caller's memory: a call of 10^5 2 -> 4 events (8 MB in, 35 MB out) takes 1.06 ms, 1.47 array by array with two slots of
-// 16 MiB, whose copies waited for one another wherever an array was a single chunk.
+// the caller's memory: a call of 10^5 2 -> 4 events (8 MB in, 35 MB out) takes 1.10 ms, 1.47 array by array
+// with two slots of 16 MiB, whose copies waited for one another wherever an array was a single chunk.
 // To the device: returns when every DMA is queued.  To the host: when all has arrived.
 int transfer(WhizardModule& w, const std::vector<Transfer>& list, bool to_device) {
   constexpr size_t kPiece = (size_t)256 << 10, kPoolBytes = (size_t)1 << 20;
@@ -254,7 +255,7 @@ int transfer(WhizardModule& w, const std::vector<Transfer>& list, bool to_device
   };
   auto dma = [&](int c) -> hipError_t {
     const Chunk& k = chunks[c];
-    hipStream_t st = c % 2 ? w.stream2 : w.stream;
+    hipStream_t st = c % 2 && !to_device ? w.stream2 : w.stream;
     hipError_t e = to_device ? hipMemcpyAsync(k.dev, slot(c), k.n, hipMemcpyHostToDevice, st)
                              : hipMemcpyAsync(slot(c), k.dev, k.n, hipMemcpyDeviceToHost, st);
     return e != hipSuccess ? e : hipEventRecord(w.pin_ev[c % kPinSlots], st);
@@ -281,9 +282,9 @@ int transfer(WhizardModule& w, const std::vector<Transfer>& list, bool to_device
   auto copied = [&](int c) { return left[c].load(std::memory_order_acquire) == 0; };
 
   hipError_t e = hipSuccess;
-  // the slots' DMAs of the previous transfer; the other stream follows what the module's has queued
+  // the slots' DMAs of the previous transfer; to the host, the other stream follows the kernels
   for (int c = 0; to_device && c < std::min(n, kPinSlots) && e == hipSuccess; c++) e = arrived(c);
-  if (n > 1 && e == hipSuccess && (e = hipEventRecord(w.kernels_ev, w.stream)) == hipSuccess)
+  if (!to_device && n > 1 && (e = hipEventRecord(w.kernels_ev, w.stream)) == hipSuccess)
     e = hipStreamWaitEvent(w.stream2, w.kernels_ev, 0);
   if (e != hipSuccess) return hip_error(e, "staging events");
   const int threads = total >= kPoolBytes ? copy_pool().start(pieces) : 0;
@@ -301,9 +302,6 @@ int transfer(WhizardModule& w, const std::vector<Transfer>& list, bool to_device
       for (; e == hipSuccess && freed + kPinSlots < n && c - freed >= kPinSlots / 2; freed++)
         if ((e = arrived(freed)) == hipSuccess) open.store(freed + kPinSlots + 1, std::memory_order_release);
     }
-    // what is queued on the module's stream next waits for the other stream's last DMA
-    const int last = n - 1 - n % 2;   // the last odd chunk
-    if (e == hipSuccess && last > 0) e = hipStreamWaitEvent(w.stream, w.pin_ev[last % kPinSlots], 0);
   } else {
     for (int c = 0, issued = 0; c < n && e == hipSuccess; c++) {
       // every chunk whose slot has been copied out; at least this one
