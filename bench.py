@@ -170,7 +170,7 @@ def run_inverse(name, steps, warmup, torch, G, W, scale=1.0, block=0):
     return dict(n_events=n, channels=nc, kernel_ms=ms, events_s=n * steps / wall,
                 pairs_s=n * nc * steps / wall, bytes_per_launch=bytes_,
                 hbm_frac=bytes_ / (ms / 1e3) / 1e9 / HBM_PEAK_GBS,
-                block=block or ("library default: 256 for up to 16 channels, else 128"))
+                block=block or ("library default: 64 (every wave works alone)"))
 
 
 def run_event_beams(steps, torch, G, W):
@@ -351,9 +351,8 @@ def cpu_baseline(wl_name, W, threads, scale, budget_s):
 
 # The launch tuning of the c3 mix that the headline line runs and the committed profiles were
 # taken with, confirmed by interleaved repeats of the shapes around it (class 0: 128-thread
-# workgroups, one event per thread, so one workgroup per tile of one sub-tile and the one-pass
-# kernels at the compiler's register budget, four waves per SIMD; class 1: 64 threads, one event
-# per thread, its one-pass kernels at three waves per SIMD; the classes share the GPU).  --autotune tunes
+# workgroups, four waves per SIMD; class 1: 64 threads, three waves per SIMD; one event per thread;
+# each class one launch per group of tree shapes; the classes share the GPU).  --autotune tunes
 # instead, and the full run reports the autotuner's own result beside it (extra.c3_autotuned).
 C3_TUNING = {"classes": [{"block": 128, "ept": 1, "grid": 0, "waves_per_eu": 0, "lds": 0},
                          {"block": 64, "ept": 1, "grid": 0, "waves_per_eu": 0, "lds": 0}],

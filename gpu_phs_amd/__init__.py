@@ -222,8 +222,9 @@ class Plan:
             self.set_config(**config)
 
     def set_merge_below(self, events):
-        """Tree shapes with fewer events than this in a tile class run in the class's generic
-        launch (0: every shape its own specialised launch)."""
+        """0: every tree shape its own launch; above 0 the shapes of a group share one, or, where
+        the launch shape has no such kernel, shapes with fewer events than this in a tile class
+        run in the class's generic launch."""
         _check(lib().gpu_phs_plan_set_merge_below(self.handle, int(events)), "plan_set_merge_below")
 
     def set_streams(self, n_streams):
@@ -314,7 +315,8 @@ class Plan:
                "plan_set_msq_output")
 
     def set_specialize(self, on=True):
-        """Shape-specialised kernels for trees of up to four final-state particles (default on)."""
+        """Shape-specialised forward and adjoint kernels for trees of up to six final-state
+        particles (default on)."""
         _check(lib().gpu_phs_plan_set_specialize(self.handle, 1 if on else 0), "plan_set_specialize")
 
     def run(self, stream=None):

@@ -371,8 +371,8 @@ __device__ __forceinline__ void forward_sub_tile(const TileDesc& td, const SegDe
 //
 // ONE: the launch has one workgroup per sub-tile (ept per tile), so there is no loop, out of
 // which the compiler would keep constants hoisted in vector registers (the kernels of 2-4
-// final-state particles: 118 instead of 159 VGPRs, four waves per SIMD instead of three; of six:
-// 150-160 instead of 199-205, three instead of two).
+// final-state particles: 110 VGPRs instead of 159, four waves per SIMD instead of three; of six:
+// 156 instead of 199-205, three instead of two).
 template <int BANK, int WPE, int XN, bool FR, bool PEV, int SID, int BLK, bool ONE = false>
 __global__ __launch_bounds__(BLK > 0 ? BLK : 256) __attribute__((amdgpu_waves_per_eu(WPE > 0 ? WPE : 1)))
 void forward_kernel(const TileDesc* __restrict__ tiles, int t_begin, int t_end, int ept,

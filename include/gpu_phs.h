@@ -149,10 +149,10 @@ int gpu_phs_plan_destroy(int plan);
  * at least that many waves per SIMD (0 = compiler's choice, 3, 4, or 5: shape-specialised
  * kernels only, others take 5 as 0), lds = bit flags: 1 keeps
  * the boosts of deferred subtrees in LDS instead of VGPRs (trees that defer two levels always
- * use LDS), 2 keeps each event's randoms in LDS instead of VGPRs (always for n_x > 16).  ept 1
- * with grid 0 (one workgroup per tile of one sub-tile) runs the shape-specialised kernels'
- * one-pass variants at the compiler's register budget (fewer registers: four waves per SIMD for
- * trees of up to four final-state particles, three for five and six).  Changing block, ept or order
+ * use LDS), 2 keeps each event's randoms in LDS instead of VGPRs (always for n_x > 16).  With grid 0
+ * every kernel runs one workgroup per sub-tile (block events) and the shape-specialised kernels at
+ * their own register budget (four waves per SIMD for trees of up to four final-state particles,
+ * three for five and six); ept is then only the sub-tiles of a tile.  Changing block, ept or order
  * rebuilds the tile table.  A block whose LDS tables (4 n_out rows of block + 1 doubles, n_x
  * more with randoms in LDS, plus the LDS save banks) exceed the device's per-workgroup LDS is
  * rejected. */
@@ -168,14 +168,15 @@ int gpu_phs_plan_get_class_config(int plan, int cls, int* block, int* ept, int* 
  * other on the caller's stream (serial = 1) or share the GPU (0: the second class on a side
  * stream, joined back by events). */
 int gpu_phs_plan_set_schedule(int plan, int order, int serial);
-/* Tree shapes with fewer than `events` events in a tile class run in that class's one launch of
- * the generic kernel instead of a launch of the kernel specialised for them (default 2^18; 0:
- * every shape its own launch).  A launch however small lasts about one wave's lifetime, so
- * small shapes are cheaper folded into a launch that runs anyway.  No counterpart in the
- * reference. */
+/* 0: every tree shape its own launch.  Above 0 (default 2^18): all shapes of a group (trees of up
+ * to four, of five, of six final-state particles) share one launch, each workgroup on the code
+ * specialised for its tile's shape, since a launch however small lasts about one wave's lifetime.
+ * Where the launch shape has no such kernel (persistent grids, workgroups it is not built for,
+ * per-event beams above four particles), shapes with fewer than `events` events in a tile class run
+ * in that class's launch of the generic kernel.  No counterpart in the reference. */
 int gpu_phs_plan_set_merge_below(int plan, int64_t events);
 /* Number of streams (1..4) the plan's launches spread over: with n_streams > 1 every launch of
- * the plan (one per tree shape, plus the generic one) goes to one of the caller's stream and
+ * the plan (one per group of tree shapes or per shape, plus the generic one) goes to one of the caller's stream and
  * n_streams - 1 side streams, heaviest first onto the least loaded, joined back into the
  * caller's stream by events; the classes' serial flag then does not apply.  A launch ends with
  * its slowest workgroups while the others' slots idle; launches on several streams fill those
@@ -204,9 +205,10 @@ int gpu_phs_plan_set_event_beams(int plan, int segment, const double* E1, const 
  * NULL (the default) turns it off; it costs no memory traffic then.  The array must outlive
  * the plan's use. */
 int gpu_phs_plan_set_msq_output(int plan, int segment, double* msq);
-/* 1 (the default): channels without friends run forward kernels specialised for their tree
- * shape (every ordered tree of 2-6 final-state particles; with per-event beam energies, those of
- * 2-4); 0: every channel runs the generic kernel.  Both give identical results. */
+/* 1 (the default): channels without friends run forward and adjoint kernels specialised for their
+ * tree shape (every ordered tree of 2-6 final-state particles; with per-event beam energies, those
+ * of 2-4); 0: every channel runs the generic kernels.  Both give identical forward results, and
+ * gradients that differ by their rounding. */
 int gpu_phs_plan_set_specialize(int plan, int on);
 /* Forward pass of every segment in one kernel launch on `stream` (hipStream_t, 0 = null). */
 int gpu_phs_plan_run(int plan, void* stream);
@@ -270,8 +272,9 @@ int gpu_phs_generate_noalloc(int process, int channel, int64_t n_events, const d
  * seg_row0[s] is the output row of segment s's first event; outputs are device arrays
  * factors [n_rows][n_channels] and x_out [n_channels][n_rows][n_x] (channel-major, as
  * Whizard reads them, phs.cu:222, 1585).  The generating channel's slot gets the forward
- * factor and randoms.  block: threads per workgroup (64..256; 0: 256 for processes of at most
- * 16 channels, 128 for more, smaller where the LDS tables do not fit).  Where the reference
+ * factor and randoms.  block: threads per workgroup (64..256; 0: 64 for processes without friend
+ * trees, whose waves work alone; with them 256 for at most 16 channels and 128 for more, smaller
+ * where the LDS tables do not fit).  Where the reference
  * has defects (the STEP_H inverse, the T/U inverse of the CPU version, the friend rotation)
  * the inverse of the generating channel returns its randoms instead. */
 int gpu_phs_plan_inverse(int plan, const int64_t* seg_row0, int64_t n_rows, double* factors, double* x_out,
