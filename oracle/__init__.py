@@ -28,7 +28,7 @@ def build(force: bool = False) -> None:
     """Compile liboracle.so, and _ref/libphs_ref.so where the reference tree is present."""
     if force or not os.path.exists(LIB):
         subprocess.run(["make", "-B" if force else "-s", "liboracle.so"], cwd=HERE, check=True)
-    if os.path.isdir(REF_SRC) and (force or not os.path.exists(REF_LIB)):
+    if os.path.exists(os.path.join(REF_SRC, "phs_cpu.cpp")) and (force or not os.path.exists(REF_LIB)):
         subprocess.run(["make", "-B" if force else "-s", "ref"], cwd=HERE, check=True)
 
 
