@@ -44,7 +44,7 @@ __device__ __forceinline__ double uniform(double v) {
   return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
 }
 
-// What the forward pass reads of a branch (fixed beams), all of it loaded at once, before the first branch
+// What the forward pass reads of a branch, all of it loaded at once, before the first branch
 // on it: the wave then waits for its program once per tree branch instead of at each use.  DERIVS: and the
 // derivatives of the constants.
 template <bool DERIVS = false>
@@ -134,17 +134,18 @@ __device__ __forceinline__ EvBeams fixed_beams(const ChannelDesc& cd) {
 
 __device__ __forceinline__ EvBeams event_beams(const ChannelDesc& cd, double E1, double E2) {
   EvBeams b;
-  const double r = math::sqrt_phys(E1 * E2);
+  math::Divisor by_r;
+  const double r = math::sqrt_phys(E1 * E2, by_r);
   b.sqrts = 2 * r;
   b.s = b.sqrts * b.sqrts;
-  b.bg_lab = (E1 - E2) / (2 * r);
+  b.bg_lab = math::divide(E1 - E2, {2 * r, 0.5 * by_r.r});
   b.g_lab = math::sqrt_phys(1 + b.bg_lab * b.bg_lab);
   b.s_friend = 4 * E1 * E2;
   // the phase-space volume (phs_cpu.cpp:195-212): s / (4 (2 pi)^2) per internal branch below
   // the root, 1 / (4 (2 pi)^5) for the root
   double v = 1;
-  for (int i = 1; i < cd.n_nodes; i++) v = v * b.sqrts * b.sqrts / (4 * GPHS_TWOPI2);
-  b.volume = v / (4 * GPHS_TWOPI5);
+  for (int i = 1; i < cd.n_nodes; i++) v = math::divide(v * b.sqrts * b.sqrts, {4 * GPHS_TWOPI2, 1 / (4 * GPHS_TWOPI2)});
+  b.volume = math::divide(v, {4 * GPHS_TWOPI5, 1 / (4 * GPHS_TWOPI5)});
   return b;
 }
 
@@ -152,42 +153,47 @@ __device__ __forceinline__ EvBeams event_beams(const ChannelDesc& cd, double E1,
 // recomputed with the expressions of init_mapping_constants_cpu (phs_cpu.cpp:452-511);
 // a0 of the Breit-Wigner, exponential and t/u maps does not depend on sqrt(s).
 __device__ __forceinline__ ChildCmd child_at(const ChildCmd& c, double sqrts, double s, double m_tot) {
-  ChildCmd r = c;
-  if (c.leaf) return r;
+  if (c.leaf) return c;
   const double m_max = sqrts - m_tot + c.m_min;
   const double msq_min = c.msq_min, msq_max = m_max * m_max, d = msq_max - msq_min;
-  r.msq_max = msq_max;
-  r.f_lin = d / s;
+  // the quotients as correctly rounded ones by divisors, that of s shared by all maps of the event
+  using math::divide;
+  using math::divisor;
+  const math::Divisor by_s = divisor(s);
+  // (in variables of their own: assigned in the copy of the record, they stayed in scratch memory)
+  double a0 = c.a0, a1 = c.a1, a2 = c.a2;
   switch (c.kind) {
-    case MK_LINEAR: r.a1 = d; r.a2 = r.a1 / s; break;
+    case MK_LINEAR: a1 = d; a2 = divide(a1, by_s); break;
     case MK_BREIT_WIGNER: {
       const double msq0 = c.m * c.m;
-      r.a1 = math::atan_radians((msq_max - msq0) / (c.m * c.w));
-      r.a2 = (r.a1 - c.a0) * (c.m * c.w) / s;
+      a1 = math::atan_radians(divide(msq_max - msq0, divisor(c.m * c.w)));
+      a2 = divide((a1 - c.a0) * (c.m * c.w), by_s);
       break;
     }
-    case MK_EXP: r.a1 = math::log_bounded(d / c.a0 + 1); r.a2 = r.a1 / s; break;
-    case MK_TU: r.a1 = 2 * math::log_bounded(d / (2 * c.a0) + 1); r.a2 = r.a1 / s; break;
+    case MK_EXP: a1 = math::log_bounded(divide(d, divisor(c.a0)) + 1); a2 = divide(a1, by_s); break;
+    case MK_TU: a1 = 2 * math::log_bounded(divide(d, divisor(2 * c.a0)) + 1); a2 = divide(a1, by_s); break;
     case MK_STEP_E: {
-      double a2 = 2 * c.m * c.w / d;
+      a2 = 2 * c.m * c.w / d;
       a2 = a2 < 0.01 ? 0.01 : a2;
-      const double a1 = math::exp_bounded(-(c.m * c.m - msq_min) / d / a2);
-      r.a2 = a2;
-      r.a1 = a1;
-      r.a0 = 1 - a2 * math::log_bounded((1 + a1 * math::exp_bounded(1 / a2)) / (1 + a1));
+      a1 = math::exp_bounded(-(c.m * c.m - msq_min) / d / a2);
+      a0 = 1 - a2 * math::log_bounded((1 + a1 * math::exp_bounded(1 / a2)) / (1 + a1));
       break;
     }
     default: {  // MK_STEP_H
-      const double a2 = (c.m * c.m - msq_min) / d;
+      a2 = (c.m * c.m - msq_min) / d;
       const double q = 2 * c.m * c.w / d;
-      double a1 = q * q / a2;
+      a1 = q * q / a2;
       a1 = a1 < 0.000001 ? 0.000001 : a1;
-      r.a2 = a2;
-      r.a1 = a1;
-      r.a0 = (1 + math::sqrt_phys(1 + 4 * a1 / (1 - a2))) / 2;
+      a0 = (1 + math::sqrt_phys(1 + 4 * a1 / (1 - a2))) / 2;
       break;
     }
   }
+  ChildCmd r = c;
+  r.msq_max = msq_max;
+  r.f_lin = divide(d, by_s);
+  r.a0 = a0;
+  r.a1 = a1;
+  r.a2 = a2;
   return r;
 }
 

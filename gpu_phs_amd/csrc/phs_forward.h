@@ -168,8 +168,8 @@ __device__ __forceinline__ void forward_event(const ChannelDesc& cd, const EvBea
 
   auto branch = [&](const int i) {
     NodeCmd held;
-    if constexpr (SID >= 0 && !PEV) held = load_branch(prog + i, W::leaf(prog[i], i, 0), W::leaf(prog[i], i, 1));
-    const NodeCmd& nc = SID >= 0 && !PEV ? held : prog[i];
+    if constexpr (SID >= 0) held = load_branch(prog + i, W::leaf(prog[i], i, 0), W::leaf(prog[i], i, 1));
+    const NodeCmd& nc = SID >= 0 ? held : prog[i];
     const bool leaf0 = W::leaf(nc, i, 0), leaf1 = W::leaf(nc, i, 1);
     double m_max = nc.m_max, cb0 = nc.b0, cb1 = nc.b1;
     if constexpr (PEV) node_at(nc, i == 0, eb, cd.m_tot, m_max, cb0, cb1);
