@@ -3,7 +3,7 @@
 // sqrt(s)-dependent map constants formed in the kernel, as in the generic kernel's per-event
 // variant, with the walk unrolled for the shape.  One-pass variants (one workgroup per sub-tile)
 // for workgroups of 64, 128 and 256 threads at the compiler's register budget, a one-pass kernel of
-// all the shapes (128 VGPRs, four waves per SIMD; 1e6 events of 2->4 44 us, 53 while the maps' constants
+// all the shapes (128 VGPRs, four waves per SIMD; 1e6 events of 2->4 46 us, 53 while the maps' constants
 // went through scratch memory and a branch's were loaded where they are used), and looping ones (persistent grids, other workgroup sizes) at
 // the compiler's budget or one for 3 waves per SIMD (asked for 4 or 5, the kernel takes 3).
 // Larger trees with per-event beams run the generic kernel.
