@@ -65,9 +65,9 @@ __device__ __forceinline__ double in_bin(const BinRec& r, double u) {
 // of the tile table (as the histogram below), builds the tables of a channel once per run of tiles
 // in LDS, and its waves then take 64 events each: every lane puts its event's randoms into its column of the
 // wave's table x[k][lane], and the wave stores the 64 rows as one contiguous run (16-byte words
-// where the row length is even and the rows are 16-byte aligned).  4e6 events of 8 randoms: 70 us
-// (57 VALU instructions per random, the vector units busy throughout; 79 us with both tables at
-// strides whose lanes met the same banks), against 103 us with nine bounds read per random, two
+// where the row length is even and the rows are 16-byte aligned).  4e6 events of 8 randoms: 68 us
+// (56 VALU instructions per random, the vector units 73% busy; 79 us with both tables at strides
+// whose lanes met the same banks), against 103 us with nine bounds read per random, two
 // divisions and a division per word stored.
 constexpr int kGenWaves = 4;
 constexpr int kGenThreads = 64 * kGenWaves;
@@ -75,7 +75,9 @@ constexpr int kGenGroups = 4096;
 constexpr int kGenRow = 68;   // the lanes that read one another's columns meet different LDS banks
 constexpr int kGenCellBits = 6, kGenCells = 1 << kGenCellBits;
 
-__global__ __launch_bounds__(kGenThreads) void grid_generate_kernel(const TileDesc* __restrict__ tiles, int n_tiles,
+// per_group, extra: workgroup b takes per_group tiles, and one more for b < extra.
+__global__ __launch_bounds__(kGenThreads) void grid_generate_kernel(const TileDesc* __restrict__ tiles, int per_group,
+                                                                    int extra,
                                                                     const SegDesc* __restrict__ segs,
                                                                     const ChannelDesc* __restrict__ chans,
                                                                     const double* __restrict__ cdf, int n_dim,
@@ -88,15 +90,19 @@ __global__ __launch_bounds__(kGenThreads) void grid_generate_kernel(const TileDe
   double* xs0 = (double*)(rec + n_dim * kGridBins);
   double* xs = xs0 + wave * n_dim * kGenRow;
   uint8_t* first = (uint8_t*)(xs0 + kGenWaves * n_dim * kGenRow);
-  const int t1 = (int)((int64_t)n_tiles * ((int64_t)blockIdx.x + 1) / gridDim.x);
-  for (int t = (int)((int64_t)n_tiles * blockIdx.x / gridDim.x); t < t1;) {
+  const int b0 = (int)blockIdx.x;
+  int t = b0 * per_group + (b0 < extra ? b0 : extra);
+  const int t1 = t + per_group + (b0 < extra ? 1 : 0);
+  while (t < t1) {
     const TileDesc td = tiles[t];
     const SegDesc sd = segs[td.seg];
     const int n_x = chans[sd.channel].n_x;
+    const uint32_t div_nx = chans[sd.channel].div_nx;
     const double* F0 = cdf + (size_t)sd.channel * n_dim * NB1;
-    // the run: this tile and the following ones of its segment, up to the range's end
-    const int64_t left = (sd.n_events - td.e0 + td.count - 1) / td.count;
-    const int run = left < t1 - t ? (int)left : t1 - t;
+    // the run: this tile and the following ones of its segment, up to the range's end (a 64-bit division
+    // only where the segment ends within it)
+    int run = t1 - t;
+    if (sd.n_events - td.e0 < (int64_t)run * td.count) run = (int)((sd.n_events - td.e0 + td.count - 1) / td.count);
     const int64_t e_run = td.e0 + (int64_t)run * td.count;
     const int64_t e_end = e_run < sd.n_events ? e_run : sd.n_events;
     t += run;
@@ -120,8 +126,8 @@ __global__ __launch_bounds__(kGenThreads) void grid_generate_kernel(const TileDe
     // word w of a wave's rows holds doubles w * step ..: event (w * step) / n_x, random the rest;
     // 64 words on, both advance by constants
     const int step = vec ? 2 : 1;
-    const int ev0 = lane * step / n_x, k0 = lane * step - ev0 * n_x;
-    const int dev = 64 * step / n_x, dk = 64 * step - dev * n_x;
+    const int ev0 = (int)__umulhi((uint32_t)(lane * step), div_nx), k0 = lane * step - ev0 * n_x;
+    const int dev = (int)__umulhi((uint32_t)(64 * step), div_nx), dk = 64 * step - dev * n_x;
     // (tiles start at multiples of 64 events, so an event's low index word is the unit's with the lane)
     for (int64_t e = td.e0 + 64 * wave; e < e_end; e += kGenThreads) {
       const int cnt = e_end - e < 64 ? (int)(e_end - e) : 64;
@@ -239,8 +245,9 @@ __global__ __launch_bounds__(kHistThreads) void grid_histogram_kernel(const Tile
       int passes = 0;
       for (int64_t e = td.e0 + r; e < e_end; e += (int64_t)per * kHistUnroll) {
         if (e_end - (e - r) <= per) {   // one element per thread: counted at once
+          const double xe = xk[e * n_x];
           if (ok[e]) {
-            const int b = (int)(xk[e * n_x] * kGridBins);
+            const int b = (int)(xe * kGridBins);
             atomicAdd(&hist[k * kGridBins + (b < 0 ? 0 : b > kGridBins - 1 ? kGridBins - 1 : b)], 1u);
             accepted++;
           }
@@ -283,6 +290,41 @@ __global__ __launch_bounds__(kHistThreads) void grid_histogram_kernel(const Tile
   }
 }
 
+// The same for few tiles, a workgroup each, a thread per event: nothing to set up, one pass (at most kHistFew
+// tiles: 18,067 events of 2 randoms 3.3 us, 4.6 with the kernel above; 1,003 of 8 3.2 and 5.0).
+constexpr int kHistFew = 128;
+__global__ __launch_bounds__(256) void grid_histogram_few_kernel(const TileDesc* __restrict__ tiles,
+                                                                 const SegDesc* __restrict__ segs,
+                                                                 const ChannelDesc* __restrict__ chans, int n_dim,
+                                                                 unsigned long long* __restrict__ counts,
+                                                                 unsigned long long* __restrict__ n_ok) {
+  extern __shared__ unsigned int hist[];   // n_dim * kGridBins bins, then the accepted count
+  const int nb = n_dim * kGridBins;
+  const TileDesc td = tiles[blockIdx.x];
+  const SegDesc sd = segs[td.seg];
+  const int n_x = chans[sd.channel].n_x;
+  for (int i = (int)threadIdx.x; i <= nb; i += (int)blockDim.x) hist[i] = 0;
+  __syncthreads();
+  for (int local = (int)threadIdx.x; local < td.count; local += (int)blockDim.x) {
+    const int64_t e = td.e0 + local;
+    if (!as_global(sd.ok)[e]) continue;
+    const gdouble* xr = as_global((const double*)sd.x) + e * n_x;
+    for (int k = 0; k < n_x; k++) {
+      int b = (int)(xr[k] * kGridBins);   // rng.cpp:52
+      b = b < 0 ? 0 : b > kGridBins - 1 ? kGridBins - 1 : b;
+      atomicAdd(&hist[k * kGridBins + b], 1u);
+    }
+    atomicAdd(&hist[nb], 1u);
+  }
+  __syncthreads();
+  for (int i = (int)threadIdx.x; i <= nb; i += (int)blockDim.x) {
+    const unsigned int v = hist[i];
+    if (v == 0) continue;
+    if (i < nb) atomicAdd(&counts[(size_t)sd.channel * nb + i], (unsigned long long)v);
+    else atomicAdd(&n_ok[sd.channel], (unsigned long long)v);
+  }
+}
+
 __global__ void fill_u64_kernel(unsigned long long* p, size_t n) {
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = 0;
 }
@@ -292,8 +334,9 @@ __global__ void fill_u64_kernel(unsigned long long* p, size_t n) {
 hipError_t launch_grid_generate(const DevicePlan& dp, const double* cdf, int n_dim, uint64_t seed, hipStream_t stream) {
   if (dp.n_tiles <= 0) return hipSuccess;
   const size_t shmem = (size_t)n_dim * (kGridBins * sizeof(BinRec) + kGenWaves * kGenRow * sizeof(double) + kGenCells);
-  hipLaunchKernelGGL(grid_generate_kernel, dim3(std::min(dp.n_tiles, kGenGroups)), dim3(kGenThreads), shmem, stream,
-                     dp.tiles, dp.n_tiles, dp.segs, dp.chans, cdf, n_dim, seed);
+  const int groups = std::min(dp.n_tiles, kGenGroups);
+  hipLaunchKernelGGL(grid_generate_kernel, dim3(groups), dim3(kGenThreads), shmem, stream, dp.tiles,
+                     dp.n_tiles / groups, dp.n_tiles % groups, dp.segs, dp.chans, cdf, n_dim, seed);
   return hipGetLastError();
 }
 
@@ -306,13 +349,16 @@ hipError_t launch_grid_histogram(const DevicePlan& dp, int64_t n_events, int n_c
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || dp.n_tiles <= 0) return e;
   const size_t shmem = ((size_t)n_dim * kGridBins + 1) * sizeof(unsigned int);
+  if (dp.n_tiles <= kHistFew) {
+    hipLaunchKernelGGL(grid_histogram_few_kernel, dim3(dp.n_tiles), dim3(256), shmem, stream, dp.tiles, dp.segs, dp.chans,
+                       n_dim, counts, n_ok);
+    return hipGetLastError();
+  }
   // at most a workgroup for each batch of loads beyond the first kHistFew: every workgroup's counts go to the
   // same few addresses one after the other, some 18 ns each (2 x 10^5 events of 2 randoms: 18 us at one
-  // workgroup per tile, 782; 7.8 at 98), and below that a workgroup per tile ends sooner than one for a
-  // batch of tiles (18,067 events: 5.3 us at 71, 7.6 at 8)
-  constexpr int64_t kHistFew = 128;
+  // workgroup per tile, 782; 7.8 at 98)
   const int64_t batches = n_events * n_dim / (kHistThreads * kHistUnroll);
-  const int groups = (int)std::min<int64_t>({dp.n_tiles, kHistGroups, std::max(kHistFew, batches)});
+  const int groups = (int)std::min<int64_t>({dp.n_tiles, kHistGroups, std::max<int64_t>(kHistFew, batches)});
   hipLaunchKernelGGL(grid_histogram_kernel, dim3(groups), dim3(kHistThreads), shmem, stream, dp.tiles,
                      dp.n_tiles / groups, dp.n_tiles % groups, dp.segs, dp.chans, n_dim, counts, n_ok);
   return hipGetLastError();

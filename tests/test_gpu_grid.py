@@ -72,6 +72,8 @@ def test_update_matches_oracle_and_adapts():
 
 @pytest.mark.parametrize("n_out,counts,cfg", [
     (4, [1], dict()),                                   # one event
+    (2, [128 * 256], dict()),                           # as many tiles as the kernel for few takes
+    (2, [128 * 256 + 1], dict()),                       # one more
     (2, [1025 * 256 + 7], dict()),                      # one tile more than the workgroups of the histogram
     (3, [1000, 255, 0, 64, 1, 4097], dict(block=64)),   # odd n_x: threads without an element; many short segments
     (6, [300, 70001, 2], dict(block=64, ept=4)),        # several tiles per run, runs that end inside a range
