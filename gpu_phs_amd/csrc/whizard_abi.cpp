@@ -116,14 +116,15 @@ int ensure_inverse_buffers(WhizardModule& w, size_t n) {
 }
 
 void free_staging(WhizardModule& w) {
+  // both streams copy from and to the ring
   if (w.stream) (void)hipStreamSynchronize(w.stream);
+  if (w.stream2) (void)hipStreamSynchronize(w.stream2);
   for (hipEvent_t& ev : w.pin_ev) {
     if (ev) (void)hipEventDestroy(ev);
     ev = nullptr;
   }
   if (w.pin) (void)hipHostFree(w.pin);
   w.pin = nullptr;
-  if (w.stream2) (void)hipStreamSynchronize(w.stream2);
   if (w.kernels_ev) (void)hipEventDestroy(w.kernels_ev);
   if (w.stream2) (void)hipStreamDestroy(w.stream2);
   if (w.stream) (void)hipStreamDestroy(w.stream);
@@ -261,6 +262,12 @@ int transfer(WhizardModule& w, const std::vector<Transfer>& list, bool to_device
     return e != hipSuccess ? e : hipEventRecord(w.pin_ev[c % kPinSlots], st);
   };
   auto arrived = [&](int c) { return hipEventSynchronize(w.pin_ev[c % kPinSlots]); };
+  // no DMA on the slots or the device arrays goes on after a transfer that failed
+  auto failed = [&](hipError_t e, const char* what) {
+    (void)hipStreamSynchronize(w.stream);
+    (void)hipStreamSynchronize(w.stream2);
+    return hip_error(e, what);
+  };
 
   // pieces [kPieces c, kPieces (c + 1)) are chunk c's (those past its end are empty); `open` chunks may be
   // copied so far: arrived from the device, or with a free slot
@@ -286,7 +293,7 @@ int transfer(WhizardModule& w, const std::vector<Transfer>& list, bool to_device
   for (int c = 0; to_device && c < std::min(n, kPinSlots) && e == hipSuccess; c++) e = arrived(c);
   if (!to_device && n > 1 && (e = hipEventRecord(w.kernels_ev, w.stream)) == hipSuccess)
     e = hipStreamWaitEvent(w.stream2, w.kernels_ev, 0);
-  if (e != hipSuccess) return hip_error(e, "staging events");
+  if (e != hipSuccess) return failed(e, "staging events");
   const int threads = total >= kPoolBytes ? copy_pool().start(pieces) : 0;
   auto copy_whole = [&](int c) {   // without threads
     if (threads > 0) return;
@@ -319,7 +326,7 @@ int transfer(WhizardModule& w, const std::vector<Transfer>& list, bool to_device
   }
   if (e != hipSuccess) abort.store(true);
   if (threads > 0) copy_pool().wait();
-  return e == hipSuccess ? GPU_PHS_OK : hip_error(e, to_device ? "host to device copy" : "device to host copy");
+  return e == hipSuccess ? GPU_PHS_OK : failed(e, to_device ? "host to device copy" : "device to host copy");
 }
 
 int compile_for_beams(WhizardModule& w, double E1, double E2) {

@@ -1,0 +1,194 @@
+// The HIP runtime calls of the library's host code, on the CPU, for tests of what that code asks for: device
+// memory is host memory, kernels are counted and not run.  Work on a stream waits until something
+// synchronises with it, the latest that the runtime may do it, so that memory which is released or reused
+// without a wait is seen to be.  Loaded with its symbols global before the library.
+#define __HIP_PLATFORM_AMD__
+#include <hip/hip_runtime_api.h>
+
+#include <chrono>
+#include <cstdlib>
+#include <cstring>
+#include <deque>
+#include <map>
+#include <string>
+#include <thread>
+#include <vector>
+
+struct ihipEvent_t {
+  hipStream_t stream = nullptr;
+  uint64_t op = 0;   // the event is the op of this number on that stream
+};
+
+struct ihipStream_t {
+  struct Op {
+    void* dst;
+    const void* src;
+    size_t n;               // a copy, n > 0
+    hipStream_t after;      // or a wait for another stream
+    uint64_t after_op;
+  };
+  std::deque<Op> queue;
+  uint64_t done = 0;        // ops executed so far
+  uint64_t last() const { return done + queue.size(); }
+};
+
+namespace {
+
+std::map<const void*, std::string> names;
+std::vector<std::string> launched;
+std::vector<hipStream_t> streams;
+std::map<char*, size_t> allocated;
+int violations = 0, fail_wait_after = -1, wait_us = 0;
+double elapsed = 0, elapsed_step = 0;
+struct Config { dim3 grid, block; size_t shmem; hipStream_t stream; } config;
+
+void run_to(hipStream_t s, uint64_t op) {
+  while (s->done < op) {
+    const ihipStream_t::Op o = s->queue.front();
+    if (o.after) run_to(o.after, o.after_op);
+    if (o.n) memcpy(o.dst, o.src, o.n);
+    s->queue.pop_front();
+    s->done++;
+  }
+}
+
+void run_all() {
+  for (hipStream_t s : streams) run_to(s, s->last());
+}
+
+bool inside(const void* p, const char* base, size_t n) { return (const char*)p >= base && (const char*)p < base + n; }
+
+hipError_t allocate(void** p, size_t n) {
+  *p = calloc(1, n ? n : 1);
+  allocated[(char*)*p] = n;
+  return hipSuccess;
+}
+
+hipError_t release(void* p) {
+  const size_t n = allocated[(char*)p];
+  int used = 0;
+  for (hipStream_t s : streams)
+    for (const auto& o : s->queue)
+      if (o.n && (inside(o.dst, (char*)p, n) || inside(o.src, (char*)p, n))) used++;
+  if (used) run_all();
+  violations += used;
+  allocated.erase((char*)p);
+  free(p);
+  return hipSuccess;
+}
+
+}  // namespace
+
+extern "C" {
+
+// ---- for the tests
+// What the streams still hold; memory released while a copy on it waited.
+int hip_host_pending() {
+  size_t n = 0;
+  for (hipStream_t s : streams) n += s->queue.size();
+  return (int)n;
+}
+int hip_host_violations() { return violations; }
+// The n-th wait for an event from now on fails (-1: none does).
+void hip_host_fail_wait(int n) { fail_wait_after = n; }
+// Every wait for an event that is not done takes this long.
+void hip_host_wait_us(int us) { wait_us = us; }
+// Elapsed times: first, then each smaller than the one before by `step`.
+void hip_host_elapsed(double first, double step) { elapsed = first; elapsed_step = step; }
+// The kernels launched since the last call, one name a line.
+int hip_host_launches(char* out, int len) {
+  std::string all;
+  for (const std::string& k : launched) all += k + "\n";
+  launched.clear();
+  snprintf(out, len, "%s", all.c_str());
+  return (int)all.size();
+}
+
+// ---- the runtime
+hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
+hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
+hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t a, int) {
+  *v = a == hipDeviceAttributeMultiprocessorCount ? 256 : 160 * 1024;
+  return hipSuccess;
+}
+const char* hipGetErrorString(hipError_t) { return "error"; }
+hipError_t hipGetLastError() { return hipSuccess; }
+
+hipError_t hipMalloc(void** p, size_t n) { return allocate(p, n); }
+hipError_t hipFree(void* p) { return release(p); }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return allocate(p, n); }
+hipError_t hipHostFree(void* p) { return release(p); }
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { run_all(); memcpy(d, s, n); return hipSuccess; }
+hipError_t hipMemset(void* d, int v, size_t n) { run_all(); memset(d, v, n); return hipSuccess; }
+hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) { return hipMemset(d, v, n); }
+
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
+  *s = new ihipStream_t;
+  streams.push_back(*s);
+  return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t s) {
+  if (s) run_to(s, s->last());
+  else run_all();
+  return hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t s) { return hipStreamSynchronize(s); }
+hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
+  if (s && e->stream) s->queue.push_back({nullptr, nullptr, 0, e->stream, e->op});
+  return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void* d, const void* src, size_t n, hipMemcpyKind k, hipStream_t s) {
+  if (!s) return hipMemcpy(d, src, n, k);
+  s->queue.push_back({d, src, n, nullptr, 0});
+  return hipSuccess;
+}
+
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { *e = new ihipEvent_t; return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e) { return hipEventCreateWithFlags(e, 0); }
+hipError_t hipEventDestroy(hipEvent_t e) { delete e; return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+  e->stream = s;
+  e->op = s ? s->last() : 0;
+  return hipSuccess;
+}
+hipError_t hipEventSynchronize(hipEvent_t e) {
+  if (fail_wait_after >= 0 && fail_wait_after-- == 0) return hipErrorUnknown;
+  if (!e->stream || e->stream->done >= e->op) return hipSuccess;
+  if (wait_us) std::this_thread::sleep_for(std::chrono::microseconds(wait_us));
+  run_to(e->stream, e->op);
+  return hipSuccess;
+}
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) {
+  *ms = (float)elapsed;
+  elapsed *= 1 - elapsed_step;
+  return hipSuccess;
+}
+
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipErrorNotSupported; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t*) { return hipErrorNotSupported; }
+hipError_t hipGraphInstantiate(hipGraphExec_t*, hipGraph_t, hipGraphNode_t*, char*, size_t) { return hipErrorNotSupported; }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipErrorNotSupported; }
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+hipError_t hipGetSymbolAddress(void** p, const void*) { return hipMalloc(p, (size_t)4 << 20); }
+
+void** __hipRegisterFatBinary(const void*) { static void* module; return &module; }
+void __hipUnregisterFatBinary(void**) {}
+void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
+void __hipRegisterFunction(void**, const void* f, char*, const char* name, unsigned, void*, void*, dim3*, dim3*, int*) {
+  names[f] = name;
+}
+hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t shmem, hipStream_t s) {
+  config = Config{grid, block, shmem, s};
+  return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* shmem, hipStream_t* s) {
+  *grid = config.grid; *block = config.block; *shmem = config.shmem; *s = config.stream;
+  return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void* f, dim3, dim3, void**, size_t, hipStream_t) {
+  launched.push_back(names[f]);
+  return hipSuccess;
+}
+
+}  // extern "C"

@@ -1,0 +1,88 @@
+"""What the library's host code asks of the HIP runtime, on the CPU: the runtime's calls are those of hip_host.cpp,
+which keeps every stream's work waiting until something synchronises with it and runs no kernels."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+# the runtime before the library, in a process of its own, without torch
+PRELUDE = """
+import ctypes, resource, sys, time
+H = ctypes.CDLL({runtime!r}, ctypes.RTLD_GLOBAL)
+sys.path[:0] = [{root!r}, {here!r}]
+import numpy as np
+import gpu_phs_amd as G
+from gpu_phs_amd import workloads as W
+H.hip_host_elapsed.argtypes = [ctypes.c_double, ctypes.c_double]
+
+def i(v):
+    return ctypes.byref(ctypes.c_int(v))
+
+def p(a):
+    return a.ctypes.data_as(ctypes.c_void_p)
+
+def launches():
+    text = ctypes.create_string_buffer(1 << 20)
+    H.hip_host_launches(text, len(text))
+    return text.value.decode().split()
+
+def whizard(proc, counts):
+    # the host program's calls up to the first event, and the call that generates
+    L, nc, n = G.lib(), proc.n_channels, sum(counts)
+    L.c_whizard_set_particle_structure(i(nc), i(nc), i(1), i(proc.n_x), i(proc.n_in), i(proc.n_out))
+    flv = np.ascontiguousarray(proc.flv_masses)
+    L.c_whizard_set_flavors(p(flv), p(np.zeros_like(flv)))
+    L.c_whizard_init_mappings()
+    L.c_whizard_init_tree_structures()
+    for c in range(nc):
+        ids, m, w, d1, d2, hc = (np.ascontiguousarray(a[c]) for a in (proc.map_ids, proc.map_masses, proc.map_widths,
+                                                                      proc.d1, proc.d2, proc.has_children))
+        L.c_whizard_fill_mapping(i(c + 1), p(ids), p(m), p(w))
+        L.c_whizard_fill_tree_structure(i(c + 1), p(d1), p(d2), p(hc), p(np.zeros(proc.n_prt, np.int32)))
+    L.c_whizard_init_gpu_phs()
+    assert L.gpu_phs_last_error() == 0, L.gpu_phs_last_error_message()
+    L.c_whizard_init_channel_ids(i(n), i(nc), (ctypes.c_int * nc)(*np.cumsum(counts).tolist()))
+    e = np.full(n, proc.sqrts / 2)
+    x, factors, volumes, oks = np.full((n, proc.n_x), 0.5), np.zeros(n * nc), np.zeros(n), np.zeros(n, np.bool_)
+    mom, x_out, boost = np.zeros((n, proc.n_out, 4)), np.zeros(n * nc * proc.n_x), ctypes.c_bool(True)
+    def call():
+        L.c_whizard_gen_phs_from_x_gpu(p(e), p(e), ctypes.byref(boost), i(n), i(nc), i(proc.n_x), p(x), p(factors),
+                                       p(volumes), p(oks), p(mom), p(x_out))
+        return L.gpu_phs_last_error()
+    return L, call
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("hip_host") / "libhip_host.so")
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-I/opt/rocm/include",
+                           os.path.join(HERE, "hip_host.cpp"), "-o", lib])
+
+    def run(body):
+        script = PRELUDE.format(runtime=lib, root=ROOT, here=HERE) + body
+        r = subprocess.run([sys.executable, "-c", script], capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, r.stdout + r.stderr
+        return r.stdout
+    return run
+
+
+@pytest.mark.parametrize("wait", [0, 5, 9, 12, 15])
+def test_failed_host_call_leaves_no_copy_behind(run, wait):
+    """A wait that fails in the middle of a host call (300,000 events: some 30 chunks, a ring of eight slots, two
+    streams) ends the call with an error and with no transfer in flight, so that the pinned slots may be
+    released at once."""
+    run(f"""
+L, call = whizard(W.process_c1(), [100_000] * 3)
+assert call() == 0
+H.hip_host_fail_wait({wait})
+assert call() != 0
+pending = H.hip_host_pending()
+L.c_whizard_finalize_gpu_phs()
+assert H.hip_host_violations() == 0, "memory released under a copy"
+assert pending == 0, pending
+""")
