@@ -86,3 +86,24 @@ L.c_whizard_finalize_gpu_phs()
 assert H.hip_host_violations() == 0, "memory released under a copy"
 assert pending == 0, pending
 """)
+
+
+def test_copy_threads_sleep_while_the_device_works(run):
+    """The threads that copy between pinned and pageable memory wait asleep: a host call whose DMAs take 20 ms each
+    (here the waits for them) takes next to no processor time."""
+    run("""
+L, call = whizard(W.process_c1(), [30_000] * 3)
+assert call() == 0   # (starts the threads, touches the arrays)
+H.hip_host_wait_us(20_000)
+def used():
+    r = resource.getrusage(resource.RUSAGE_SELF)
+    return r.ru_utime + r.ru_stime
+best = 1e9
+for _ in range(4):   # (numpy's own threads may spin for a while after the start)
+    cpu, wall = used(), time.perf_counter()
+    assert call() == 0
+    cpu, wall = used() - cpu, time.perf_counter() - wall
+    assert wall > 0.15, wall
+    best = min(best, cpu / wall)
+assert best < 0.5, best
+""")
