@@ -132,6 +132,31 @@ void free_staging(WhizardModule& w) {
   w.kernels_ev = nullptr;
 }
 
+// The transfers of a few calls, so that the runtime sets up here, in c_whizard_init_gpu_phs, what it otherwise does
+// in the middle of the first calls: the streams' queues (3 ms each), and a copy engine (5-7 ms) whenever one
+// is first used, by the second stream or because the ones in use are busy.  A process's first call of
+// 10^5 2 -> 4 events takes 13 ms, as before the second stream (32 without this), and the ones after it 1.1 (one
+// of the first ten 7 ms without this).
+hipError_t warm_up(WhizardModule& w) {
+  char* dev = nullptr;
+  hipError_t e = hipMalloc(&dev, kPinChunk);
+  for (int call = 0; call < 3 && e == hipSuccess; call++) {
+    for (int k = 0; k < 2 && e == hipSuccess; k++)
+      e = hipMemcpyAsync(dev, w.pin + k * kPinChunk, kPinChunk, hipMemcpyHostToDevice, w.stream);
+    if (e == hipSuccess) e = hipEventRecord(w.kernels_ev, w.stream);
+    if (e == hipSuccess) e = hipStreamWaitEvent(w.stream2, w.kernels_ev, 0);
+    for (int k = 0; k < kPinSlots && e == hipSuccess; k++) {
+      hipStream_t st = k % 2 ? w.stream2 : w.stream;
+      if ((e = hipMemcpyAsync(w.pin + k * kPinChunk, dev, kPinChunk, hipMemcpyDeviceToHost, st)) == hipSuccess)
+        e = hipEventRecord(w.pin_ev[k], st);
+    }
+    const hipError_t e1 = hipStreamSynchronize(w.stream), e2 = hipStreamSynchronize(w.stream2);
+    if (e == hipSuccess) e = e1 != hipSuccess ? e1 : e2;
+  }
+  (void)hipFree(dev);
+  return e;
+}
+
 int ensure_staging(WhizardModule& w) {
   if (w.stream) return GPU_PHS_OK;
   hipError_t e = hipStreamCreateWithFlags(&w.stream, hipStreamNonBlocking);
@@ -140,8 +165,8 @@ int ensure_staging(WhizardModule& w) {
       (e = hipEventCreateWithFlags(&w.kernels_ev, hipEventDisableTiming)) == hipSuccess)
     e = hipHostMalloc((void**)&w.pin, kPinSlots * kPinChunk, hipHostMallocDefault);
   for (int k = 0; k < kPinSlots && e == hipSuccess; k++)
-    if ((e = hipEventCreateWithFlags(&w.pin_ev[k], hipEventDisableTiming)) == hipSuccess)
-      e = hipEventRecord(w.pin_ev[k], w.stream);
+    e = hipEventCreateWithFlags(&w.pin_ev[k], hipEventDisableTiming);
+  if (e == hipSuccess) e = warm_up(w);
   if (e != hipSuccess) {
     free_staging(w);
     return hip_error(e, "pinned staging buffers");
@@ -507,6 +532,7 @@ void c_whizard_init_gpu_phs(void) {
   if (!err.empty()) { set_error(GPU_PHS_E_TREE, err); return; }
   if (require_device()) return;
   w.initialized = true;
+  (void)ensure_staging(w);   // (a failure is the next generate call's, which tries again)
   ok_status();
 }
 

@@ -89,6 +89,13 @@ int hip_host_pending() {
   return (int)n;
 }
 int hip_host_violations() { return violations; }
+// Streams made so far, and those that have had a transfer.
+int hip_host_streams() { return (int)streams.size(); }
+int hip_host_used_streams() {
+  int n = 0;
+  for (hipStream_t s : streams) n += s->last() > 0 ? 1 : 0;
+  return n;
+}
 // The n-th wait for an event from now on fails (-1: none does).
 void hip_host_fail_wait(int n) { fail_wait_after = n; }
 // Every wait for an event that is not done takes this long.

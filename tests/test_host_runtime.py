@@ -107,3 +107,21 @@ for _ in range(4):   # (numpy's own threads may spin for a while after the start
     best = min(best, cpu / wall)
 assert best < 0.5, best
 """)
+
+
+def test_init_makes_the_streams_of_the_host_calls(run):
+    """The streams of the host calls are made, and have had their first transfers, when c_whizard_init_gpu_phs
+    returns, not in the first call for events; the program may end, or call again, at any time after it."""
+    run("""
+L, call = whizard(W.process_c1(), [100_000] * 3)
+made = H.hip_host_streams()
+assert made > 0 and H.hip_host_used_streams() == made
+assert H.hip_host_pending() == 0
+for _ in range(2):
+    assert call() == 0
+    assert H.hip_host_streams() == made
+L.c_whizard_reset_generator()
+assert call() == 0
+L.c_whizard_finalize_gpu_phs()
+assert H.hip_host_violations() == 0
+""")
