@@ -5,6 +5,7 @@
 // module object, so the calls keep their order-dependent semantics.
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cmath>
 #include <condition_variable>
 #include <cstdio>
@@ -236,15 +237,21 @@ CopyPool& copy_pool() {
   return pool;
 }
 
-// A condition that other threads bring about and announce with changed(): waited for asleep, so that the copy
-// threads take no time from the host program while the kernels run and the DMAs are on their way.  A call of
-// 10^6 2 -> 4 events uses 41 ms of processor time, of 10^5 3.7; with threads that wait actively 67 and 7.7, and
-// no less of the clock (9.1 and 1.06 ms either way; 20 or 60 us of active waiting first change nothing).
+// A condition that other threads bring about and announce with changed(): waited for asleep after the time between
+// two chunks, so that the copy threads take no time from the host program while the kernels run.  A call of
+// 10^6 2 -> 4 events uses 50 ms of processor time, of 10^5 4.4 (41 and 3.7 without the active wait, which the
+// 10^5 repay with 2% of their 1.06 ms; 67 and 7.7 with threads that only wait actively).
 class Waiting {
  public:
   template <class Done>
   void until(Done done) {
-    if (done()) return;
+    const auto end = std::chrono::steady_clock::now() + std::chrono::microseconds(20);
+    do {
+      for (int k = 0; k < 32; k++) {
+        if (done()) return;
+        __builtin_ia32_pause();
+      }
+    } while (std::chrono::steady_clock::now() < end);
     std::unique_lock<std::mutex> lk(m_);
     cv_.wait(lk, done);
   }
@@ -370,6 +377,8 @@ int transfer(WhizardModule& w, const std::vector<Transfer>& list, bool to_device
   if (e != hipSuccess) {
     abort.store(true);
     for_open.changed();
+  } else if (threads > 0) {
+    pieces();   // of the last chunk, while the threads wake up
   }
   if (threads > 0) copy_pool().wait();
   return e == hipSuccess ? GPU_PHS_OK : failed(e, to_device ? "host to device copy" : "device to host copy");
