@@ -191,9 +191,12 @@ __global__ __launch_bounds__(kGenThreads) void grid_generate_kernel(const TileDe
 // fields go to the workgroup's LDS histogram before they can overflow, and that to the global
 // counts once per workgroup and channel: device atomics on the few hundred shared counters
 // serialise (1.27 million of them, one set per 256-event tile, made the kernel 251 us for 4e6
-// events of 8 randoms in 3 channels).  Four workgroups per CU fill it with loads in flight:
-// 49 us at 1024 workgroups (5.3 TB/s of the randoms), 55 at 512, 87 at 256, 62 at 2048, where the
-// atomics show again; fewer for few events (launch_grid_histogram).
+// events of 8 randoms in 3 channels).  Four workgroups per CU fill it with loads in flight: eight
+// randoms and flags per thread, which the whole batches load without a test (guarded, each load waits in a
+// branch of its own: 63 us for the same events after a forward pass, 66 with the one element per thread tested
+// for in the loop, 46 as it is, 5.6 TB/s of the randoms).  The workgroups were chosen on the first version: 49
+// us at 1024, 55 at 512, 87 at 256, 62 at 2048, where the atomics show again; fewer for few events
+// (launch_grid_histogram).
 constexpr int kHistThreads = 512;
 constexpr int kHistGroups = 1024;
 constexpr int kHistUnroll = 8;                                     // loads in flight per thread
@@ -242,35 +245,55 @@ __global__ __launch_bounds__(kHistThreads) void grid_histogram_kernel(const Tile
         }
         fields = 0;
       };
+      // element u of a batch from its first one: its bin and whether it counts
+      auto count = [&](double xe, unsigned int accept) {
+        int b = (int)(xe * kGridBins);   // rng.cpp:52
+        b = b < 0 ? 0 : b > kGridBins - 1 ? kGridBins - 1 : b;
+        const unsigned int one = accept ? 1u : 0u;
+        fields += (unsigned long long)one << (kHistField * b);
+        accepted += one;
+      };
       int passes = 0;
-      for (int64_t e = td.e0 + r; e < e_end; e += (int64_t)per * kHistUnroll) {
-        if (e_end - (e - r) <= per) {   // one element per thread: counted at once
-          const double xe = xk[e * n_x];
-          if (ok[e]) {
-            const int b = (int)(xe * kGridBins);
-            atomicAdd(&hist[k * kGridBins + (b < 0 ? 0 : b > kGridBins - 1 ? kGridBins - 1 : b)], 1u);
-            accepted++;
-          }
-          break;
-        }
+      const int step = per * n_x;   // from one element of the thread to the next
+      int64_t e = td.e0;            // first event of the pass
+      const gdouble* px = xk + (e + r) * n_x;
+      const guint8* po = ok + (e + r);
+      // whole batches: every load is inside, without a test
+      for (; e + per * kHistUnroll <= e_end; e += per * kHistUnroll) {
         double xv[kHistUnroll];
         unsigned int in[kHistUnroll];
 #pragma unroll
         for (int u = 0; u < kHistUnroll; u++) {
-          const int64_t eu = e + (int64_t)u * per;
-          const bool inside = eu < e_end;
-          in[u] = inside ? ok[eu] : 0;
-          xv[u] = inside ? xk[eu * n_x] : 0.0;
+          in[u] = po[u * per];
+          xv[u] = px[u * step];
         }
+        px += kHistUnroll * step;
+        po += kHistUnroll * per;
+#pragma unroll
+        for (int u = 0; u < kHistUnroll; u++) count(xv[u], in[u]);
+        if (++passes == kHistPasses) { flush(); passes = 0; }
+      }
+      const int left = (int)(e_end - e);   // events after them
+      if (left > per) {
+        // elements past the end read the thread's first one, which is inside, and do not count
+        double xv[kHistUnroll];
+        unsigned int in[kHistUnroll];
 #pragma unroll
         for (int u = 0; u < kHistUnroll; u++) {
-          int b = (int)(xv[u] * kGridBins);   // rng.cpp:52
-          b = b < 0 ? 0 : b > kGridBins - 1 ? kGridBins - 1 : b;
-          const unsigned int one = in[u] ? 1u : 0u;
-          fields += (unsigned long long)one << (kHistField * b);
-          accepted += one;
+          const bool inside = u * per + r < left;
+          in[u] = po[inside ? u * per : 0];
+          xv[u] = px[inside ? u * step : 0];
+          if (!inside) in[u] = 0;
         }
-        if (++passes == kHistPasses) { flush(); passes = 0; }
+#pragma unroll
+        for (int u = 0; u < kHistUnroll; u++) count(xv[u], in[u]);
+      } else if (r < left) {   // one element per thread: counted at once
+        const double xe = *px;
+        if (*po) {
+          const int b = (int)(xe * kGridBins);
+          atomicAdd(&hist[k * kGridBins + (b < 0 ? 0 : b > kGridBins - 1 ? kGridBins - 1 : b)], 1u);
+          accepted++;
+        }
       }
       if (fields) flush();
       if (k == 0 && accepted) atomicAdd(&hist[nb], accepted);

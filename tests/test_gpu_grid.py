@@ -128,3 +128,42 @@ def test_generate_edges_match_oracle(n_out, counts, cfg):
     for s, (b, c) in enumerate(zip(bufs, chans)):
         got = b.x.cpu().numpy()
         assert np.array_equal(got, oracle.grid_sample(F[c], oracle.grid_uniforms(seed, s, got.shape[0], proc.n_x)))
+
+
+@pytest.mark.parametrize("n_out,counts,cfg,bin_", [
+    # 140 tiles, a workgroup each: 64 elements a thread, all in one bin, one more than its private count holds
+    (4, [140 * 4096], dict(block=256, ept=16), 3),
+    (4, [140 * 4096], dict(block=256, ept=16), 9),
+    # 1025 tiles on 1024 workgroups: one of two tiles
+    (4, [1024 * 512 + 1], dict(block=256, ept=2), None),
+    # 11 randoms: 6 of 512 threads without an element; 400 tiles of 42 segments on 128 workgroups, whose ranges
+    # hold the ends of several segments and channels
+    (5, [65 + 613 * k % 997 for k in range(42)], dict(block=64, ept=1), None),
+    # one to ten tiles of 1024 events and a last one that is a pass of 64 events, or a batch of 8, or next to it
+    (4, [1024 * (12 - k) + n for k, n in enumerate([64, 65, 63, 511, 512, 513, 575, 576, 577, 1, 128])] + [12 * 1024] * 4,
+     dict(block=256, ept=4), None),
+])
+def test_update_counts_on_many_tiles(n_out, counts, cfg, bin_):
+    """The histogram of more than 128 tiles where its loops begin and end: threads that hand over their counts in
+    the middle of a range, threads without an element, ranges across segments, whole batches and what is left."""
+    import torch
+    import gpu_phs_amd as G
+    proc = W.process_shapes(n_out, 3)
+    counts = (counts + [0] * proc.n_channels)[:proc.n_channels]
+    ph, plan, bufs, chans = _plan(proc, counts, **cfg)
+    assert plan.info()["n_tiles"] > 128
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    for b in bufs:
+        if bin_ is None:
+            b.x.copy_(torch.rand(b.x.shape, generator=gen, device="cuda", dtype=torch.float64) ** 2)
+            b.ok.copy_(torch.rand(b.ok.shape, generator=gen, device="cuda") < 0.7)
+        else:
+            b.x.fill_((bin_ + 0.5) / 10)
+            b.ok.fill_(1)
+    grid = G.Grid(ph)
+    w = grid.weights()
+    grid.update(plan)
+    x = np.concatenate([b.x.cpu().numpy() for b in bufs])
+    ok = np.concatenate([b.ok.cpu().numpy().astype(bool) for b in bufs])
+    ch = np.repeat(chans, [b.x.shape[0] for b in bufs])
+    assert np.array_equal(grid.weights(), oracle.grid_update(w, x, ok, ch))
