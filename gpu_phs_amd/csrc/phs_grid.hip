@@ -357,6 +357,7 @@ __global__ void fill_u64_kernel(unsigned long long* p, size_t n) {
 hipError_t launch_grid_generate(const DevicePlan& dp, const double* cdf, int n_dim, uint64_t seed, hipStream_t stream) {
   if (dp.n_tiles <= 0) return hipSuccess;
   const size_t shmem = (size_t)n_dim * (kGridBins * sizeof(BinRec) + kGenWaves * kGenRow * sizeof(double) + kGenCells);
+  if (shmem > forward_lds_limit()) return hipErrorInvalidValue;   // 84 KB for the 32 randoms of twelve particles
   const int groups = std::min(dp.n_tiles, kGenGroups);
   hipLaunchKernelGGL(grid_generate_kernel, dim3(groups), dim3(kGenThreads), shmem, stream, dp.tiles,
                      dp.n_tiles / groups, dp.n_tiles % groups, dp.segs, dp.chans, cdf, n_dim, seed);

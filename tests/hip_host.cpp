@@ -38,7 +38,7 @@ std::map<const void*, std::string> names;
 std::vector<std::string> launched;
 std::vector<hipStream_t> streams;
 std::map<char*, size_t> allocated;
-int violations = 0, fail_wait_after = -1, wait_us = 0;
+int violations = 0, fail_wait_after = -1, wait_us = 0, lds = 160 * 1024;
 double elapsed = 0, elapsed_step = 0;
 struct Config { dim3 grid, block; size_t shmem; hipStream_t stream; } config;
 
@@ -100,6 +100,8 @@ int hip_host_used_streams() {
 void hip_host_fail_wait(int n) { fail_wait_after = n; }
 // Every wait for an event that is not done takes this long.
 void hip_host_wait_us(int us) { wait_us = us; }
+// The LDS of a workgroup from now on.
+void hip_host_lds(int bytes) { lds = bytes; }
 // Elapsed times: first, then each smaller than the one before by `step`.
 void hip_host_elapsed(double first, double step) { elapsed = first; elapsed_step = step; }
 // The kernels launched since the last call, one name a line.
@@ -115,7 +117,7 @@ int hip_host_launches(char* out, int len) {
 hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
 hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
 hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t a, int) {
-  *v = a == hipDeviceAttributeMultiprocessorCount ? 256 : 160 * 1024;
+  *v = a == hipDeviceAttributeMultiprocessorCount ? 256 : lds;
   return hipSuccess;
 }
 const char* hipGetErrorString(hipError_t) { return "error"; }

@@ -167,3 +167,29 @@ def test_update_counts_on_many_tiles(n_out, counts, cfg, bin_):
     ok = np.concatenate([b.ok.cpu().numpy().astype(bool) for b in bufs])
     ch = np.repeat(chans, [b.x.shape[0] for b in bufs])
     assert np.array_equal(grid.weights(), oracle.grid_update(w, x, ok, ch))
+
+
+@pytest.mark.parametrize("n_out", [7, 8, 12])
+def test_grids_of_large_trees(n_out):
+    """Trees above six particles: the draw's tables in LDS grow with the randoms (2,640 bytes each, 84 KB for
+    twelve particles), as does the histogram's."""
+    import torch
+    import gpu_phs_amd as G
+    proc = W.process_large(n_out)
+    counts = [700, 33_000][:proc.n_channels]
+    ph, plan, bufs, chans = _plan(proc, counts)
+    grid = G.Grid(ph)
+    w = np.random.default_rng(n_out).random(grid.shape) + 0.01
+    grid.set_weights(w)
+    grid.generate(plan, 77)
+    torch.cuda.synchronize()
+    F = oracle.grid_cdf(w)
+    for s, (b, c) in enumerate(zip(bufs, chans)):
+        got = b.x.cpu().numpy()
+        assert np.array_equal(got, oracle.grid_sample(F[c], oracle.grid_uniforms(77, s, got.shape[0], proc.n_x)))
+    plan.run()
+    grid.update(plan)
+    x = np.concatenate([b.x.cpu().numpy() for b in bufs])
+    ok = np.concatenate([b.ok.cpu().numpy().astype(bool) for b in bufs])
+    ch = np.repeat(chans, [b.x.shape[0] for b in bufs])
+    assert np.array_equal(grid.weights(), oracle.grid_update(w, x, ok, ch))

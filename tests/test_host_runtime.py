@@ -30,6 +30,27 @@ def launches():
     H.hip_host_launches(text, len(text))
     return text.value.decode().split()
 
+class Array:
+    # a segment's array: host memory, as the runtime's device memory is
+    def __init__(self, shape, dtype=np.float64):
+        self.a = np.zeros(shape, dtype)
+        self.shape, self.dtype = self.a.shape, self.a.dtype
+    def is_contiguous(self):
+        return True
+    def data_ptr(self):
+        return self.a.ctypes.data
+
+class Stream:
+    cuda_stream = 0
+
+def plan(proc, counts, **config):
+    ph, segs = G.ProcessHandle(proc), []
+    for c, n in enumerate(counts):
+        if n:
+            segs.append((ph, c, G.EventBuffers(Array((n, proc.n_x)), Array((n, proc.n_out, 4)), Array(n), Array(n),
+                                               Array(n, np.uint8))))
+    return G.Plan(segs, **config)
+
 def whizard(proc, counts):
     # the host program's calls up to the first event, and the call that generates
     L, nc, n = G.lib(), proc.n_channels, sum(counts)
@@ -124,4 +145,22 @@ L.c_whizard_reset_generator()
 assert call() == 0
 L.c_whizard_finalize_gpu_phs()
 assert H.hip_host_violations() == 0
+""")
+
+
+def test_grid_draw_asks_for_its_lds(run):
+    """The draw's tables (2,640 bytes of LDS per random) are checked against the device's limit before the launch."""
+    run("""
+H.hip_host_lds(65536)
+for n_out, fits in ((8, True), (12, False)):
+    pl = plan(W.process_large(n_out), [100, 100])
+    grid = G.Grid(pl._keep[0][0])
+    launches()
+    try:
+        grid.generate(pl, 1, Stream)
+        ok = True
+    except G.GpuPhsError:
+        ok = False
+    assert ok == fits
+    assert any("grid_generate" in k for k in launches()) == fits
 """)
