@@ -826,20 +826,23 @@ int gpu_phs_plan_autotune(int plan, void* stream_v, int reps, char* report, int 
       return GPU_PHS_OK;
     };
     const bool banks = pl->dps[cls].n_banks > 0;
-    // the shape-specialised kernels keep randoms and banks in registers: where only they run,
-    // the placement flags change nothing; those of up to four particles also have a budget for
-    // 5 waves per SIMD, the larger ones only the compiler's
+    // the shape-specialised kernels keep randoms and banks in registers: where only they run, the placement
+    // flags change nothing, and of the register budgets only that for 5 waves per SIMD selects other kernels,
+    // those of one shape of up to four particles with fixed beams (the kernels of a group of shapes have
+    // their own, whatever is asked for: timed, the budgets would be told apart by noise)
+    LaunchConfig unit = pl->lcs[cls];
+    unit.grid = 0;
     bool placement = false, small = false;
-    for (const ShapeRun& r : launch_runs(*pl, cls, pl->lcs[cls])) {
+    for (const ShapeRun& r : launch_runs(*pl, cls, unit)) {
       placement = placement || r.sid == -1;
-      small = small || r.sid == kRunOfGroup || (r.sid >= 0 && kShapes[r.sid].n_out <= 4);
+      small = small || (r.sid >= 0 && kShapes[r.sid].n_out <= 4 && !pl->dps[cls].per_event_beams);
     }
-    const int wpe_max = placement ? 4 : (small ? 5 : 0);
+    auto budget = [&](int wpe) { return wpe == 0 || (wpe == 5 ? small && !placement : placement); };
     // stage 1: register budget (occupancy target), where deferred boosts wait (lds bit 0) and
     // where the randoms are kept (lds bit 1)
     for (int wpe : {0, 3, 4, 5})
       for (int lds : {0, 1, 2, 3})
-        if (!rc && wpe <= wpe_max && (!(lds & 1) || banks) && (placement || lds == 0)) {
+        if (!rc && budget(wpe) && (!(lds & 1) || banks) && (placement || lds == 0)) {
           LaunchConfig lc = best.lc;
           lc.waves_per_eu = wpe; lc.lds = lds; lc.grid = 0;
           rc = consider(lc);
@@ -861,7 +864,7 @@ int gpu_phs_plan_autotune(int plan, void* stream_v, int reps, char* report, int 
       const LaunchConfig shape = best.lc;
       for (int wpe : {0, 3, 4, 5})
         for (int lds : {0, 1, 2, 3})
-          if (!rc && wpe <= wpe_max && (!(lds & 1) || banks) && (placement || lds == 0) &&
+          if (!rc && budget(wpe) && (!(lds & 1) || banks) && (placement || lds == 0) &&
               !(wpe == shape.waves_per_eu && lds == shape.lds)) {
             LaunchConfig lc = shape;
             lc.waves_per_eu = wpe; lc.lds = lds;

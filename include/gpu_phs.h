@@ -152,7 +152,9 @@ int gpu_phs_plan_destroy(int plan);
  * use LDS), 2 keeps each event's randoms in LDS instead of VGPRs (always for n_x > 16).  With grid 0
  * every kernel runs one workgroup per sub-tile (block events) and the shape-specialised kernels at
  * their own register budget (four waves per SIMD for trees of up to four final-state particles,
- * three for five and six); ept is then only the sub-tiles of a tile.  Changing block, ept or order
+ * three for five and six); ept is then only the sub-tiles of a tile.  The kernels of one shape asked
+ * for 5 waves per SIMD (up to four particles), or for a workgroup size they are not built for (192
+ * threads; for five and six particles all but 64), loop over a tile's sub-tiles instead.  Changing block, ept or order
  * rebuilds the tile table.  A block whose LDS tables (4 n_out rows of block + 1 doubles, n_x
  * more with randoms in LDS, plus the LDS save banks) exceed the device's per-workgroup LDS is
  * rejected. */

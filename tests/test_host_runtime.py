@@ -164,3 +164,29 @@ for n_out, fits in ((8, True), (12, False)):
     assert ok == fits
     assert any("grid_generate" in k for k in launches()) == fits
 """)
+
+
+@pytest.mark.parametrize("process,counts,beams,budgets", [
+    ("W.process_c1()", [5000] * 3, False, {0}),                # three shapes of a group in one launch
+    ("W.process_shapes(5)", [300] * 42, False, {0}),
+    ("W.process_c1()", [5000, 0, 0], False, {0, 5}),           # one shape of four particles: its own kernels
+    ("W.process_c1()", [5000, 0, 0], True, {0}),               # with per-event beams it has one budget
+    ("W.process_friends(4)", [5000] * 4, False, {0, 3, 4}),    # the generic kernel
+])
+def test_autotuner_tries_the_budgets_that_select_a_kernel(run, process, counts, beams, budgets):
+    """Launches that ignore waves_per_eu are not timed under several values of it: each is as fast as the others, and
+    the one left in place (here every later candidate looks faster) would mean something to other launches."""
+    run(f"""
+proc = {process}
+pl = plan(proc, ({counts} + [0] * proc.n_channels)[:proc.n_channels])
+if {beams}:
+    for k, (_, buf) in enumerate(pl._keep):
+        e = Array(buf.x.shape[0])
+        e.a[:] = proc.sqrts / 2
+        pl.set_event_beams(k, e, e)
+H.hip_host_elapsed(30.0, 0.001)
+report = pl.autotune(stream=Stream, reps=1)
+tried = [k.split(":")[1].split("/") for k in report.split(";")[-1].split()]
+assert len(tried) > 5
+assert {{int(t[3]) for t in tried if int(t[2]) == 0}} == {budgets}, report
+""")
