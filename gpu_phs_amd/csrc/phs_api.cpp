@@ -4,7 +4,7 @@
 #include <cstdio>
 #include <cstring>
 #include <functional>
-#include <numeric>
+#include <tuple>
 
 #include "phs_shapes.h"
 #include "phs_state.h"
@@ -148,77 +148,78 @@ int plan_build(PlanObj& pl) {
     }
     pl.chan_class[c] = small ? 0 : 1;
   }
-  // tiles of each segment (segment order, for the plain launches), then the table in class
-  // order, and within a class in segment order or deepest programs first
-  std::vector<TileDesc> tiles;
-  std::vector<int> tile_depth, tile_class;
-  pl.seg_tile_begin.assign(pl.segs.size(), 0);
-  pl.seg_tile_end.assign(pl.segs.size(), 0);
-  for (size_t s = 0; s < pl.segs.size(); s++) {
-    const int cl = pl.chan_class[pl.segs[s].channel];
-    const int64_t tile = (int64_t)pl.lcs[cl].block * pl.lcs[cl].ept;
-    for (int64_t e0 = 0; e0 < pl.segs[s].n_events; e0 += tile) {
-      TileDesc td{};
-      td.seg = (int32_t)s;
-      td.e0 = e0;
-      td.count = (int32_t)std::min<int64_t>(tile, pl.segs[s].n_events - e0);
-      tiles.push_back(td);
-      tile_depth.push_back(pl.chans[pl.segs[s].channel].n_nodes);
-      tile_class.push_back(cl);
-    }
-  }
-  if (tiles.size() > (size_t)0x7fffffff) return set_error(GPU_PHS_E_ARG, "too many tiles");
-  std::vector<int> idx(tiles.size());
-  std::iota(idx.begin(), idx.end(), 0);
-  // each class by group of shapes, in a group by tree shape, the shapes with fewer than merge_below
-  // events in the class after the others; shapeless channels last
+  // per-event beam energies, and events per shape
+  bool pev[kTileClasses] = {};
+  for (const SegDesc& sd : pl.segs) pev[pl.chan_class[sd.channel]] |= sd.e1 != nullptr;
   std::vector<int64_t> shape_events((size_t)kTileClasses * kNumShapes, 0);
-  for (size_t t = 0; t < tiles.size(); t++) {
-    const int sh = pl.chans[pl.segs[tiles[t].seg].channel].shape;
-    if (sh >= 0) shape_events[(size_t)tile_class[t] * kNumShapes + sh] += tiles[t].count;
-  }
-  auto shape_key = [&](int t) {
-    const int sh = pl.chans[pl.segs[tiles[t].seg].channel].shape;
-    if (sh < 0) return 8 * kNumShapes;
-    const bool small = shape_events[(size_t)tile_class[t] * kNumShapes + sh] < pl.merge_below;
-    return (2 * shape_group(kShapes[sh].n_out) + (small ? 1 : 0)) * kNumShapes + sh;
+  for (const SegDesc& sd : pl.segs)
+    if (sd.shape >= 0) shape_events[(size_t)pl.chan_class[sd.channel] * kNumShapes + sd.shape] += sd.n_events;
+  auto is_small = [&](int cl, int sh) { return shape_events[(size_t)cl * kNumShapes + sh] < pl.merge_below; };
+  // The tile table: segment by segment, each class by group of shapes, in a group by tree shape, the shapes with
+  // fewer than merge_below events in the class after the others; shapeless channels last.
+  struct Order {
+    int cls, shape, depth, seg;
   };
-  std::stable_sort(idx.begin(), idx.end(), [&](int a, int b) {
-    if (tile_class[a] != tile_class[b]) return tile_class[a] < tile_class[b];
-    if (shape_key(a) != shape_key(b)) return shape_key(a) < shape_key(b);
+  std::vector<Order> order(pl.segs.size());
+  int64_t n_tiles = 0;
+  auto tile_events = [&](int cl) { return (int64_t)pl.lcs[cl].block * pl.lcs[cl].ept; };
+  for (size_t s = 0; s < pl.segs.size(); s++) {
+    const SegDesc& sd = pl.segs[s];
+    const int cl = pl.chan_class[sd.channel], sh = sd.shape;
+    const bool small = sh >= 0 && is_small(cl, sh);
+    const int key = sh < 0 ? 8 * kNumShapes : (2 * shape_group(kShapes[sh].n_out) + (small ? 1 : 0)) * kNumShapes + sh;
     // order 1: heaviest programs first, so the tail of the launch is made of short tiles
-    return pl.order == 1 && tile_depth[a] > tile_depth[b];
+    order[s] = Order{cl, key, pl.order == 1 ? -pl.chans[sd.channel].n_nodes : 0, (int)s};
+    n_tiles += (sd.n_events + tile_events(cl) - 1) / tile_events(cl);
+  }
+  if (n_tiles > 0x7fffffff) return set_error(GPU_PHS_E_ARG, "too many tiles");
+  std::sort(order.begin(), order.end(), [](const Order& a, const Order& b) {
+    return std::tie(a.cls, a.shape, a.depth, a.seg) < std::tie(b.cls, b.shape, b.depth, b.seg);
   });
-  pl.tiles.resize(tiles.size());
+  pl.tiles.reserve(n_tiles);
   pl.tile_max = 0;
   pl.n_units = 0;
-  for (const TileDesc& td : tiles) {
-    pl.tile_max = std::max(pl.tile_max, (int)td.count);
-    pl.n_units += (td.count + 63) / 64;
+  pl.seg_tile_begin.assign(pl.segs.size(), 0);
+  pl.seg_tile_end.assign(pl.segs.size(), 0);
+  for (int c = 0; c < kTileClasses; c++) {
+    pl.class_begin[c] = pl.class_end[c] = 0;
+    pl.shape_runs[c].clear();
+    pl.group_runs[c].clear();
   }
-  for (int c = 0; c < kTileClasses; c++) pl.class_begin[c] = pl.class_end[c] = 0;
-  for (size_t i = 0; i < idx.size(); i++) {
-    const TileDesc& td = tiles[idx[i]];
-    pl.tiles[i] = td;
-    const int cl = tile_class[idx[i]];
-    if (pl.class_end[cl] == 0) pl.class_begin[cl] = (int)i;
-    pl.class_end[cl] = (int)i + 1;
+  auto extend = [](std::vector<ShapeRun>& runs, int sid, int begin, int end, double bytes) {
+    if (runs.empty() || runs.back().sid != sid) runs.push_back(ShapeRun{sid, begin, begin, 0});
+    runs.back().end = end;
+    runs.back().bytes += bytes;
+  };
+  for (const Order& o : order) {
+    const SegDesc& sd = pl.segs[o.seg];
+    const ChannelDesc& cd = pl.chans[sd.channel];
+    if (sd.n_events == 0) continue;
+    const int c = o.cls, begin = (int)pl.tiles.size();
+    const int64_t tile = tile_events(c);
+    for (int64_t e0 = 0; e0 < sd.n_events; e0 += tile)
+      pl.tiles.push_back(TileDesc{o.seg, (int32_t)std::min<int64_t>(tile, sd.n_events - e0), e0});
+    const int end = (int)pl.tiles.size();
+    pl.seg_tile_begin[o.seg] = begin;
+    pl.seg_tile_end[o.seg] = end;
+    if (pl.class_end[c] == 0) pl.class_begin[c] = begin;
+    pl.class_end[c] = end;
+    pl.tile_max = std::max(pl.tile_max, (int)std::min<int64_t>(tile, sd.n_events));
+    pl.n_units += (sd.n_events + 63) / 64;   // (tiles are whole units but for a segment's last)
+    // the class by shape and by shape group (with per-event beams, only the trees of up to four final-state
+    // particles have specialised kernels; the others run the generic one)
+    const double bytes = (double)sd.n_events * (8.0 * cd.n_x + 32.0 * cd.n_out + 17.0);
+    const int sh = !pl.specialize || (pev[c] && sd.shape >= kPevShapes) ? -1 : sd.shape;
+    extend(pl.shape_runs[c], sh >= 0 && is_small(c, sh) ? -1 : sh, begin, end, bytes);
+    extend(pl.group_runs[c], sh < 0 ? -1 : kRunOfGroup - shape_group(kShapes[sh].n_out), begin, end, bytes);
   }
-  // plain launches: the table positions of each segment's tiles (contiguous per segment,
-  // except under order 1, where a segment keeps its own range only if its tiles stay adjacent)
-  {
-    std::vector<int> pos(tiles.size());
-    for (size_t i = 0; i < idx.size(); i++) pos[idx[i]] = (int)i;
-    size_t t = 0;
-    for (size_t s = 0; s < pl.segs.size(); s++) {
-      int lo = 0x7fffffff, hi = 0;
-      const size_t t0 = t;
-      while (t < tiles.size() && tiles[t].seg == (int32_t)s) { lo = std::min(lo, pos[t]); hi = std::max(hi, pos[t] + 1); t++; }
-      if (t == t0) lo = hi = 0;
-      pl.seg_tile_begin[s] = lo;
-      pl.seg_tile_end[s] = hi;
+  // a group run of one shape: that shape's kernel
+  for (int c = 0; c < kTileClasses; c++)
+    for (ShapeRun& r : pl.group_runs[c]) {
+      if (r.sid > kRunOfGroup) continue;
+      const int first = pl.segs[pl.tiles[r.begin].seg].shape, last = pl.segs[pl.tiles[r.end - 1].seg].shape;
+      if (first == last) r.sid = first;   // (a shape is either small or not: its tiles are together)
     }
-  }
 
   // upload: one allocation, 256-byte aligned sections
   auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
@@ -270,35 +271,8 @@ int plan_build(PlanObj& pl) {
     pl.dps[c] = pl.dp;
     maxima(pl.dps[c], c);
   }
-  for (const SegDesc& sd : pl.segs)
-    if (sd.e1) pl.dp.per_event_beams = pl.dps[pl.chan_class[sd.channel]].per_event_beams = 1;
-  // each class by shape and by shape group (with per-event beams, only the trees of up to four
-  // final-state particles have specialised kernels; the others run the generic one)
-  for (int c = 0; c < kTileClasses; c++) {
-    pl.shape_runs[c].clear();
-    pl.group_runs[c].clear();
-    const bool pev = pl.dps[c].per_event_beams != 0;
-    auto extend = [](std::vector<ShapeRun>& runs, int sid, int t, double bytes) {
-      if (runs.empty() || runs.back().sid != sid) runs.push_back(ShapeRun{sid, t, t, 0});
-      runs.back().end = t + 1;
-      runs.back().bytes += bytes;
-    };
-    for (int t = pl.class_begin[c]; t < pl.class_end[c]; t++) {
-      const ChannelDesc& cd = pl.chans[pl.segs[pl.tiles[t].seg].channel];
-      const double bytes = (double)pl.tiles[t].count * (8.0 * cd.n_x + 32.0 * cd.n_out + 17.0);
-      const int sh = !pl.specialize || (pev && cd.shape >= kPevShapes) ? -1 : cd.shape;
-      const bool small = sh >= 0 && shape_events[(size_t)c * kNumShapes + sh] < pl.merge_below;
-      extend(pl.shape_runs[c], small ? -1 : sh, t, bytes);
-      extend(pl.group_runs[c], sh < 0 ? -1 : kRunOfGroup - shape_group(kShapes[sh].n_out), t, bytes);
-    }
-    // a group run of one shape: that shape's kernel
-    for (ShapeRun& r : pl.group_runs[c]) {
-      if (r.sid > kRunOfGroup) continue;
-      const int first = pl.chans[pl.segs[pl.tiles[r.begin].seg].channel].shape;
-      const int last = pl.chans[pl.segs[pl.tiles[r.end - 1].seg].channel].shape;
-      if (first == last) r.sid = first;   // (a shape is either small or not: its tiles are together)
-    }
-  }
+  for (int c = 0; c < kTileClasses; c++)
+    if (pev[c]) pl.dp.per_event_beams = pl.dps[c].per_event_beams = 1;
   return ok_status();
 }
 

@@ -190,3 +190,34 @@ tried = [k.split(":")[1].split("/") for k in report.split(";")[-1].split()]
 assert len(tried) > 5
 assert {{int(t[3]) for t in tried if int(t[2]) == 0}} == {budgets}, report
 """)
+
+
+def test_plan_building_sorts_segments_not_tiles(run):
+    """The tile table of 20 million events (78,000 tiles, 150 segments of four processes) is built in less time than
+    numpy takes to sort as many random numbers stably."""
+    run("""
+class Events(Array):   # a segment's array that only an address is wanted of
+    def __init__(self, *shape):
+        self.shape, self.dtype = shape, np.float64
+    def data_ptr(self):
+        return 1 << 20
+
+segs = []
+for proc in (W.process_c0(), W.process_c1(), W.process_c2(), W.process_2to6()):
+    ph = G.ProcessHandle(proc)
+    for c in range(proc.n_channels):
+        n = 2 * 5_000_000 * (c + 1) // (proc.n_channels * (proc.n_channels + 1))
+        segs.append((ph, c, G.EventBuffers(Events(n, proc.n_x), Events(n, proc.n_out, 4), Events(n), Events(n), Events(n))))
+def fastest(f):
+    t = []
+    for _ in range(9):
+        start = time.perf_counter()
+        f()
+        t.append(time.perf_counter() - start)
+    return min(t)
+tiles = G.Plan(segs).info()["n_tiles"]
+numbers = np.random.default_rng(1).random(tiles)
+build, sort = fastest(lambda: G.Plan(segs).close()), fastest(lambda: np.argsort(numbers, kind="stable"))
+assert tiles > 70_000
+assert build < sort, (build, sort)
+""")
