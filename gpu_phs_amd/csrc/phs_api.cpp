@@ -84,6 +84,12 @@ static void drop_graph(PlanObj& pl) {
   if (pl.graph) { (void)hipGraphDestroy(pl.graph); pl.graph = nullptr; }
 }
 
+// Whether a class's tile table is another under b than under a: the tiles, or (a persistent grid has no launches by
+// group of shapes) their order.
+static bool other_tiles(const LaunchConfig& a, const LaunchConfig& b) {
+  return a.block != b.block || a.ept != b.ept || (a.grid == 0) != (b.grid == 0);
+}
+
 // Tables of a plan: channels of every process the segments use (deduplicated), their
 // programs, segment descriptors, and the tile table (tiles never cross a segment, so every
 // workgroup runs a single channel).
@@ -148,15 +154,27 @@ int plan_build(PlanObj& pl) {
     }
     pl.chan_class[c] = small ? 0 : 1;
   }
-  // per-event beam energies, and events per shape
-  bool pev[kTileClasses] = {};
+  // per-event beam energies, events per shape, and whether the launches of a class are by group of shapes
+  // (launch_runs): not where a group of several shapes has no kernel
+  bool pev[kTileClasses] = {}, grouped[kTileClasses];
   for (const SegDesc& sd : pl.segs) pev[pl.chan_class[sd.channel]] |= sd.e1 != nullptr;
   std::vector<int64_t> shape_events((size_t)kTileClasses * kNumShapes, 0);
   for (const SegDesc& sd : pl.segs)
     if (sd.shape >= 0) shape_events[(size_t)pl.chan_class[sd.channel] * kNumShapes + sd.shape] += sd.n_events;
+  for (int c = 0; c < kTileClasses; c++) {
+    grouped[c] = true;
+    int shapes[3] = {0, 0, 0};   // of each group
+    DevicePlan beams;
+    beams.per_event_beams = pev[c] ? 1 : 0;
+    for (int sh = 0; sh < (pev[c] ? kPevShapes : kNumShapes); sh++)
+      if (shape_events[(size_t)c * kNumShapes + sh] > 0 && ++shapes[shape_group(kShapes[sh].n_out)] > 1 &&
+          !has_shapes_kernel(beams, shape_group(kShapes[sh].n_out), pl.lcs[c]))
+        grouped[c] = false;
+  }
   auto is_small = [&](int cl, int sh) { return shape_events[(size_t)cl * kNumShapes + sh] < pl.merge_below; };
   // The tile table: segment by segment, each class by group of shapes, in a group by tree shape, the shapes with
-  // fewer than merge_below events in the class after the others; shapeless channels last.
+  // fewer than merge_below events in the class after the others; shapeless channels last.  A class without
+  // launches by group has its small shapes together with the shapeless channels, one generic launch.
   struct Order {
     int cls, shape, depth, seg;
   };
@@ -167,7 +185,9 @@ int plan_build(PlanObj& pl) {
     const SegDesc& sd = pl.segs[s];
     const int cl = pl.chan_class[sd.channel], sh = sd.shape;
     const bool small = sh >= 0 && is_small(cl, sh);
-    const int key = sh < 0 ? 8 * kNumShapes : (2 * shape_group(kShapes[sh].n_out) + (small ? 1 : 0)) * kNumShapes + sh;
+    const int key = sh < 0 || (small && !grouped[cl]) ? 8 * kNumShapes
+                    : grouped[cl]                     ? (2 * shape_group(kShapes[sh].n_out) + (small ? 1 : 0)) * kNumShapes + sh
+                                                      : sh;
     // order 1: heaviest programs first, so the tail of the launch is made of short tiles
     order[s] = Order{cl, key, pl.order == 1 ? -pl.chans[sd.channel].n_nodes : 0, (int)s};
     n_tiles += (sd.n_events + tile_events(cl) - 1) / tile_events(cl);
@@ -218,7 +238,8 @@ int plan_build(PlanObj& pl) {
     for (ShapeRun& r : pl.group_runs[c]) {
       if (r.sid > kRunOfGroup) continue;
       const int first = pl.segs[pl.tiles[r.begin].seg].shape, last = pl.segs[pl.tiles[r.end - 1].seg].shape;
-      if (first == last) r.sid = first;   // (a shape is either small or not: its tiles are together)
+      // (a shape is either small or not: its tiles are together, unless small shapes of this group are)
+      if (first == last && (grouped[c] || !is_small(c, first))) r.sid = first;
     }
 
   // upload: one allocation, 256-byte aligned sections
@@ -556,7 +577,7 @@ int gpu_phs_plan_set_config(int plan, int block, int ept, int grid, int order, i
   bool rebuild = order != pl->order;
   for (int c = 0; c < kTileClasses; c++) {
     const LaunchConfig& o = pl->lcs[c];
-    if (block != o.block || ept != o.ept) rebuild = true;
+    if (other_tiles(want, o)) rebuild = true;
     if (grid != o.grid || waves_per_eu != o.waves_per_eu || lds != o.lds) drop_graph(*pl);
     pl->lcs[c] = want;
   }
@@ -578,7 +599,7 @@ int gpu_phs_plan_set_class_config(int plan, int cls, int block, int ept, int gri
   if (pl->class_end[cls] > pl->class_begin[cls] && forward_lds_bytes(pl->dps[cls], want) > forward_lds_limit())
     return set_error(GPU_PHS_E_ARG, "the staging tables of this block size (and LDS save banks) exceed the LDS a "
                                     "workgroup may use on this device; choose a smaller block");
-  const bool rebuild = block != pl->lcs[cls].block || ept != pl->lcs[cls].ept;
+  const bool rebuild = other_tiles(want, pl->lcs[cls]);
   pl->lcs[cls] = want;
   drop_graph(*pl);
   if (rebuild) return plan_build(*pl);
@@ -783,7 +804,7 @@ int gpu_phs_plan_autotune(int plan, void* stream_v, int reps, char* report, int 
     Cfg best{cls, pl->lcs[cls], pl->order, 1e30f};
     auto consider = [&](LaunchConfig lc) -> int {
       if (forward_lds_bytes(pl->dps[cls], lc) > forward_lds_limit()) return GPU_PHS_OK;   // does not fit
-      const bool rebuild = lc.block != pl->lcs[cls].block || lc.ept != pl->lcs[cls].ept;
+      const bool rebuild = other_tiles(lc, pl->lcs[cls]);
       pl->lcs[cls] = lc;
       drop_graph(*pl);
       if (rebuild) {

@@ -48,7 +48,7 @@ struct PlanObj {
   // the class's launch shape has such a kernel; where not, a shape whose tiles in the class hold
   // fewer events than this runs in the class's one launch of the generic kernel
   int64_t merge_below = kMergeBelowDefault;
-  // each tile class split by shape (empty: one generic launch), and by shape group
+  // each tile class split by shape (-1: the generic launch), and by shape group
   std::vector<ShapeRun> shape_runs[2], group_runs[2];
   std::vector<ChannelDesc> chans;
   std::vector<NodeCmd> nodes;

@@ -221,3 +221,32 @@ build, sort = fastest(lambda: G.Plan(segs).close()), fastest(lambda: np.argsort(
 assert tiles > 70_000
 assert build < sort, (build, sort)
 """)
+
+
+@pytest.mark.parametrize("order", [0, 1])
+def test_small_shapes_share_one_generic_launch(run, order):
+    """Where a launch shape has no kernels for groups of shapes (a persistent grid), the small shapes of a tile class
+    run in one launch of the generic kernel, whatever their numbers of particles, and every large one in its own; else
+    each group in one of its own."""
+    run(f"""
+segs, large = [], 0
+for n_out in (5, 6):
+    ph = G.ProcessHandle(W.process_shapes(n_out, 1))
+    for c in range(ph.proc.n_channels):
+        n = 140 if c % 3 == 0 else 70
+        large += n == 140
+        segs.append((ph, c, G.EventBuffers(Array((n, ph.n_x)), Array((n, n_out, 4)), Array(n), Array(n),
+                                           Array(n, np.uint8))))
+pl = G.Plan(segs)
+pl.set_config(block=64, ept=1, order={order})
+pl.set_merge_below(100)
+for grid in (0, 256, 0, 256):
+    pl.set_config(grid=grid)
+    launches()
+    pl.run(Stream)
+    names = launches()
+    if grid:
+        assert len(names) == large + 1 and sum("ELin1E" in k for k in names) == 1, names
+    else:
+        assert len(names) == 2 and all("forward_shapes_kernel" in k for k in names), names
+""")
