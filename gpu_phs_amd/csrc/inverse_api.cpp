@@ -46,20 +46,19 @@ std::string association(const NodeCmd* prog, const ChildCmd& k) {
   return "(" + a + " " + b + ")";
 }
 
-// Per branch of channel c in visit order: everything its geometry depends on.
-std::vector<std::string> branch_keys(const CompiledProcess& cp, int c) {
-  const ChannelDesc& cd = cp.channels[c];
-  const NodeCmd* prog = &cp.nodes[cd.node0];
+// Per branch of channel c in visit order, of the first n: everything its geometry depends on.
+std::vector<std::string> branch_keys(const CompiledProcess& cp, int c, int n) {
+  const NodeCmd* prog = &cp.nodes[cp.channels[c].node0];
   std::vector<std::string> keys;
-  for (int i = 0; i < cd.n_nodes; i++) {
+  for (int i = 0; i < n; i++) {
     std::string up = i == 0 ? "" : keys[prog[i].parent] + "/" + std::to_string(prog[i].slot) + ":";
     keys.push_back(up + association(prog, prog[i].k[0]) + "," + association(prog, prog[i].k[1]));
   }
   return keys;
 }
 
-// Device tables of the inverse: per-segment (generating channel, first row), then the
-// process's channels and programs.  Re-uploaded only when the rows change.
+// Device tables of the inverse: per-segment (generating channel, first row), uploaded again when the rows
+// change, then the process's channels and programs.
 int inverse_prepare(PlanObj& pl, const int64_t* seg_row0, int64_t n_rows) {
   if (pl.segs.empty()) return set_error(GPU_PHS_E_ARG, "inverse: the plan has no segments");
   const int proc = pl.chan_process.empty() ? -1 : pl.chan_process[0];
@@ -78,15 +77,24 @@ int inverse_prepare(PlanObj& pl, const int64_t* seg_row0, int64_t n_rows) {
   }
   const bool shared = !cp.has_friends && pl.specialize;
   if (pl.inv_dev && pl.inv_process == proc && pl.inv.per_event_beams == pl.dp.per_event_beams &&
-      pl.inv.shared_roots == (shared ? 1 : 0) && is.size() == pl.inv_segs.size() &&
-      std::memcmp(is.data(), pl.inv_segs.data(), is.size() * sizeof(InvSeg)) == 0)
+      pl.inv.shared_roots == (shared ? 1 : 0) && is.size() == pl.inv_segs.size()) {
+    // the process's tables are there; the rows may be others
+    if (std::memcmp(is.data(), pl.inv_segs.data(), is.size() * sizeof(InvSeg)) == 0) return ok_status();
+    hipError_t e = hipMemcpy(pl.inv_dev, is.data(), is.size() * sizeof(InvSeg), hipMemcpyHostToDevice);
+    if (e != hipSuccess) return hip_error(e, "hipMemcpy(inverse rows)");
+    pl.inv_segs = std::move(is);
     return ok_status();
+  }
   const int n_ch = (int)cp.channels.size();
+  // the walk that reads a channel's structure from its program
+  bool generic = cp.spec.n_out > (pl.dp.per_event_beams ? kInvShapeOutPev : kInvShapeOut);
+  for (const ChannelDesc& c : cp.channels) generic = generic || c.shape < 0;
   // channel order: by what each branch, root first, computes from an event -- where it hangs, and both
   // daughters' final-state particles with the association their momenta are added in -- so that
-  // channels sharing their first branches' evaluation are adjacent; channel index within a group
+  // channels sharing their first branches' evaluation are adjacent (the generic walk shares the root's
+  // only); channel index within a group
   std::vector<std::vector<std::string>> keys(n_ch);
-  for (int c = 0; shared && c < n_ch; c++) keys[c] = branch_keys(cp, c);
+  for (int c = 0; shared && c < n_ch; c++) keys[c] = branch_keys(cp, c, generic ? 1 : cp.channels[c].n_nodes);
   std::vector<int> order(n_ch);
   for (int c = 0; c < n_ch; c++) order[c] = c;
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return keys[a] < keys[b]; });
@@ -130,7 +138,9 @@ int inverse_prepare(PlanObj& pl, const int64_t* seg_row0, int64_t n_rows) {
   const size_t o_nodes = o_chans + al(cp.channels.size() * sizeof(ChannelDesc));
   const size_t o_steps = o_nodes + al(cp.nodes.size() * sizeof(NodeCmd));
   const size_t o_maps = o_steps + al(steps.size() * sizeof(InvStep));
-  const size_t total = o_maps + al(cp.nodes.size() * sizeof(InvNode));
+  // (the walks specialised per tree shape read the maps' records; with per-event beams they read the programs)
+  const size_t n_maps = generic || pl.dp.per_event_beams ? 0 : cp.nodes.size();
+  const size_t total = o_maps + al(n_maps * sizeof(InvNode));
   if (total > pl.inv_bytes) {
     if (pl.inv_dev) (void)hipFree(pl.inv_dev);
     pl.inv_dev = nullptr;
@@ -144,7 +154,7 @@ int inverse_prepare(PlanObj& pl, const int64_t* seg_row0, int64_t n_rows) {
   std::memcpy(host.data() + o_chans, cp.channels.data(), cp.channels.size() * sizeof(ChannelDesc));
   std::memcpy(host.data() + o_nodes, cp.nodes.data(), cp.nodes.size() * sizeof(NodeCmd));
   std::memcpy(host.data() + o_steps, steps.data(), steps.size() * sizeof(InvStep));
-  for (size_t i = 0; i < cp.nodes.size(); i++) {
+  for (size_t i = 0; i < n_maps; i++) {
     const InvNode nd = inv_node(cp.nodes[i]);
     std::memcpy(host.data() + o_maps + i * sizeof(InvNode), &nd, sizeof nd);
   }
@@ -174,10 +184,8 @@ int inverse_prepare(PlanObj& pl, const int64_t* seg_row0, int64_t n_rows) {
   // a repeated branch saves about a third of its channel's work, the tests for it cost a tenth of
   // every channel's: worth it where a quarter of the branches repeat
   pl.inv.shared_branches = shared && 4 * evaluated <= 3 * branches ? 1 : 0;
-  pl.inv.generic = cp.spec.n_out > (pl.dp.per_event_beams ? kInvShapeOutPev : kInvShapeOut) ? 1 : 0;
-  for (const ChannelDesc& c : cp.channels)
-    if (c.shape < 0) pl.inv.generic = 1;
-  if (pl.inv.generic || cp.spec.n_out > 4) pl.inv.shared_branches = 0;
+  pl.inv.generic = generic ? 1 : 0;
+  if (generic || cp.spec.n_out > 4) pl.inv.shared_branches = 0;
   pl.inv_segs = std::move(is);
   pl.inv_process = proc;
   return ok_status();

@@ -250,3 +250,29 @@ for grid in (0, 256, 0, 256):
     else:
         assert len(names) == 2 and all("forward_shapes_kernel" in k for k in names), names
 """)
+
+
+def test_inverse_tables_are_cheap(run):
+    """Preparing the inverse of a process (2,000 channels of eight particles) takes a small part of the time that
+    compiling its trees takes, and a call with other output rows prepares nothing again."""
+    run("""
+proc = W.process_large(8, 2000)
+ph, L = G.ProcessHandle(proc), G.lib()
+buf = Array((64, 8))
+one = [(ph, 0, G.EventBuffers(Array((64, proc.n_x)), Array((64, 8, 4)), Array(64), Array(64), Array(64, np.uint8)))]
+def seconds(f):
+    start = time.perf_counter()
+    f()
+    return time.perf_counter() - start
+def inverse(pl, row):
+    rows = np.array([row], np.int64)
+    assert L.gpu_phs_plan_inverse(pl.handle, p(rows), 1000, p(buf.a), p(buf.a), 0, None) == 0
+compiled = min(seconds(lambda: G.ProcessHandle(proc).close()) for _ in range(7))
+first, again = [], []
+for _ in range(7):
+    pl = G.Plan(one)
+    first.append(seconds(lambda: inverse(pl, 0)))
+    again += [seconds(lambda: inverse(pl, row)) for row in (1, 2, 3)]
+assert min(first) < 0.08 * compiled, (min(first), compiled)
+assert min(again) < 0.1 * min(first), (min(again), min(first))
+""")
