@@ -177,8 +177,9 @@ int ensure_staging(WhizardModule& w) {
 
 // Threads that copy between pinned and pageable memory beside the calling one: started at the first large
 // transfer and kept until the library is unloaded.  One thread copies some 10-15 GB/s, well below what
-// PCIe moves.
-constexpr int kCopyThreads = 7;
+// PCIe moves (a call of 10^5 2 -> 4 events with four threads 1.10 ms, with five 1.07, with seven 1.06 and a quarter
+// more processor time).
+constexpr int kCopyThreads = 5;
 class CopyPool {
  public:
   // Runs `job` on every thread, until wait(); the number of threads (0 if none can be started).
@@ -237,15 +238,17 @@ CopyPool& copy_pool() {
   return pool;
 }
 
-// A condition that other threads bring about and announce with changed(): waited for asleep after the time between
-// two chunks, so that the copy threads take no time from the host program while the kernels run.  A call of
-// 10^6 2 -> 4 events uses 50 ms of processor time, of 10^5 4.4 (41 and 3.7 without the active wait, which the
-// 10^5 repay with 2% of their 1.06 ms; 67 and 7.7 with threads that only wait actively).
+// A condition that other threads bring about and announce with changed(): waited for asleep after kAwake, about the
+// time from one chunk to the next, so that the copy threads take nothing from the host program while the
+// kernels run or the link is slow.  Calls of 1,818 2 -> 6, 10^5 and 10^6 2 -> 4 events, time and processor time:
+// 208 us and 0.82 ms, 1.07 and 4.9 ms, 8.9 and 48 ms; with seven threads that only wait actively 209 us and 1.2 ms,
+// 1.07 and 7.9 ms, 9.0 and 68 ms; asleep after 20 us 218 us and 0.74 ms, 1.06 and 4.7 ms, 9.2 and 50 ms.
+constexpr std::chrono::microseconds kAwake{100};
 class Waiting {
  public:
   template <class Done>
   void until(Done done) {
-    const auto end = std::chrono::steady_clock::now() + std::chrono::microseconds(20);
+    const auto end = std::chrono::steady_clock::now() + kAwake;
     do {
       for (int k = 0; k < 32; k++) {
         if (done()) return;
@@ -341,16 +344,18 @@ int transfer(WhizardModule& w, const std::vector<Transfer>& list, bool to_device
   hipError_t e = hipSuccess;
   // the slots' DMAs of the previous transfer; to the host, the other stream follows the kernels
   for (int c = 0; to_device && c < std::min(n, kPinSlots) && e == hipSuccess; c++) e = arrived(c);
-  if (!to_device && n > 1 && (e = hipEventRecord(w.kernels_ev, w.stream)) == hipSuccess)
+  if (!to_device && (e = hipEventRecord(w.kernels_ev, w.stream)) == hipSuccess && n > 1)
     e = hipStreamWaitEvent(w.stream2, w.kernels_ev, 0);
   if (e != hipSuccess) return failed(e, "staging events");
-  const int threads = total >= kPoolBytes ? copy_pool().start(pieces) : 0;
+  int threads = 0;
+  auto start = [&] { threads = total >= kPoolBytes ? copy_pool().start(pieces) : 0; };
   auto copy_whole = [&](int c) {   // without threads
     if (threads > 0) return;
     host_copy(c, 0, chunks[c].n);
     left[c].store(0, std::memory_order_relaxed);
   };
   if (to_device) {
+    start();
     for (int c = 0, freed = 0; c < n && e == hipSuccess; c++) {
       copy_whole(c);
       for_copied.until([&] { return copied(c); });
@@ -369,6 +374,8 @@ int transfer(WhizardModule& w, const std::vector<Transfer>& list, bool to_device
         }
         e = dma(issued);
       }
+      // the threads sleep through the kernels and wake up during the first DMA
+      if (c == 0 && e == hipSuccess && (e = hipEventSynchronize(w.kernels_ev)) == hipSuccess) start();
       if (e == hipSuccess) e = arrived(c);
       if (e == hipSuccess) open_to(c + 1);
       if (e == hipSuccess) copy_whole(c);

@@ -273,6 +273,6 @@ for _ in range(7):
     pl = G.Plan(one)
     first.append(seconds(lambda: inverse(pl, 0)))
     again += [seconds(lambda: inverse(pl, row)) for row in (1, 2, 3)]
-assert min(first) < 0.08 * compiled, (min(first), compiled)
+assert min(first) < 0.1 * compiled, (min(first), compiled)
 assert min(again) < 0.1 * min(first), (min(again), min(first))
 """)
