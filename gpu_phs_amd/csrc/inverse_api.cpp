@@ -226,8 +226,11 @@ int gphs::plan_inverse(PlanObj& pl, const int64_t* seg_row0, int64_t n_rows, dou
   }
   if (inverse_lds_bytes(pl.inv, block) > forward_lds_limit())
     return set_error(GPU_PHS_E_ARG, "inverse: the trees need more LDS than a workgroup of this size may use");
-  hipError_t e = launch_inverse(pl.inv, pl.dp.tiles, pl.dp.n_tiles, std::max(1, (pl.tile_max + 63) / 64), pl.dp.segs,
-                                block, inverse_chunks(pl.inv, pl.n_units), factors, x_out, n_rows, stream);
+  // shared roots: a wave per 64-event unit, of every tile as many as the largest has or of those that have events
+  const bool listed = pl.inv.shared_roots && pl.dp.units;
+  hipError_t e = launch_inverse(pl.inv, listed ? pl.dp.units : pl.dp.tiles, listed ? (int)pl.units.size() : pl.dp.n_tiles,
+                                listed ? 1 : std::max(1, (pl.tile_max + 63) / 64), pl.dp.segs, block,
+                                inverse_chunks(pl.inv, pl.n_units), factors, x_out, n_rows, stream);
   if (e != hipSuccess) return hip_error(e, "inverse launch");
   return ok_status();
 }

@@ -233,6 +233,35 @@ int plan_build(PlanObj& pl) {
     extend(pl.shape_runs[c], sh >= 0 && is_small(c, sh) ? -1 : sh, begin, end, bytes);
     extend(pl.group_runs[c], sh < 0 ? -1 : kRunOfGroup - shape_group(kShapes[sh].n_out), begin, end, bytes);
   }
+  // A launch takes ept workgroups for every tile, or a wave for each 64 events that the largest one has.  Where more
+  // than one in nine would find no events (many segments of fewer events than a tile), the parts with
+  // events are listed instead: 1,500 segments of 70 events of 2 -> 8 trees, tiles of 256, 64 us, 119 with the
+  // empty workgroups (tiles of 1024: 64 and 428); 400 segments and 120 channels of 2 -> 4, the inverse, 0.29 and
+  // 2.46 ms with one segment of 20,000 events beside them.
+  pl.subs.clear();
+  pl.units.clear();
+  pl.sub_begin.clear();
+  auto parts = [&](int begin, int end, int events, std::vector<TileDesc>& out, std::vector<int>* first) {
+    for (int t = begin; t < end; t++) {
+      if (first) (*first)[t] = (int)out.size();
+      const TileDesc& td = pl.tiles[t];
+      for (int e = 0; e < td.count; e += events)
+        out.push_back(TileDesc{td.seg, std::min(events, td.count - e), td.e0 + e});
+    }
+    if (first) (*first)[end] = (int)out.size();
+  };
+  bool listed[kTileClasses];
+  for (int c = 0; c < kTileClasses; c++) {
+    int64_t used = 0;
+    for (int t = pl.class_begin[c]; t < pl.class_end[c]; t++)
+      used += (pl.tiles[t].count + pl.lcs[c].block - 1) / pl.lcs[c].block;
+    listed[c] = 8 * (int64_t)pl.lcs[c].ept * (pl.class_end[c] - pl.class_begin[c]) > 9 * used;
+    if (!listed[c]) continue;
+    pl.sub_begin.resize(pl.tiles.size() + 1);
+    parts(pl.class_begin[c], pl.class_end[c], pl.lcs[c].block, pl.subs, &pl.sub_begin);
+  }
+  if (8 * (int64_t)pl.tiles.size() * ((pl.tile_max + 63) / 64) > 9 * pl.n_units)
+    parts(0, (int)pl.tiles.size(), 64, pl.units, nullptr);
   // a group run of one shape: that shape's kernel
   for (int c = 0; c < kTileClasses; c++)
     for (ShapeRun& r : pl.group_runs[c]) {
@@ -247,7 +276,9 @@ int plan_build(PlanObj& pl) {
   size_t o_tiles = 0, o_segs = al(pl.tiles.size() * sizeof(TileDesc));
   size_t o_chans = o_segs + al(pl.segs.size() * sizeof(SegDesc));
   size_t o_nodes = o_chans + al(pl.chans.size() * sizeof(ChannelDesc));
-  size_t total = o_nodes + al(pl.nodes.size() * sizeof(NodeCmd)) + 256;
+  const size_t o_subs = o_nodes + al(pl.nodes.size() * sizeof(NodeCmd));
+  const size_t o_units = o_subs + al(pl.subs.size() * sizeof(TileDesc));
+  size_t total = o_units + al(pl.units.size() * sizeof(TileDesc)) + 256;
   drop_graph(pl);
   if (total > pl.dev_bytes) {
     if (pl.dev) (void)hipFree(pl.dev);
@@ -262,6 +293,8 @@ int plan_build(PlanObj& pl) {
   if (!pl.segs.empty()) std::memcpy(host.data() + o_segs, pl.segs.data(), pl.segs.size() * sizeof(SegDesc));
   if (!pl.chans.empty()) std::memcpy(host.data() + o_chans, pl.chans.data(), pl.chans.size() * sizeof(ChannelDesc));
   if (!pl.nodes.empty()) std::memcpy(host.data() + o_nodes, pl.nodes.data(), pl.nodes.size() * sizeof(NodeCmd));
+  if (!pl.subs.empty()) std::memcpy(host.data() + o_subs, pl.subs.data(), pl.subs.size() * sizeof(TileDesc));
+  if (!pl.units.empty()) std::memcpy(host.data() + o_units, pl.units.data(), pl.units.size() * sizeof(TileDesc));
   hipError_t e = hipMemcpy(pl.dev, host.data(), total, hipMemcpyHostToDevice);
   if (e != hipSuccess) return hip_error(e, "hipMemcpy(plan tables)");
   char* base = (char*)pl.dev;
@@ -270,6 +303,7 @@ int plan_build(PlanObj& pl) {
   pl.dp.chans = (const ChannelDesc*)(base + o_chans);
   pl.dp.nodes = (const NodeCmd*)(base + o_nodes);
   pl.dp.n_tiles = (int)pl.tiles.size();
+  pl.dp.units = pl.units.empty() ? nullptr : (const TileDesc*)(base + o_units);
   // maxima over all channels (adjoint) and over each class (forward launches)
   auto maxima = [&](DevicePlan& d, int cl) {
     d.n_banks = 0; d.nx_max = d.nout_max = 0; d.root_banks_only = 1; d.has_friends = 0; d.per_event_beams = 0;
@@ -291,6 +325,10 @@ int plan_build(PlanObj& pl) {
   for (int c = 0; c < kTileClasses; c++) {
     pl.dps[c] = pl.dp;
     maxima(pl.dps[c], c);
+    if (listed[c]) {
+      pl.dps[c].subs = (const TileDesc*)(base + o_subs);
+      pl.dps[c].sub_begin = pl.sub_begin.data();
+    }
   }
   for (int c = 0; c < kTileClasses; c++)
     if (pev[c]) pl.dp.per_event_beams = pl.dps[c].per_event_beams = 1;

@@ -80,14 +80,18 @@ size_t forward_lds_limit() {
 namespace {
 
 // Workgroups of a launch over n tiles: one per tile (looping kernels; lc.grid > 0 strides) or one per
-// sub-tile.
+// sub-tile (of those that have events, where they are listed).
 hipError_t launch(FwdKernel k, bool one, const DevicePlan& dp, int t_begin, int t_end, const LaunchConfig& lc,
                   size_t shmem, int nx_max, int nout_max, hipStream_t stream) {
   if (!k || lc.ept < 1) return hipErrorInvalidValue;
-  const int64_t n = t_end - t_begin;
-  const int64_t grid = one ? n * lc.ept : lc.grid > 0 ? std::min<int64_t>(lc.grid, n) : n;
+  const bool listed = one && dp.subs;
+  const TileDesc* tiles = listed ? dp.subs : dp.tiles;
+  const int begin = listed ? dp.sub_begin[t_begin] : t_begin, end = listed ? dp.sub_begin[t_end] : t_end;
+  const int ept = listed ? 1 : lc.ept;
+  const int64_t n = end - begin;
+  const int64_t grid = one ? n * ept : lc.grid > 0 ? std::min<int64_t>(lc.grid, n) : n;
   if (grid > 0x7fffffff) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(lc.block), shmem, stream, dp.tiles, t_begin, t_end, lc.ept, dp.segs,
+  hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(lc.block), shmem, stream, tiles, begin, end, ept, dp.segs,
                      dp.chans, dp.nodes, nx_max, nout_max);
   return hipGetLastError();
 }

@@ -9,6 +9,11 @@ namespace gphs {
 // Device copies of one plan's tables.
 struct DevicePlan {
   const TileDesc* tiles = nullptr;
+  // where many tiles are not full, the tiles' sub-tiles of one workgroup of the class (sub_begin, on the host: the
+  // first of each tile), and the 64-event units of all tiles; else null
+  const TileDesc* subs = nullptr;
+  const int* sub_begin = nullptr;
+  const TileDesc* units = nullptr;
   const SegDesc* segs = nullptr;
   const ChannelDesc* chans = nullptr;
   const NodeCmd* nodes = nullptr;

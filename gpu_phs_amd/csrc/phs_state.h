@@ -56,6 +56,9 @@ struct PlanObj {
   std::vector<TileDesc> tiles;
   int tile_max = 0;                        // events of the largest tile
   int64_t n_units = 0;                     // wavefronts of 64 events the tiles fill
+  // the parts of tiles that are not full (DevicePlan::subs, units); empty where the tiles are mostly full
+  std::vector<TileDesc> subs, units;
+  std::vector<int> sub_begin;
   std::vector<int> seg_tile_begin, seg_tile_end;  // tile ranges per segment (segment order)
   int n_banks = 0;
   // Tile classes: channels of up to 8 randoms whose only deferring branch is the root (class 0)
@@ -69,7 +72,7 @@ struct PlanObj {
   std::vector<int> chan_class;   // class of each plan channel
   int order = 0;
   int serial_classes = 0;                   // 1: the two classes run one after the other on one stream
-  void* dev = nullptr;                      // one allocation: tiles | segs | chans | nodes
+  void* dev = nullptr;                      // one allocation: tiles | segs | chans | nodes | subs | units
   size_t dev_bytes = 0;
   DevicePlan dp;
   hipGraph_t graph = nullptr;

@@ -5,6 +5,7 @@
 #define __HIP_PLATFORM_AMD__
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
 #include <chrono>
 #include <cstdlib>
 #include <cstring>
@@ -38,6 +39,8 @@ std::map<const void*, std::string> names;
 std::vector<std::string> launched;
 std::vector<hipStream_t> streams;
 std::map<char*, size_t> allocated;
+int64_t groups = 0;
+size_t most_lds = 0;
 int violations = 0, fail_wait_after = -1, wait_us = 0, lds = 160 * 1024;
 double elapsed = 0, elapsed_step = 0;
 struct Config { dim3 grid, block; size_t shmem; hipStream_t stream; } config;
@@ -111,6 +114,14 @@ int hip_host_launches(char* out, int len) {
   launched.clear();
   snprintf(out, len, "%s", all.c_str());
   return (int)all.size();
+}
+// The most LDS that a launch has asked for so far.
+int64_t hip_host_most_lds() { return (int64_t)most_lds; }
+// The workgroups launched since the last call.
+int64_t hip_host_groups() {
+  const int64_t n = groups;
+  groups = 0;
+  return n;
 }
 
 // ---- the runtime
@@ -195,8 +206,10 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* shmem, hip
   *grid = config.grid; *block = config.block; *shmem = config.shmem; *s = config.stream;
   return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void* f, dim3, dim3, void**, size_t, hipStream_t) {
+hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3, void**, size_t shmem, hipStream_t) {
   launched.push_back(names[f]);
+  most_lds = std::max(most_lds, shmem);
+  groups += (int64_t)grid.x * grid.y * grid.z;
   return hipSuccess;
 }
 

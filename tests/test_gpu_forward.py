@@ -294,3 +294,42 @@ def test_shared_launches_identical_to_own(parts, cfg):
         for r in results[1:]:
             for a, b in zip(results[0], r):
                 assert torch.equal(torch.nan_to_num(a), torch.nan_to_num(b))
+
+
+@pytest.mark.parametrize("process", ["c1", "2to6", "large8", "friends6"])
+def test_short_segments_in_large_tiles(process):
+    """Many segments of fewer events than a tile has room for, whose sub-tiles with events are listed: forward, plain
+    and graph launches and the inverse give the bits that tiles of one sub-tile give."""
+    import torch
+    import gpu_phs_amd as G
+    proc = {"c1": W.process_c1, "2to6": W.process_2to6, "large8": lambda: W.process_large(8),
+            "friends6": lambda: W.process_friends(6)}[process]()
+    ph = G.ProcessHandle(proc)
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    segs = []
+    for k in range(90):
+        n = (70, 64, 1, 129, 63, 1025)[k % 6]
+        x = torch.rand((n, proc.n_x), generator=gen, device="cuda", dtype=torch.float64)
+        segs.append((ph, (7 * k) % proc.n_channels, G.EventBuffers.allocate(x, proc.n_out)))
+    plan = G.Plan(segs)
+
+    def outputs(run):
+        for _, _, b in segs:
+            for t in (b.p, b.factor, b.volume, b.ok):
+                t.zero_()
+        run()
+        torch.cuda.synchronize()
+        return [t.cpu().numpy().copy() for _, _, b in segs for t in (b.p, b.factor, b.volume, b.ok)]
+
+    want, inv = None, None
+    for block, ept in ((64, 1), (64, 16), (64, 4), (128, 3)):
+        if process == "large8" and block > 64:
+            continue
+        plan.set_config(block=block, ept=ept)
+        for run in (plan.run, plan.run_plain, plan.run_graph, plan.run_graph):
+            got = outputs(run)
+            want = got if want is None else want
+            assert all(np.array_equal(a, b, equal_nan=True) for a, b in zip(got, want)), (block, ept)
+        got = [t.cpu().numpy() for t in plan.inverse()]
+        inv = got if inv is None else inv
+        assert all(np.array_equal(a, b, equal_nan=True) for a, b in zip(got, inv)), (block, ept)

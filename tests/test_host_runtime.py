@@ -18,6 +18,7 @@ import numpy as np
 import gpu_phs_amd as G
 from gpu_phs_amd import workloads as W
 H.hip_host_elapsed.argtypes = [ctypes.c_double, ctypes.c_double]
+H.hip_host_groups.restype = H.hip_host_most_lds.restype = ctypes.c_int64
 
 def i(v):
     return ctypes.byref(ctypes.c_int(v))
@@ -275,4 +276,35 @@ for _ in range(7):
     again += [seconds(lambda: inverse(pl, row)) for row in (1, 2, 3)]
 assert min(first) < 0.1 * compiled, (min(first), compiled)
 assert min(again) < 0.1 * min(first), (min(again), min(first))
+""")
+
+
+@pytest.mark.parametrize("process", ["W.process_c1()", "W.process_2to6()", "W.process_large(8)", "W.process_friends(6)"])
+def test_launches_have_no_empty_workgroups(run, process):
+    """A plan of many segments shorter than a tile launches workgroups for the events there are, not for those its
+    tiles have room for: forward, plain and inverse, at every number of sub-tiles per tile."""
+    run(f"""
+proc = {process}
+ph, segs = G.ProcessHandle(proc), []
+for k in range(300):
+    n = (70, 64, 1, 129)[k % 4]
+    segs.append((ph, k % proc.n_channels, G.EventBuffers(Array((n, proc.n_x)), Array((n, proc.n_out, 4)), Array(n), Array(n),
+                                                         Array(n, np.uint8))))
+used = 75 * (2 + 1 + 1 + 3)   # workgroups of 64 events
+rows = np.zeros(300, np.int64)
+pl = G.Plan(segs)
+for ept in (1, 4, 16, 2):
+    pl.set_config(block=64, ept=ept, grid=0)
+    H.hip_host_groups()
+    pl.run(Stream)
+    assert used <= H.hip_host_groups() <= 1.2 * used, ept
+    pl.run_plain(Stream)
+    assert used <= H.hip_host_groups() <= 1.2 * used, ept
+    if not proc.friends_or_zero().any():
+        assert G.lib().gpu_phs_plan_inverse(pl.handle, p(rows), 1000, p(rows), p(rows), 64, None) == 0
+        n = H.hip_host_groups()
+        assert n % used == 0 and n // used <= proc.n_channels, (ept, n)
+pl.set_config(ept=16, grid=100)   # a persistent grid goes through tiles
+pl.run(Stream)
+assert H.hip_host_groups() <= 400
 """)
