@@ -152,9 +152,7 @@ int gpu_phs_grid_update(int grid, int plan, void* stream) {
       return hip_error(e, "hipMalloc(grid counts)");
     g->counts_cap = need;
   }
-  int64_t n_events = 0;
-  for (const SegDesc& sd : pl->segs) n_events += sd.n_events;
-  if ((e = launch_grid_histogram(pl->dp, n_events, (int)nch, g->n_dim, g->counts_d, (hipStream_t)stream)) != hipSuccess)
+  if ((e = launch_grid_histogram(pl->dp, pl->n_events, pl->busiest, (int)nch, g->n_dim, g->counts_d, (hipStream_t)stream)) != hipSuccess)
     return hip_error(e, "grid histogram launch");
   std::vector<unsigned long long> h(need);
   if ((e = hipMemcpyAsync(h.data(), g->counts_d, need * sizeof(unsigned long long), hipMemcpyDeviceToHost,

@@ -198,7 +198,8 @@ int plan_build(PlanObj& pl) {
   });
   pl.tiles.reserve(n_tiles);
   pl.tile_max = 0;
-  pl.n_units = 0;
+  pl.n_events = pl.n_units = 0;
+  std::vector<int> chan_tiles(pl.chans.size(), 0);
   pl.seg_tile_begin.assign(pl.segs.size(), 0);
   pl.seg_tile_end.assign(pl.segs.size(), 0);
   for (int c = 0; c < kTileClasses; c++) {
@@ -225,6 +226,8 @@ int plan_build(PlanObj& pl) {
     if (pl.class_end[c] == 0) pl.class_begin[c] = begin;
     pl.class_end[c] = end;
     pl.tile_max = std::max(pl.tile_max, (int)std::min<int64_t>(tile, sd.n_events));
+    pl.n_events += sd.n_events;
+    chan_tiles[sd.channel] += end - begin;
     pl.n_units += (sd.n_events + 63) / 64;   // (tiles are whole units but for a segment's last)
     // the class by shape and by shape group (with per-event beams, only the trees of up to four final-state
     // particles have specialised kernels; the others run the generic one)
@@ -233,6 +236,7 @@ int plan_build(PlanObj& pl) {
     extend(pl.shape_runs[c], sh >= 0 && is_small(c, sh) ? -1 : sh, begin, end, bytes);
     extend(pl.group_runs[c], sh < 0 ? -1 : kRunOfGroup - shape_group(kShapes[sh].n_out), begin, end, bytes);
   }
+  pl.busiest = chan_tiles.empty() ? 0 : *std::max_element(chan_tiles.begin(), chan_tiles.end());
   // A launch takes ept workgroups for every tile, or a wave for each 64 events that the largest one has.  Where more
   // than one in nine would find no events (many segments of fewer events than a tile), the parts with
   // events are listed instead: 1,500 segments of 70 events of 2 -> 8 trees, tiles of 256, 64 us, 119 with the

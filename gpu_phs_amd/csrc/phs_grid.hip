@@ -194,9 +194,10 @@ __global__ __launch_bounds__(kGenThreads) void grid_generate_kernel(const TileDe
 // events of 8 randoms in 3 channels).  Four workgroups per CU fill it with loads in flight: eight
 // randoms and flags per thread, which the whole batches load without a test (guarded, each load waits in a
 // branch of its own: 63 us for the same events after a forward pass, 66 with the one element per thread tested
-// for in the loop, 46 as it is, 5.6 TB/s of the randoms).  The workgroups were chosen on the first version: 49
-// us at 1024, 55 at 512, 87 at 256, 62 at 2048, where the atomics show again; fewer for few events
-// (launch_grid_histogram).
+// for in the loop, 46 as it is, 5.6 TB/s of the randoms).  The flags come a batch ahead, and the randoms of
+// rejected events are not read: deep trees reject most of theirs (2e6 events of 2 -> 8 trees 29 us, 54 with all
+// rows read).  The workgroups were chosen on the first version: 49 us at 1024, 55 at 512, 87 at 256, 62 at
+// 2048, where the atomics show again; fewer for few events (launch_grid_histogram).
 constexpr int kHistThreads = 512;
 constexpr int kHistGroups = 1024;
 constexpr int kHistUnroll = 8;                                     // loads in flight per thread
@@ -246,7 +247,7 @@ __global__ __launch_bounds__(kHistThreads) void grid_histogram_kernel(const Tile
         fields = 0;
       };
       // element u of a batch from its first one: its bin and whether it counts
-      auto count = [&](double xe, unsigned int accept) {
+      auto count = [&](double xe, bool accept) {
         int b = (int)(xe * kGridBins);   // rng.cpp:52
         b = b < 0 ? 0 : b > kGridBins - 1 ? kGridBins - 1 : b;
         const unsigned int one = accept ? 1u : 0u;
@@ -258,33 +259,46 @@ __global__ __launch_bounds__(kHistThreads) void grid_histogram_kernel(const Tile
       int64_t e = td.e0;            // first event of the pass
       const gdouble* px = xk + (e + r) * n_x;
       const guint8* po = ok + (e + r);
-      // whole batches: every load is inside, without a test
-      for (; e + per * kHistUnroll <= e_end; e += per * kHistUnroll) {
-        double xv[kHistUnroll];
-        unsigned int in[kHistUnroll];
+      const gdouble* x0 = as_global(sd.x);   // read in the place of the randoms of rejected events
+      unsigned int in[kHistUnroll];
+      auto load_flags = [&]() {
+#pragma unroll
+        for (int u = 0; u < kHistUnroll; u++) in[u] = po[u * per];
+        po += kHistUnroll * per;
+      };
+      // whole batches: every load is inside, without a test; the flags of the next one with the randoms of this
+      const int batch = per * kHistUnroll;
+      if (e + batch <= e_end) load_flags();
+      for (; e + batch <= e_end; e += batch) {
+        bool accept[kHistUnroll], any = false;
 #pragma unroll
         for (int u = 0; u < kHistUnroll; u++) {
-          in[u] = po[u * per];
-          xv[u] = px[u * step];
+          accept[u] = in[u] != 0;
+          any = any || accept[u];
+        }
+        if (e + 2 * batch <= e_end) load_flags();
+        if (__any(any)) {
+          double xv[kHistUnroll];
+#pragma unroll
+          for (int u = 0; u < kHistUnroll; u++) xv[u] = *(accept[u] ? px + u * step : x0);
+#pragma unroll
+          for (int u = 0; u < kHistUnroll; u++) count(xv[u], accept[u]);
         }
         px += kHistUnroll * step;
-        po += kHistUnroll * per;
-#pragma unroll
-        for (int u = 0; u < kHistUnroll; u++) count(xv[u], in[u]);
         if (++passes == kHistPasses) { flush(); passes = 0; }
       }
       const int left = (int)(e_end - e);   // events after them
       if (left > per) {
-        // elements past the end read the thread's first one, which is inside, and do not count
+        // elements past the end read the thread's first flag, which is inside, and do not count
         double xv[kHistUnroll];
-        unsigned int in[kHistUnroll];
 #pragma unroll
         for (int u = 0; u < kHistUnroll; u++) {
           const bool inside = u * per + r < left;
           in[u] = po[inside ? u * per : 0];
-          xv[u] = px[inside ? u * step : 0];
           if (!inside) in[u] = 0;
         }
+#pragma unroll
+        for (int u = 0; u < kHistUnroll; u++) xv[u] = *(in[u] ? px + u * step : x0);
 #pragma unroll
         for (int u = 0; u < kHistUnroll; u++) count(xv[u], in[u]);
       } else if (r < left) {   // one element per thread: counted at once
@@ -313,9 +327,15 @@ __global__ __launch_bounds__(kHistThreads) void grid_histogram_kernel(const Tile
   }
 }
 
-// The same for few tiles, a workgroup each, a thread per event: nothing to set up, one pass (at most kHistFew
-// tiles: 18,067 events of 2 randoms 3.3 us, 4.6 with the kernel above; 1,003 of 8 3.2 and 5.0).
-constexpr int kHistFew = 128;
+// The same a tile per workgroup and a thread per event: nothing to set up, one pass.  For few events (18,067 of 2
+// randoms 3.3 us, 4.6 with the kernel above; 1,003 of 8 3.2 and 5.0), and few tiles of any one channel, whose
+// counts meet at the same addresses (whole updates of 1 x 10^5 and 2 x 10^5 events in 3 channels, 130 and 260
+// tiles each: 33.3 and 39.0 us, 34.2 and 34.7 above; 2000 tiles of 70 events in 42 channels 40 and 44): at most
+// kHistFew.  A row per thread is read less well than a row's words by neighbouring threads, which shows in large
+// updates: 4.5 x 10^5 events 39.7 and 39.5 us (5 particles), 41.2 and 38.9 (6), 36.7 and 41.7 (8), 2 x 10^6
+// 82 and 51 (5): at most kHistFewEvents.
+constexpr int kHistFew = 192;
+constexpr int64_t kHistFewEvents = 1 << 19;
 __global__ __launch_bounds__(256) void grid_histogram_few_kernel(const TileDesc* __restrict__ tiles,
                                                                  const SegDesc* __restrict__ segs,
                                                                  const ChannelDesc* __restrict__ chans, int n_dim,
@@ -364,8 +384,8 @@ hipError_t launch_grid_generate(const DevicePlan& dp, const double* cdf, int n_d
   return hipGetLastError();
 }
 
-hipError_t launch_grid_histogram(const DevicePlan& dp, int64_t n_events, int n_chans, int n_dim, unsigned long long* counts,
-                                 hipStream_t stream) {
+hipError_t launch_grid_histogram(const DevicePlan& dp, int64_t n_events, int busiest, int n_chans, int n_dim,
+                                 unsigned long long* counts, hipStream_t stream) {
   unsigned long long* n_ok = counts + (size_t)n_chans * n_dim * kGridBins;
   const size_t n = (size_t)n_chans * n_dim * kGridBins + n_chans;
   hipLaunchKernelGGL(fill_u64_kernel, dim3((unsigned)std::min<size_t>((n + 255) / 256, 1024)), dim3(256), 0, stream,
@@ -373,16 +393,17 @@ hipError_t launch_grid_histogram(const DevicePlan& dp, int64_t n_events, int n_c
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || dp.n_tiles <= 0) return e;
   const size_t shmem = ((size_t)n_dim * kGridBins + 1) * sizeof(unsigned int);
-  if (dp.n_tiles <= kHistFew) {
+  const int64_t batches = n_events * n_dim / (kHistThreads * kHistUnroll);
+  if (busiest <= kHistFew && n_events <= kHistFewEvents) {
     hipLaunchKernelGGL(grid_histogram_few_kernel, dim3(dp.n_tiles), dim3(256), shmem, stream, dp.tiles, dp.segs, dp.chans,
                        n_dim, counts, n_ok);
     return hipGetLastError();
   }
-  // at most a workgroup for each batch of loads beyond the first kHistFew: every workgroup's counts go to the
-  // same few addresses one after the other, some 18 ns each (2 x 10^5 events of 2 randoms: 18 us at one
-  // workgroup per tile, 782; 7.8 at 98)
-  const int64_t batches = n_events * n_dim / (kHistThreads * kHistUnroll);
-  const int groups = (int)std::min<int64_t>({dp.n_tiles, kHistGroups, std::max<int64_t>(kHistFew, batches)});
+  // at most a workgroup for each batch of loads beyond the first kHistFew of a channel: every workgroup's counts go
+  // to the channel's few addresses one after the other, some 18 ns each (2 x 10^5 events of 2 randoms: 18 us at
+  // one workgroup per tile, 782; 7.8 at 98)
+  const int64_t channels = dp.n_tiles / std::max(1, busiest);
+  const int groups = (int)std::min<int64_t>({dp.n_tiles, kHistGroups, std::max<int64_t>(kHistFew * channels, batches)});
   hipLaunchKernelGGL(grid_histogram_kernel, dim3(groups), dim3(kHistThreads), shmem, stream, dp.tiles,
                      dp.n_tiles / groups, dp.n_tiles % groups, dp.segs, dp.chans, n_dim, counts, n_ok);
   return hipGetLastError();

@@ -133,8 +133,9 @@ constexpr int kGridBins = 10;
 // Randoms of every segment of the plan drawn from the grids: cdf [plan channel][n_dim][11].
 hipError_t launch_grid_generate(const DevicePlan& dp, const double* cdf, int n_dim, uint64_t seed, hipStream_t stream);
 // counts [plan channel][n_dim][10] histogram of the accepted events' randoms, then the accepted
-// count of every plan channel (n_chans more entries); cleared first.
-hipError_t launch_grid_histogram(const DevicePlan& dp, int64_t n_events, int n_chans, int n_dim, unsigned long long* counts,
-                                 hipStream_t stream);
+// count of every plan channel (n_chans more entries); cleared first.  busiest: tiles of the channel that
+// has most.
+hipError_t launch_grid_histogram(const DevicePlan& dp, int64_t n_events, int busiest, int n_chans, int n_dim,
+                                 unsigned long long* counts, hipStream_t stream);
 
 }  // namespace gphs

@@ -55,6 +55,8 @@ struct PlanObj {
   std::vector<SegDesc> segs;
   std::vector<TileDesc> tiles;
   int tile_max = 0;                        // events of the largest tile
+  int64_t n_events = 0;
+  int busiest = 0;                         // tiles of the channel that has most
   int64_t n_units = 0;                     // wavefronts of 64 events the tiles fill
   // the parts of tiles that are not full (DevicePlan::subs, units); empty where the tiles are mostly full
   std::vector<TileDesc> subs, units;

@@ -169,6 +169,46 @@ def test_update_counts_on_many_tiles(n_out, counts, cfg, bin_):
     assert np.array_equal(grid.weights(), oracle.grid_update(w, x, ok, ch))
 
 
+@pytest.mark.parametrize("n_out,segments,cfg,accept", [
+    # a channel of one more tile than the kernel of a tile per workgroup takes, and one of as many
+    (2, [(0, 193 * 256)], dict(), 0.7),
+    (2, [(0, 192 * 256)], dict(), 0.7),
+    # as many events as it takes, and one more
+    (4, [(k, 34_952) for k in range(14)] + [(14, 34_960)], dict(), 0.7),
+    (4, [(k, 34_952) for k in range(14)] + [(14, 34_961)], dict(), 0.7),
+    # 5 randoms: 2 of 512 threads without an element; ranges across many segments of two channels in turn
+    (3, [(k % 2, (65, 64, 1, 130, 63)[k % 5]) for k in range(500)], dict(block=64, ept=1), 0.7),
+    # tiles of 1024 events, the last of a segment a pass of 64 events, or a batch of 8, or next to it
+    (4, [(0, 200 * 1024)] + [(1 + k, 1024 * (k % 3) + n) for k, n in enumerate([64, 65, 63, 511, 512, 513, 575, 576, 577, 1, 128])],
+     dict(block=256, ept=4), 0.7),
+    # whole waves without an accepted event, and none at all
+    (4, [(0, 300 * 256), (1, 300 * 256)], dict(), 0.002),
+    (4, [(0, 300 * 256), (1, 5)], dict(), 0.0),
+])
+def test_update_counts_by_either_kernel(n_out, segments, cfg, accept):
+    """The histogram on both sides of the rule that picks its kernel, and where the one for many tiles begins and ends
+    a pass, a batch or a segment; randoms of rejected events, NaN here, do not matter."""
+    import torch
+    import gpu_phs_amd as G
+    proc = W.process_shapes(n_out, 3)
+    ph = G.ProcessHandle(proc)
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    segs = []
+    for c, n in segments:
+        b = G.EventBuffers.allocate(torch.rand((n, proc.n_x), generator=gen, device="cuda", dtype=torch.float64) ** 2, n_out)
+        b.ok.copy_(torch.rand(n, generator=gen, device="cuda") < accept)
+        b.x[b.ok == 0] = float("nan")
+        segs.append((ph, c, b))
+    plan = G.Plan(segs, **cfg)
+    grid = G.Grid(ph)
+    w = grid.weights()
+    grid.update(plan)
+    x = np.concatenate([b.x.cpu().numpy() for _, _, b in segs])
+    ok = np.concatenate([b.ok.cpu().numpy().astype(bool) for _, _, b in segs])
+    ch = np.concatenate([np.full(b.ok.shape[0], c) for _, c, b in segs])
+    assert np.array_equal(grid.weights(), oracle.grid_update(w, np.nan_to_num(x), ok, ch))
+
+
 @pytest.mark.parametrize("n_out", [7, 8, 12])
 def test_grids_of_large_trees(n_out):
     """Trees above six particles: the draw's tables in LDS grow with the randoms (2,640 bytes each, 84 KB for
