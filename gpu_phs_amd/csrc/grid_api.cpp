@@ -127,7 +127,7 @@ int gpu_phs_grid_generate(int grid, int plan, uint64_t seed, void* stream) {
   }
   if ((e = hipMemcpy(g->cdf_d, cdf.data(), cdf.size() * sizeof(double), hipMemcpyHostToDevice)) != hipSuccess)
     return hip_error(e, "hipMemcpy(grid)");
-  if ((e = launch_grid_generate(pl->dp, g->cdf_d, g->n_dim, seed, (hipStream_t)stream)) != hipSuccess)
+  if ((e = launch_grid_generate(pl->dp, pl->n_events, g->cdf_d, g->n_dim, seed, (hipStream_t)stream)) != hipSuccess)
     return hip_error(e, "grid generate launch");
   return ok_status();
 }

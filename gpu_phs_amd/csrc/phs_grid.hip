@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "phs_device.h"
 #include "phs_kernels.h"
@@ -68,15 +69,16 @@ __device__ __forceinline__ double in_bin(const BinRec& r, double u) {
 // where the row length is even and the rows are 16-byte aligned).  4e6 events of 8 randoms: 68 us
 // (56 VALU instructions per random, the vector units 73% busy; 79 us with both tables at strides
 // whose lanes met the same banks), against 103 us with nine bounds read per random, two
-// divisions and a division per word stored.
-constexpr int kGenWaves = 4;
-constexpr int kGenThreads = 64 * kGenWaves;
+// divisions and a division per word stored.  A run of at most kGenCellEvents events does not repay the first-bin
+// table and compares with the nine bounds (20,000 events of 32 randoms in 12 channels 36 and 46 us, but 2e6
+// of 8 60 and 58 us at twice as many events).
+constexpr int kGenWaves = 4;   // at most (launch_grid_generate)
 constexpr int kGenGroups = 4096;
 constexpr int kGenRow = 68;   // the lanes that read one another's columns meet different LDS banks
-constexpr int kGenCellBits = 6, kGenCells = 1 << kGenCellBits;
+constexpr int kGenCellBits = 6, kGenCells = 1 << kGenCellBits, kGenCellEvents = 256;
 
 // per_group, extra: workgroup b takes per_group tiles, and one more for b < extra.
-__global__ __launch_bounds__(kGenThreads) void grid_generate_kernel(const TileDesc* __restrict__ tiles, int per_group,
+__global__ __launch_bounds__(64 * kGenWaves) void grid_generate_kernel(const TileDesc* __restrict__ tiles, int per_group,
                                                                     int extra,
                                                                     const SegDesc* __restrict__ segs,
                                                                     const ChannelDesc* __restrict__ chans,
@@ -89,7 +91,8 @@ __global__ __launch_bounds__(kGenThreads) void grid_generate_kernel(const TileDe
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   double* xs0 = (double*)(rec + n_dim * kGridBins);
   double* xs = xs0 + wave * n_dim * kGenRow;
-  uint8_t* first = (uint8_t*)(xs0 + kGenWaves * n_dim * kGenRow);
+  const int threads = (int)blockDim.x;
+  uint8_t* first = (uint8_t*)(xs0 + (threads >> 6) * n_dim * kGenRow);
   const int b0 = (int)blockIdx.x;
   int t = b0 * per_group + (b0 < extra ? b0 : extra);
   const int t1 = t + per_group + (b0 < extra ? 1 : 0);
@@ -107,14 +110,16 @@ __global__ __launch_bounds__(kGenThreads) void grid_generate_kernel(const TileDe
     const int64_t e_end = e_run < sd.n_events ? e_run : sd.n_events;
     t += run;
     __syncthreads();   // the previous run's records have been read
-    for (int i = (int)threadIdx.x; i < n_x * kGridBins; i += kGenThreads) {
+    for (int i = (int)threadIdx.x; i < n_x * kGridBins; i += threads) {
       const int k = i / kGridBins, b = i - k * kGridBins;
       const double f0 = F0[k * NB1 + b], f1 = F0[k * NB1 + b + 1];
       const double rho = (f1 - f0) * kGridBins;
       // (no u is above the last bin's bound)
       rec[i] = BinRec{f0, b < kGridBins - 1 ? f1 : 2.0, rho, rho > 0x1.0p-1000 ? 1.0 / rho : 0.0, (double)b / kGridBins};
     }
-    for (int i = (int)threadIdx.x; i < n_x * kGenCells; i += kGenThreads) {
+    // the first-bin table pays for itself from some hundred events on
+    const bool cells = e_end - td.e0 > kGenCellEvents;
+    for (int i = (int)threadIdx.x; cells && i < n_x * kGenCells; i += threads) {
       const double* F = F0 + i / kGenCells * NB1;
       const double u = (double)(i % kGenCells) / kGenCells;
       int b = 0;
@@ -129,23 +134,36 @@ __global__ __launch_bounds__(kGenThreads) void grid_generate_kernel(const TileDe
     const int ev0 = (int)__umulhi((uint32_t)(lane * step), div_nx), k0 = lane * step - ev0 * n_x;
     const int dev = (int)__umulhi((uint32_t)(64 * step), div_nx), dk = 64 * step - dev * n_x;
     // (tiles start at multiples of 64 events, so an event's low index word is the unit's with the lane)
-    for (int64_t e = td.e0 + 64 * wave; e < e_end; e += kGenThreads) {
+    for (int64_t e = td.e0 + 64 * wave; e < e_end; e += threads) {
       const int cnt = e_end - e < 64 ? (int)(e_end - e) : 64;
       const uint32_t e_lo = (uint32_t)e + (uint32_t)lane, e_hi = (uint32_t)((uint64_t)e >> 32);
-      for (int j = 0; 2 * j < n_x; j++) {
-        uint32_t c[4] = {e_lo, e_hi, (uint32_t)td.seg, (uint32_t)j};
-        philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
+      auto draw = [&](auto by_cells) {
+        for (int j = 0; 2 * j < n_x; j++) {
+          uint32_t c[4] = {e_lo, e_hi, (uint32_t)td.seg, (uint32_t)j};
+          philox4x32_10(c, (uint32_t)seed, (uint32_t)(seed >> 32));
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-          const int k = 2 * j + h;
-          if (k >= n_x) break;
-          const double u = u53(c[2 * h], c[2 * h + 1]);
-          const BinRec* at = rec + k * kGridBins + first[k * kGenCells + (int)(c[2 * h] >> (32 - kGenCellBits))];
-          BinRec r = *at;
-          while (r.next <= u) r = *++at;
-          xs[k * kGenRow + lane] = r.edge + in_bin(r, u);
+          for (int h = 0; h < 2; h++) {
+            const int k = 2 * j + h;
+            if (k >= n_x) break;
+            const double u = u53(c[2 * h], c[2 * h + 1]);
+            const BinRec* at = rec + k * kGridBins;
+            BinRec r;
+            if constexpr (decltype(by_cells)::value) {
+              at += first[k * kGenCells + (int)(c[2 * h] >> (32 - kGenCellBits))];
+              r = *at;
+              while (r.next <= u) r = *++at;
+            } else {
+              int b = 0;
+#pragma unroll
+              for (int q = 1; q < kGridBins; q++) b += at[q].F <= u ? 1 : 0;
+              r = at[b];
+            }
+            xs[k * kGenRow + lane] = r.edge + in_bin(r, u);
+          }
         }
-      }
+      };
+      if (cells) draw(std::true_type{});
+      else draw(std::false_type{});
       // the wave's lanes read one another's columns: no other wave is concerned
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
@@ -374,12 +392,23 @@ __global__ void fill_u64_kernel(unsigned long long* p, size_t n) {
 
 }  // namespace
 
-hipError_t launch_grid_generate(const DevicePlan& dp, const double* cdf, int n_dim, uint64_t seed, hipStream_t stream) {
+hipError_t launch_grid_generate(const DevicePlan& dp, int64_t n_events, const double* cdf, int n_dim, uint64_t seed,
+                                hipStream_t stream) {
   if (dp.n_tiles <= 0) return hipSuccess;
-  const size_t shmem = (size_t)n_dim * (kGridBins * sizeof(BinRec) + kGenWaves * kGenRow * sizeof(double) + kGenCells);
-  if (shmem > forward_lds_limit()) return hipErrorInvalidValue;   // 84 KB for the 32 randoms of twelve particles
   const int groups = std::min(dp.n_tiles, kGenGroups);
-  hipLaunchKernelGGL(grid_generate_kernel, dim3(groups), dim3(kGenThreads), shmem, stream, dp.tiles,
+  // waves of a workgroup: no more than have events to draw, and, where the launch fills the device, as many as let
+  // a CU hold the most waves (2000 tiles of 70 events of 32 randoms: 118 us with four, 69 with two)
+  const size_t limit = forward_lds_limit();
+  auto lds = [&](int waves) {
+    return (size_t)n_dim * (kGridBins * sizeof(BinRec) + waves * kGenRow * sizeof(double) + kGenCells);
+  };
+  int waves = kGenWaves;
+  while (waves > 1 && n_events <= (int64_t)32 * waves * groups) waves /= 2;
+  for (int w = waves / 2; w > 0 && (size_t)groups > 256 * (limit / lds(waves)); w /= 2)
+    if (limit / lds(w) * w > limit / lds(waves) * waves) waves = w;
+  const size_t shmem = lds(waves);
+  if (shmem > limit) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(grid_generate_kernel, dim3(groups), dim3(64 * waves), shmem, stream, dp.tiles,
                      dp.n_tiles / groups, dp.n_tiles % groups, dp.segs, dp.chans, cdf, n_dim, seed);
   return hipGetLastError();
 }

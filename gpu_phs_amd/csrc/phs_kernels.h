@@ -131,7 +131,8 @@ hipError_t launch_inverse(const InverseTables& it, const TileDesc* tiles, int n_
 // Adaptive grids of the randoms (rng.cpp:5: 10 equal bins per channel and dimension).
 constexpr int kGridBins = 10;
 // Randoms of every segment of the plan drawn from the grids: cdf [plan channel][n_dim][11].
-hipError_t launch_grid_generate(const DevicePlan& dp, const double* cdf, int n_dim, uint64_t seed, hipStream_t stream);
+hipError_t launch_grid_generate(const DevicePlan& dp, int64_t n_events, const double* cdf, int n_dim, uint64_t seed,
+                                hipStream_t stream);
 // counts [plan channel][n_dim][10] histogram of the accepted events' randoms, then the accepted
 // count of every plan channel (n_chans more entries); cleared first.  busiest: tiles of the channel that
 // has most.

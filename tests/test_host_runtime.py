@@ -150,20 +150,17 @@ assert H.hip_host_violations() == 0
 
 
 def test_grid_draw_asks_for_its_lds(run):
-    """The draw's tables (2,640 bytes of LDS per random) are checked against the device's limit before the launch."""
+    """The draw's tables (464 bytes of LDS per random, and 544 for each wave) stay within the device's limit: where four
+    waves do not fit, fewer draw."""
     run("""
 H.hip_host_lds(65536)
-for n_out, fits in ((8, True), (12, False)):
+for n_out in (8, 12):
     pl = plan(W.process_large(n_out), [100, 100])
     grid = G.Grid(pl._keep[0][0])
     launches()
-    try:
-        grid.generate(pl, 1, Stream)
-        ok = True
-    except G.GpuPhsError:
-        ok = False
-    assert ok == fits
-    assert any("grid_generate" in k for k in launches()) == fits
+    grid.generate(pl, 1, Stream)
+    assert any("grid_generate" in k for k in launches())
+assert 0 < H.hip_host_most_lds() <= 65536, H.hip_host_most_lds()
 """)
 
 
