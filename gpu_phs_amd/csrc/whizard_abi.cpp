@@ -27,8 +27,15 @@ namespace {
 // and 50, 8 MiB 52 and 53), small ones start the first DMA and end the last host copy early (a call of
 // 10^5 2 -> 4 events on one stream: 1.40 ms at 2 MiB, 1.27 at 4, 1.40 at 8).  A second stream for the smaller
 // transfers to the device gained another 0.04 ms, but cost two more calls of 7-14 ms at the start of a process.
+//
+// From kOneStream bytes on, transfers to the host take one stream and chunks of two slots: in a process that has
+// used other streams the copy engines that the runtime gives to two streams made every second of the first ten
+// calls of 10^6 events take 13.4 ms, the others 9.7, before they settled at 9.0; one stream takes 9.4 from the
+// first.  (Below, two streams take 208 us for 1,818 2 -> 6 events, 1.06 and 2.85 ms for 10^5 and 3 x 10^5 of
+// 2 -> 4, also beside others; one stream with chunks of two slots 226 us, 1.13 and 2.92.)
 constexpr int kPinSlots = 8;
 constexpr size_t kPinChunk = (size_t)4 << 20;
+constexpr size_t kOneStream = (size_t)128 << 20;
 
 struct WhizardModule {
   int n_channels = 0, n_in = 0, n_out = 0, n_x = 0;
@@ -281,7 +288,6 @@ struct Transfer {
 // To the device: returns when every DMA is queued.  To the host: when all has arrived.
 int transfer(WhizardModule& w, const std::vector<Transfer>& list, bool to_device) {
   constexpr size_t kPiece = (size_t)256 << 10, kPoolBytes = (size_t)1 << 20;
-  constexpr int kPieces = (int)(kPinChunk / kPiece);
   struct Chunk {
     char* host;
     char* dev;
@@ -289,13 +295,15 @@ int transfer(WhizardModule& w, const std::vector<Transfer>& list, bool to_device
   };
   std::vector<Chunk> chunks;
   size_t total = 0;
-  for (const Transfer& t : list) {
-    total += t.n;
-    for (size_t off = 0; off < t.n; off += kPinChunk)
-      chunks.push_back(Chunk{(char*)t.host + off, (char*)t.dev + off, std::min(kPinChunk, t.n - off)});
-  }
+  for (const Transfer& t : list) total += t.n;
+  const bool large = !to_device && total >= kOneStream, one_stream = to_device || large;
+  const size_t chunk = large ? 2 * kPinChunk : kPinChunk;
+  const int slots = (int)(kPinSlots * kPinChunk / chunk), pieces_of = (int)(chunk / kPiece);
+  for (const Transfer& t : list)
+    for (size_t off = 0; off < t.n; off += chunk)
+      chunks.push_back(Chunk{(char*)t.host + off, (char*)t.dev + off, std::min(chunk, t.n - off)});
   const int n = (int)chunks.size();
-  auto slot = [&](int c) { return w.pin + (size_t)(c % kPinSlots) * kPinChunk; };
+  auto slot = [&](int c) { return w.pin + (size_t)(c % slots) * chunk; };
   auto host_copy = [&](int c, size_t off, size_t bytes) {
     char* pinned = slot(c) + off;
     char* user = chunks[c].host + off;
@@ -304,12 +312,12 @@ int transfer(WhizardModule& w, const std::vector<Transfer>& list, bool to_device
   };
   auto dma = [&](int c) -> hipError_t {
     const Chunk& k = chunks[c];
-    hipStream_t st = c % 2 && !to_device ? w.stream2 : w.stream;
+    hipStream_t st = c % 2 && !one_stream ? w.stream2 : w.stream;
     hipError_t e = to_device ? hipMemcpyAsync(k.dev, slot(c), k.n, hipMemcpyHostToDevice, st)
                              : hipMemcpyAsync(slot(c), k.dev, k.n, hipMemcpyDeviceToHost, st);
-    return e != hipSuccess ? e : hipEventRecord(w.pin_ev[c % kPinSlots], st);
+    return e != hipSuccess ? e : hipEventRecord(w.pin_ev[c % slots], st);
   };
-  auto arrived = [&](int c) { return hipEventSynchronize(w.pin_ev[c % kPinSlots]); };
+  auto arrived = [&](int c) { return hipEventSynchronize(w.pin_ev[c % slots]); };
   // no DMA on the slots or the device arrays goes on after a transfer that failed
   auto failed = [&](hipError_t e, const char* what) {
     (void)hipStreamSynchronize(w.stream);
@@ -317,11 +325,11 @@ int transfer(WhizardModule& w, const std::vector<Transfer>& list, bool to_device
     return hip_error(e, what);
   };
 
-  // pieces [kPieces c, kPieces (c + 1)) are chunk c's (those past its end are empty); `open` chunks may be
+  // pieces [pieces_of c, pieces_of (c + 1)) are chunk c's (those past its end are empty); `open` chunks may be
   // copied so far: arrived from the device, or with a free slot
   std::unique_ptr<std::atomic<int>[]> left(new std::atomic<int>[n > 0 ? n : 1]);
-  for (int c = 0; c < n; c++) left[c].store(kPieces, std::memory_order_relaxed);
-  std::atomic<int> next{0}, open{to_device ? std::min(n, kPinSlots) : 0};
+  for (int c = 0; c < n; c++) left[c].store(pieces_of, std::memory_order_relaxed);
+  std::atomic<int> next{0}, open{to_device ? std::min(n, slots) : 0};
   std::atomic<bool> abort{false};
   Waiting for_open, for_copied;
   auto open_to = [&](int c) {
@@ -330,11 +338,11 @@ int transfer(WhizardModule& w, const std::vector<Transfer>& list, bool to_device
   };
   const std::function<void()> pieces = [&] {
     for (;;) {
-      const int q = next.fetch_add(1, std::memory_order_relaxed), c = q / kPieces;
+      const int q = next.fetch_add(1, std::memory_order_relaxed), c = q / pieces_of;
       if (c >= n) return;
       for_open.until([&] { return open.load(std::memory_order_acquire) > c || abort.load(std::memory_order_relaxed); });
       if (abort.load(std::memory_order_relaxed)) return;
-      const size_t off = (size_t)(q % kPieces) * kPiece;
+      const size_t off = (size_t)(q % pieces_of) * kPiece;
       if (off < chunks[c].n) host_copy(c, off, std::min(kPiece, chunks[c].n - off));
       if (left[c].fetch_sub(1, std::memory_order_release) == 1) for_copied.changed();
     }
@@ -343,8 +351,8 @@ int transfer(WhizardModule& w, const std::vector<Transfer>& list, bool to_device
 
   hipError_t e = hipSuccess;
   // the slots' DMAs of the previous transfer; to the host, the other stream follows the kernels
-  for (int c = 0; to_device && c < std::min(n, kPinSlots) && e == hipSuccess; c++) e = arrived(c);
-  if (!to_device && (e = hipEventRecord(w.kernels_ev, w.stream)) == hipSuccess && n > 1)
+  for (int c = 0; to_device && c < std::min(n, slots) && e == hipSuccess; c++) e = arrived(c);
+  if (!to_device && (e = hipEventRecord(w.kernels_ev, w.stream)) == hipSuccess && !one_stream)
     e = hipStreamWaitEvent(w.stream2, w.kernels_ev, 0);
   if (e != hipSuccess) return failed(e, "staging events");
   int threads = 0;
@@ -361,16 +369,16 @@ int transfer(WhizardModule& w, const std::vector<Transfer>& list, bool to_device
       for_copied.until([&] { return copied(c); });
       e = dma(c);
       // half the ring stays in flight
-      for (; e == hipSuccess && freed + kPinSlots < n && c - freed >= kPinSlots / 2; freed++)
-        if ((e = arrived(freed)) == hipSuccess) open_to(freed + kPinSlots + 1);
+      for (; e == hipSuccess && freed + slots < n && c - freed >= slots / 2; freed++)
+        if ((e = arrived(freed)) == hipSuccess) open_to(freed + slots + 1);
     }
   } else {
     for (int c = 0, issued = 0; c < n && e == hipSuccess; c++) {
       // every chunk whose slot has been copied out; at least this one
-      for (; issued < n && issued < c + kPinSlots && e == hipSuccess; issued++) {
-        if (issued >= kPinSlots) {
-          if (issued > c && !copied(issued - kPinSlots)) break;
-          for_copied.until([&] { return copied(issued - kPinSlots); });
+      for (; issued < n && issued < c + slots && e == hipSuccess; issued++) {
+        if (issued >= slots) {
+          if (issued > c && !copied(issued - slots)) break;
+          for_copied.until([&] { return copied(issued - slots); });
         }
         e = dma(issued);
       }

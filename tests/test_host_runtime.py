@@ -93,13 +93,14 @@ def run(tmp_path_factory):
     return run
 
 
-@pytest.mark.parametrize("wait", [0, 5, 9, 12, 15])
-def test_failed_host_call_leaves_no_copy_behind(run, wait):
+@pytest.mark.parametrize("events,wait", [(100_000, 0), (100_000, 5), (100_000, 9), (100_000, 12), (100_000, 15),
+                                         (150_000, 12), (150_000, 20)])
+def test_failed_host_call_leaves_no_copy_behind(run, events, wait):
     """A wait that fails in the middle of a host call (300,000 events: some 30 chunks, a ring of eight slots, two
-    streams) ends the call with an error and with no transfer in flight, so that the pinned slots may be
+    streams; 450,000: larger chunks on one) ends the call with an error and with no transfer in flight, so that the pinned slots may be
     released at once."""
     run(f"""
-L, call = whizard(W.process_c1(), [100_000] * 3)
+L, call = whizard(W.process_c1(), [{events}] * 3)
 assert call() == 0
 H.hip_host_fail_wait({wait})
 assert call() != 0
