@@ -86,11 +86,11 @@ def run_workload(name, steps, warmup, torch, G, W, tune=True, fixed=None, tuning
     # the batched launches submitted from a hipGraph and directly; a graph replay costs a few
     # microseconds more than a direct launch, which shows on the smallest workloads
     wall, ev_s = time_steps(plan.run_graph, steps, warmup, torch)
-    launch = "one batched launch per tile class, replayed from a hipGraph"
+    launch = "one launch per tile class and group of tree shapes, replayed from a hipGraph"
     d_wall, d_ev = time_steps(plan.run, steps, warmup, torch)
     if d_ev < ev_s:
         wall, ev_s = d_wall, d_ev
-        launch = "one batched launch per tile class, submitted directly"
+        launch = "one launch per tile class and group of tree shapes, submitted directly"
     plain_wall, plain_ev = time_steps(plan.run_plain, max(1, steps // 2), warmup, torch)
     n = wl.n_events
     res = dict(workload=name, n_events=n, n_segments=len(segs),
@@ -623,7 +623,7 @@ def main():
                      "frac": achieved / HBM_PEAK_GBS,
                      "traffic": counters["traffic"] if counters else None,
                      "traffic_counted_with": counters["tuning"] if counters else None,
-                     "kernel": "forward_kernel (every launch of one step)", "kernel_ms": main_res["batched_kernel_ms"],
+                     "kernel": "forward_shapes_kernel (every launch of one step)", "kernel_ms": main_res["batched_kernel_ms"],
                      "bytes_per_launch": main_res["algorithmic_bytes"], "fp64": fp64,
                      "copy_ceiling": {"gb_s": copy_gb_s, "frac": achieved / copy_gb_s,
                                       "what": "the device's streaming copy of 2 GiB, one 16-byte word per thread"}},

@@ -194,11 +194,12 @@ int inverse_prepare(PlanObj& pl, const int64_t* seg_row0, int64_t n_rows) {
 // Ranges of channels that each 64-event unit is split over, one wave each: as many as give every
 // SIMD its three waves (any split, also single channels), then as many as give a dozen rounds of
 // waves, so that the last round's idle SIMDs cost little, but no fewer than min_channels channels
-// each, since a range stages the momenta and evaluates its first root anew.  2e5 events x 120
-// channels (3190 units): 0.96 ms at 13 ranges, 1.08 at 4, 1.05 at 51; 1e6 events x 3 channels (15,627
-// units): 113 us unsplit, 138 at 3 ranges.  Above four particles a channel is more work and a SIMD holds two
-// waves, and three channels are enough: 1e5 events x 16 channels of 2->6 (1592 units) 154 us at 4 ranges,
-// 145 at 5, 146 at 8, 157 at 3.
+// each, since a range stages the momenta and evaluates its first root anew.  With the walks as they
+// were when this was chosen (0.69 ms and 102 us since): 2e5 events x 120 channels (3190 units) 0.96 ms
+// at 13 ranges, 1.08 at 4, 1.05 at 51; 1e6 events x 3 channels (15,627 units) 113 us unsplit, 138 at 3
+// ranges.  Above four particles a channel is more work and a SIMD holds two waves, and three channels
+// are enough: 1e5 events x 16 channels of 2->6 (1592 units) 154 us at 4 ranges, 145 at 5, 146 at 8, 157
+// at 3.
 int inverse_chunks(const InverseTables& it, int64_t units) {
   constexpr int64_t kFillWaves = 256 * 4 * 3, kManyWaves = 40000;
   const int64_t min_channels = it.n_out <= 4 ? 4 : 3;

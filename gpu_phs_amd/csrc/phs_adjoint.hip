@@ -243,7 +243,8 @@ using AdjKernel = adj::Kernel;
 // The kernel of the shapes [lo, hi] that a launch has (of one group): those of one number of final-state
 // particles, or of all of two to four.  Waves per SIMD: as many as the registers hold without spills, so two
 // for the trees of four with given cotangents (10^6 events: 96 us; at three, with 108 bytes of scratch per
-// lane, 129).
+// lane, 129).  The trees of six with given cotangents take all 256 registers that two leave a lane, and
+// 44 bytes of scratch.
 template <int LM>
 adj::Kernel pick_shapes(int lo, int hi) {
   if (hi < 1) return adj::shapes_kernel<0, 1, LM, 4>;

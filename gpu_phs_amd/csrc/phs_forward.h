@@ -411,9 +411,10 @@ constexpr int shape_bank() {
 }
 
 // Sub-tiles of several shapes in one launch: every workgroup takes the code specialised for its
-// tile's shape, one of [LO, HI).  A launch lasts at least one wave's lifetime however few tiles it
-// has, so the shapes that are too small for a launch of their own share this one.  The tiles are
-// sorted by shape: the waves of a CU mostly run the same code.
+// tile's shape, one of [LO, HI): the launch of every group of two or more shapes, unless merge_below is 0.
+// A launch lasts at least one wave's lifetime however few tiles it has, and one for all shapes was the
+// fastest at every size (launch_runs).  The tiles are sorted by shape: the waves of a CU mostly run the
+// same code.
 template <int LO, int HI, bool PEV, int BLK>
 __device__ __forceinline__ void sub_tile_of_shape(int shape, const TileDesc& td, const SegDesc& sd,
                                                   const ChannelDesc& cd, const NodeCmd* __restrict__ prog, int base) {

@@ -1,5 +1,5 @@
 // The one-pass forward kernel of all the shapes of six final-state particles ([22, 64) of the shape
-// table): plans whose shapes are too small for launches of their own.
+// table), the launch of every group of two or more of them unless merge_below is 0.
 #include "phs_forward.h"
 
 namespace gphs {

@@ -527,11 +527,11 @@ __device__ __forceinline__ double inverse_walk(const ChannelDesc& cd, const EvBe
 // association, and not on any map.  The host orders the channels by the branches of their trees, root
 // first, and marks in each step which branches differ from the last ones evaluated
 // (InvStep::eval); the others keep their numbers, and the channel only applies its maps.  The 120
-// channels of random 2->4 trees evaluate 30 roots and 129 branches instead of 240 (690 VALU
+// channels of random 2->4 trees evaluate 30 roots and 129 branches instead of 240 (680 VALU
 // instructions per event and channel instead of 897).  Where few branches repeat, the tests keep the
 // compiler from interleaving a branch's evaluation with the maps and cost more than they save (the
-// three 2->4 resonance channels, which share nothing: 134 against 120 us for 1e6 events), so
-// inverse_walk runs, which also leaves out the generating channel's branches.
+// three 2->4 resonance channels, which share nothing: 134 against 120 us for 1e6 events when the branches
+// were first shared), so inverse_walk runs, which also leaves out the generating channel's branches.
 
 // What a branch below the root leaves behind: msq of its internal daughter (if any), sqrt(lambda) /
 // msq, the first daughter's angles, and what its daughters' frame is formed from.
@@ -714,9 +714,9 @@ __device__ __forceinline__ double inverse_channel(const ChannelDesc& cd, const E
 // range's, so that the waves of a CU mostly read the same records and run the same code (16 channels
 // of 2->6 trees 157 against 168 us for 1e5 events, 120 2->4 channels equal).  Its lanes exchange data
 // only through the wave's own randoms table.  1e6 events x 3 channels: 102 us (116 with each constant
-// loaded where it is used); 2e5 x 120: 0.70 ms cold, the clock falling under a sustained load (0.80), the
-// vector units 80% busy; 1e5 x 16 of 2->6: 157 us (310 on the walk that reads its structure from the
-// program, whose LDS bank held it to one wave per SIMD).
+// loaded where it is used), the vector units 60% busy; 2e5 x 120: 0.69 ms cold, the clock falling under a
+// sustained load (0.80), 75% busy; 1e5 x 16 of 2->6: 146 us, 51% busy (310 on the walk that reads its
+// structure from the program, whose LDS bank held it to one wave per SIMD).
 // LDS per wave: the momenta column (4 n_out rows of 64 doubles), the generic walk's save banks of
 // subtrees deferred below the root (19 rows of 64 doubles per level), then the randoms table of the
 // channel being inverted (n_x rows of kInvRow doubles).
