@@ -10,7 +10,7 @@ namespace {
 
 // Device tables for the adjoint of a plan: the plan's tiles, channels and programs, a segment
 // table carrying the gradient buffers, the per-tile partials and the tiles of each channel.
-int adjoint_prepare(PlanObj& pl, const gpu_phs_adjoint_segment* adj, int write_forward) {
+int adjoint_prepare(PlanObj& pl, const gpu_phs_adjoint_segment* adj, int write_forward, hipStream_t stream) {
   const int n_seg = (int)pl.segs.size(), n_ch = (int)pl.chans.size(), n_t = pl.dp.n_tiles;
 
   int max_nodes = 0, max_banks = 0;
@@ -81,7 +81,8 @@ int adjoint_prepare(PlanObj& pl, const gpu_phs_adjoint_segment* adj, int write_f
   }
   char* base = (char*)pl.adj_dev;
   hipError_t e;
-  if ((e = hipMemcpy(base, pl.adj_segs.data(), n_seg * sizeof(SegDesc), hipMemcpyHostToDevice)) != hipSuccess ||
+  if ((e = wait_for_queued(stream)) != hipSuccess ||
+      (e = hipMemcpy(base, pl.adj_segs.data(), n_seg * sizeof(SegDesc), hipMemcpyHostToDevice)) != hipSuccess ||
       (e = hipMemcpy(base + b_segs + b_part, list.data(), n_t * sizeof(int), hipMemcpyHostToDevice)) != hipSuccess ||
       (e = hipMemcpy(base + b_segs + b_part + b_list, off.data(), (n_ch + 1) * sizeof(int), hipMemcpyHostToDevice)) !=
           hipSuccess ||
@@ -145,7 +146,7 @@ int gpu_phs_plan_adjoint(int plan, const gpu_phs_adjoint_segment* adj, int loss_
   if (pl->dp.per_event_beams && loss_mode == 1)
     return set_error(GPU_PHS_E_ARG, "adjoint: the built-in loss assumes symmetric beams; with per-event beam energies "
                                     "give the cotangents (loss_mode 0)");
-  int rc = adjoint_prepare(*pl, adj, write_forward);
+  int rc = adjoint_prepare(*pl, adj, write_forward, (hipStream_t)stream);
   if (rc) return rc;
   // the tile table in runs of one tree shape, whose adjoint is specialised (the forward pass's merge_below
   // plays no part); launch_adjoint gives consecutive runs of one group one launch.  Other channels run the

@@ -59,7 +59,7 @@ std::vector<std::string> branch_keys(const CompiledProcess& cp, int c, int n) {
 
 // Device tables of the inverse: per-segment (generating channel, first row), uploaded again when the rows
 // change, then the process's channels and programs.
-int inverse_prepare(PlanObj& pl, const int64_t* seg_row0, int64_t n_rows) {
+int inverse_prepare(PlanObj& pl, const int64_t* seg_row0, int64_t n_rows, hipStream_t stream) {
   if (pl.segs.empty()) return set_error(GPU_PHS_E_ARG, "inverse: the plan has no segments");
   const int proc = pl.chan_process.empty() ? -1 : pl.chan_process[0];
   for (int p : pl.chan_process)
@@ -80,7 +80,9 @@ int inverse_prepare(PlanObj& pl, const int64_t* seg_row0, int64_t n_rows) {
       pl.inv.shared_roots == (shared ? 1 : 0) && is.size() == pl.inv_segs.size()) {
     // the process's tables are there; the rows may be others
     if (std::memcmp(is.data(), pl.inv_segs.data(), is.size() * sizeof(InvSeg)) == 0) return ok_status();
-    hipError_t e = hipMemcpy(pl.inv_dev, is.data(), is.size() * sizeof(InvSeg), hipMemcpyHostToDevice);
+    hipError_t e = wait_for_queued(stream);
+    if (e != hipSuccess) return hip_error(e, "hipStreamSynchronize(inverse rows)");
+    e = hipMemcpy(pl.inv_dev, is.data(), is.size() * sizeof(InvSeg), hipMemcpyHostToDevice);
     if (e != hipSuccess) return hip_error(e, "hipMemcpy(inverse rows)");
     pl.inv_segs = std::move(is);
     return ok_status();
@@ -158,7 +160,8 @@ int inverse_prepare(PlanObj& pl, const int64_t* seg_row0, int64_t n_rows) {
     const InvNode nd = inv_node(cp.nodes[i]);
     std::memcpy(host.data() + o_maps + i * sizeof(InvNode), &nd, sizeof nd);
   }
-  hipError_t e = hipMemcpy(pl.inv_dev, host.data(), total, hipMemcpyHostToDevice);
+  hipError_t e = wait_for_queued(stream);
+  if (e == hipSuccess) e = hipMemcpy(pl.inv_dev, host.data(), total, hipMemcpyHostToDevice);
   if (e != hipSuccess) return hip_error(e, "hipMemcpy(inverse tables)");
   char* base = (char*)pl.inv_dev;
   pl.inv.isegs = (const InvSeg*)base;
@@ -217,7 +220,7 @@ int gphs::plan_inverse(PlanObj& pl, const int64_t* seg_row0, int64_t n_rows, dou
     return set_error(GPU_PHS_E_ARG, "inverse: need seg_row0, n_rows > 0, factors and x_out");
   if (block != 0 && (block < 64 || block > 256 || block % 64))
     return set_error(GPU_PHS_E_ARG, "inverse: block must be 64, 128, 192 or 256");
-  int rc = inverse_prepare(pl, seg_row0, n_rows);
+  int rc = inverse_prepare(pl, seg_row0, n_rows, stream);
   if (rc) return rc;
   // the default workgroup: one wave with shared roots (its waves work alone), else 256 threads for
   // processes of a few channels, 128 for many, each where its LDS tables fit

@@ -30,6 +30,13 @@ int hip_error(hipError_t e, const char* what) {
   return set_error(GPU_PHS_E_HIP, m);
 }
 
+hipError_t wait_for_queued(hipStream_t stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (stream && hipStreamIsCapturing(stream, &status) == hipSuccess && status != hipStreamCaptureStatusNone)
+    return hipSuccess;
+  return hipStreamSynchronize(stream);
+}
+
 std::mutex& api_mutex() {
   static std::mutex m;
   return m;
@@ -284,12 +291,14 @@ int plan_build(PlanObj& pl) {
   const size_t o_units = o_subs + al(pl.subs.size() * sizeof(TileDesc));
   size_t total = o_units + al(pl.units.size() * sizeof(TileDesc)) + 256;
   drop_graph(pl);
+  hipError_t e = hipSuccess;
+  // launches on any stream may still read the tables of before
+  if (pl.dev && (e = hipDeviceSynchronize()) != hipSuccess) return hip_error(e, "hipDeviceSynchronize(plan tables)");
   if (total > pl.dev_bytes) {
     if (pl.dev) (void)hipFree(pl.dev);
     pl.dev = nullptr;
     pl.dev_bytes = 0;
-    hipError_t e = hipMalloc(&pl.dev, total);
-    if (e != hipSuccess) return hip_error(e, "hipMalloc(plan tables)");
+    if ((e = hipMalloc(&pl.dev, total)) != hipSuccess) return hip_error(e, "hipMalloc(plan tables)");
     pl.dev_bytes = total;
   }
   std::vector<char> host(total, 0);
@@ -299,8 +308,8 @@ int plan_build(PlanObj& pl) {
   if (!pl.nodes.empty()) std::memcpy(host.data() + o_nodes, pl.nodes.data(), pl.nodes.size() * sizeof(NodeCmd));
   if (!pl.subs.empty()) std::memcpy(host.data() + o_subs, pl.subs.data(), pl.subs.size() * sizeof(TileDesc));
   if (!pl.units.empty()) std::memcpy(host.data() + o_units, pl.units.data(), pl.units.size() * sizeof(TileDesc));
-  hipError_t e = hipMemcpy(pl.dev, host.data(), total, hipMemcpyHostToDevice);
-  if (e != hipSuccess) return hip_error(e, "hipMemcpy(plan tables)");
+  if ((e = hipMemcpy(pl.dev, host.data(), total, hipMemcpyHostToDevice)) != hipSuccess)
+    return hip_error(e, "hipMemcpy(plan tables)");
   char* base = (char*)pl.dev;
   pl.dp.tiles = (const TileDesc*)(base + o_tiles);
   pl.dp.segs = (const SegDesc*)(base + o_segs);

@@ -20,6 +20,9 @@ constexpr int64_t kMergeBelowDefault = (int64_t)1 << 18;
 int set_error(int code, const std::string& msg);
 inline int ok_status() { return set_error(GPU_PHS_OK, ""); }
 int hip_error(hipError_t e, const char* what);
+// Waits for what is queued on `stream`, before tables that it may still read are written over: hipMemcpy is ordered
+// behind the null stream's work only.  Not where the stream is being captured (nothing runs there).
+hipError_t wait_for_queued(hipStream_t stream);
 
 std::mutex& api_mutex();
 

@@ -18,6 +18,7 @@
 struct ihipEvent_t {
   hipStream_t stream = nullptr;
   uint64_t op = 0;   // the event is the op of this number on that stream
+  uint64_t kernel = 0;   // and the kernel of this number
 };
 
 struct ihipStream_t {
@@ -26,9 +27,10 @@ struct ihipStream_t {
     const void* src;
     size_t n;               // a copy, n > 0
     hipStream_t after;      // or a wait for another stream
-    uint64_t after_op;
+    uint64_t after_op, after_kernel;
   };
   std::deque<Op> queue;
+  uint64_t kernel = 0, kernel_done = 0;   // the last one launched, and waited for, by their numbers in the process
   uint64_t done = 0;        // ops executed so far
   uint64_t last() const { return done + queue.size(); }
 };
@@ -39,16 +41,24 @@ std::map<const void*, std::string> names;
 std::vector<std::string> launched;
 std::vector<hipStream_t> streams;
 std::map<char*, size_t> allocated;
+std::map<char*, uint64_t> allocated_at;   // after this kernel
+uint64_t kernels = 0;
+int overwritten = 0;
 int64_t groups = 0;
 size_t most_lds = 0;
 int violations = 0, fail_wait_after = -1, wait_us = 0, lds = 160 * 1024;
 double elapsed = 0, elapsed_step = 0;
 struct Config { dim3 grid, block; size_t shmem; hipStream_t stream; } config;
 
+bool inside(const void* p, const char* base, size_t n) { return (const char*)p >= base && (const char*)p < base + n; }
+
 void run_to(hipStream_t s, uint64_t op) {
   while (s->done < op) {
     const ihipStream_t::Op o = s->queue.front();
-    if (o.after) run_to(o.after, o.after_op);
+    if (o.after) {
+      run_to(o.after, o.after_op);
+      o.after->kernel_done = std::max(o.after->kernel_done, o.after_kernel);
+    }
     if (o.n) memcpy(o.dst, o.src, o.n);
     s->queue.pop_front();
     s->done++;
@@ -56,14 +66,24 @@ void run_to(hipStream_t s, uint64_t op) {
 }
 
 void run_all() {
-  for (hipStream_t s : streams) run_to(s, s->last());
+  for (hipStream_t s : streams) {
+    run_to(s, s->last());
+    s->kernel_done = s->kernel;
+  }
 }
 
-bool inside(const void* p, const char* base, size_t n) { return (const char*)p >= base && (const char*)p < base + n; }
+// A write to memory that kernels which no one has waited for may read: all but what was allocated after them.
+void check_write(const char* p) {
+  auto a = allocated.upper_bound((char*)p);
+  if (a == allocated.begin() || !(--a, inside(p, a->first, a->second))) return;
+  for (hipStream_t s : streams)
+    if (s->kernel > s->kernel_done && s->kernel > allocated_at[a->first]) overwritten++;
+}
 
 hipError_t allocate(void** p, size_t n) {
   *p = calloc(1, n ? n : 1);
   allocated[(char*)*p] = n;
+  allocated_at[(char*)*p] = kernels;
   return hipSuccess;
 }
 
@@ -92,6 +112,8 @@ int hip_host_pending() {
   return (int)n;
 }
 int hip_host_violations() { return violations; }
+// Memory written from the host while a kernel that may read it waited on a stream.
+int hip_host_overwritten() { return overwritten; }
 // Streams made so far, and those that have had a transfer.
 int hip_host_streams() { return (int)streams.size(); }
 int hip_host_used_streams() {
@@ -138,8 +160,9 @@ hipError_t hipMalloc(void** p, size_t n) { return allocate(p, n); }
 hipError_t hipFree(void* p) { return release(p); }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return allocate(p, n); }
 hipError_t hipHostFree(void* p) { return release(p); }
-hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { run_all(); memcpy(d, s, n); return hipSuccess; }
-hipError_t hipMemset(void* d, int v, size_t n) { run_all(); memset(d, v, n); return hipSuccess; }
+// (the streams do not wait for the null stream, nor it for them)
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { check_write((char*)d); memcpy(d, s, n); return hipSuccess; }
+hipError_t hipMemset(void* d, int v, size_t n) { check_write((char*)d); memset(d, v, n); return hipSuccess; }
 hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) { return hipMemset(d, v, n); }
 
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
@@ -148,18 +171,21 @@ hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
   return hipSuccess;
 }
 hipError_t hipStreamSynchronize(hipStream_t s) {
-  if (s) run_to(s, s->last());
-  else run_all();
+  if (!s) return hipSuccess;
+  run_to(s, s->last());
+  s->kernel_done = s->kernel;
   return hipSuccess;
 }
+hipError_t hipDeviceSynchronize() { run_all(); return hipSuccess; }
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* st) { *st = hipStreamCaptureStatusNone; return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t s) { return hipStreamSynchronize(s); }
 hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
-  if (s && e->stream) s->queue.push_back({nullptr, nullptr, 0, e->stream, e->op});
+  if (s && e->stream) s->queue.push_back({nullptr, nullptr, 0, e->stream, e->op, e->kernel});
   return hipSuccess;
 }
 hipError_t hipMemcpyAsync(void* d, const void* src, size_t n, hipMemcpyKind k, hipStream_t s) {
   if (!s) return hipMemcpy(d, src, n, k);
-  s->queue.push_back({d, src, n, nullptr, 0});
+  s->queue.push_back({d, src, n, nullptr, 0, 0});
   return hipSuccess;
 }
 
@@ -169,11 +195,14 @@ hipError_t hipEventDestroy(hipEvent_t e) { delete e; return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
   e->stream = s;
   e->op = s ? s->last() : 0;
+  e->kernel = s ? s->kernel : 0;
   return hipSuccess;
 }
 hipError_t hipEventSynchronize(hipEvent_t e) {
   if (fail_wait_after >= 0 && fail_wait_after-- == 0) return hipErrorUnknown;
-  if (!e->stream || e->stream->done >= e->op) return hipSuccess;
+  if (!e->stream) return hipSuccess;
+  e->stream->kernel_done = std::max(e->stream->kernel_done, e->kernel);
+  if (e->stream->done >= e->op) return hipSuccess;
   if (wait_us) std::this_thread::sleep_for(std::chrono::microseconds(wait_us));
   run_to(e->stream, e->op);
   return hipSuccess;
@@ -206,7 +235,9 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* shmem, hip
   *grid = config.grid; *block = config.block; *shmem = config.shmem; *s = config.stream;
   return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3, void**, size_t shmem, hipStream_t) {
+hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3, void**, size_t shmem, hipStream_t s) {
+  kernels++;
+  if (s) s->kernel = kernels;
   launched.push_back(names[f]);
   most_lds = std::max(most_lds, shmem);
   groups += (int64_t)grid.x * grid.y * grid.z;

@@ -306,3 +306,46 @@ pl.set_config(ept=16, grid=100)   # a persistent grid goes through tiles
 pl.run(Stream)
 assert H.hip_host_groups() <= 400
 """)
+
+
+@pytest.mark.parametrize("process", ["W.process_c1()", "W.process_2to6()", "W.process_friends(6)"])
+def test_tables_are_not_written_under_queued_launches(run, process):
+    """A plan's tables are written over only when what is queued on a stream of its own (which no copy waits for)
+    has run: other launch shapes, beams and orders, other output rows of the inverse, other buffers of the
+    adjoint, other weights of a grid."""
+    run(f"""
+proc, L = {process}, G.lib()
+n = proc.n_channels
+pl = plan(proc, [200] * n)
+stream = ctypes.c_void_p()
+assert H.hipStreamCreateWithFlags(ctypes.byref(stream), 1) == 0
+class Own:
+    cuda_stream = stream.value
+def quiet(what, change):
+    # a launch, the change, and a launch again
+    pl.run(Own)
+    change()
+    pl.run(Own)
+    assert H.hip_host_overwritten() == 0, what
+quiet("nothing", lambda: None)
+for config in (dict(grid=256), dict(grid=0), dict(block=64), dict(ept=4), dict(order=1)):
+    quiet(config, lambda: pl.set_config(**config))
+quiet("merge_below", lambda: L.gpu_phs_plan_set_merge_below(pl.handle, 0))
+beams = Array(200)
+quiet("beams", lambda: L.gpu_phs_plan_set_event_beams(pl.handle, 0, p(beams.a), p(beams.a)))
+quiet("beams off", lambda: L.gpu_phs_plan_set_event_beams(pl.handle, 0, None, None))
+buf = Array(64)
+for row in (0, 1, 2, 2):
+    rows = np.arange(n, dtype=np.int64) * 200 + row
+    assert L.gpu_phs_plan_inverse(pl.handle, p(rows), 10 ** 6, p(buf.a), p(buf.a), 0, stream) == 0
+    assert H.hip_host_overwritten() == 0, ("inverse", row)
+for _ in range(3):
+    keep = [Array((200, proc.n_x)) for _ in range(n)]
+    adj = (G._AdjSegment * n)(*(G._AdjSegment(None, None, k.data_ptr(), None) for k in keep))
+    assert L.gpu_phs_plan_adjoint(pl.handle, adj, 0, 0, p(buf.a), stream) == 0
+    assert H.hip_host_overwritten() == 0, "adjoint"
+grid = L.gpu_phs_grid_create(pl._keep[0][0].handle)
+for seed in range(3):
+    assert L.gpu_phs_grid_generate(grid, pl.handle, ctypes.c_uint64(seed), stream) == 0
+    assert H.hip_host_overwritten() == 0, "grid"
+""")
